@@ -81,6 +81,20 @@ __device__ __forceinline__ void stage_x8(const u32x4 raw, int v8, uint32_t* xp, 
     }
 }
 
+// Run that thread `tid` loads in pass i of staging `runs` runs: its own, or
+// one that exists (not used) where it has none -- its first one, and with
+// fewer runs than threads (K = 1024: 128) the last one.
+__host__ __device__ constexpr int staged_run(int runs, int i, int tid) {
+    const int own = i * kBlock + tid;
+    return own < runs ? own : tid < runs ? tid : runs - 1;
+}
+constexpr bool staged_runs_exist(int runs) {
+    for (int i = 0; i * kBlock < runs; ++i)
+        for (int t = 0; t < kBlock; ++t)
+            if (staged_run(runs, i, t) < 0 || staged_run(runs, i, t) >= runs) return false;
+    return true;
+}
+
 // x staging split in two so its global loads can be issued before the weight
 // loads: vmcnt retires loads in order, so x issued last would wait for every
 // weight load.  kRuns = K / 8 runs of eight values; thread t stages runs
@@ -93,15 +107,13 @@ template <int kLayout, int kRuns, bool kNorm = false>
 struct XStage {
     static constexpr int kIter = (kRuns + kBlock - 1) / kBlock;
     static_assert(kRuns % kWave == 0, "whole waves of runs");
+    static_assert(staged_runs_exist(kRuns), "no load past x, the residual or the norm weight");
     u32x4 raw[kIter];
     u32x4 dr[kNorm ? kIter : 1], wr[kNorm ? kIter : 1];
     __device__ static __forceinline__ bool has_run(int i) {
         return kRuns % kBlock == 0 || i * kBlock + (int)threadIdx.x < kRuns;
     }
-    // run index of pass i (a thread without a run re-reads its first one)
-    __device__ static __forceinline__ size_t run_of(int i) {
-        return has_run(i) ? (size_t)i * kBlock + threadIdx.x : (size_t)threadIdx.x;
-    }
+    __device__ static __forceinline__ size_t run_of(int i) { return (size_t)staged_run(kRuns, i, (int)threadIdx.x); }
     __device__ static __forceinline__ u32x4 keep(u32x4 v, int i) {
         if (has_run(i)) return v;
         return u32x4{0u, 0u, 0u, 0u};   // zeros: add nothing to the sum of squares
