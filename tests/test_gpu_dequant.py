@@ -84,3 +84,33 @@ def test_embed_q6k_rounds_ties_to_even(hip):
     dd = hip.DeviceArray(hidden * 2)
     hip.device.dequant_f16("q6k", dt, hidden, dd)
     assert np.all(dd.download(np.uint16, hidden) == rne + 1)
+
+
+@pytest.mark.parametrize("kind", ["q4k", "q6k"])
+@pytest.mark.parametrize("w_off,o_off", [(0, 0), (2, 2), (5, 6)])
+def test_device_dequant_scale_range_and_alignment(hip, orc, kind, w_off, o_off):
+    """Scales on both sides of the bound below which no value of a block can
+    overflow fp16 (one kernel path each), Inf / NaN / subnormal / negative
+    ones, a partial last block, and buffers at any alignment: bit for bit the
+    host routine's output (no tolerance)."""
+    nb = 300
+    rng = hip.synth.Rng(77)
+    blocks = (hip.synth.q4k_blocks(rng, nb) if kind == "q4k" else hip.synth.q6k_blocks(rng, nb)).reshape(nb, -1)
+    edge = 65000 / 945 if kind == "q4k" else 65000 / 4096
+    scales = np.array([edge * f for f in (0.5, 0.999, 1.0, 1.001, 1.1, 3, 60)] +
+                      [0.0, -0.0, -1e-3, 6e-8, -3e-6, 1e-5, np.inf, -np.inf, np.nan, 65504.0], np.float16)
+    d = scales[np.arange(nb) % scales.size].view(np.uint8).reshape(nb, 2)
+    dmin = scales[(np.arange(nb) // scales.size) % scales.size].view(np.uint8).reshape(nb, 2)
+    if kind == "q4k":
+        blocks[:, 0:2], blocks[:, 2:4] = d, dmin
+    else:
+        blocks[:, 208:210] = d
+    count = nb * 256 - 37
+    dw = hip.DeviceArray.from_numpy(np.concatenate([np.zeros(w_off, np.uint8), blocks.reshape(-1)]))
+    do = hip.DeviceArray(o_off + count * 2 + 64)
+    do.zero()
+    hip.device.dequant_f16(kind, dw.at(w_off), count, do.at(o_off))
+    out = do.download(np.uint8)
+    got = out[o_off:o_off + 2 * count].copy().view(np.uint16)
+    np.testing.assert_array_equal(got, orc.dequant_f16(kind, blocks.reshape(-1), count))
+    assert not out[:o_off].any() and not out[o_off + 2 * count:].any(), "wrote outside the output"
