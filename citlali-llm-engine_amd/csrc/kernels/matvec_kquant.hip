@@ -22,6 +22,7 @@
 //    sum(x) over each group; the block computes those sums while staging x.
 //  * No MFMA: M = 1 is not a dense contraction.  The bound is HBM.
 #include <algorithm>
+#include <atomic>
 #include <type_traits>
 
 #include "device_common.hpp"
@@ -45,20 +46,15 @@ constexpr int kWavesPerSimd = 2;
 // x staging: permuted fp16 pairs + per-group sums.
 // ---------------------------------------------------------------------------
 
-// Permutes one run of eight x values into LDS and writes its share of the
-// group sums in the layout kLayout.
+// A run of eight x values as the dot operands meet them.
+__device__ __forceinline__ u32x4 permute_x8(const u32x4 raw) {
+    return u32x4{__builtin_amdgcn_perm(raw.y, raw.x, 0x05040100u), __builtin_amdgcn_perm(raw.y, raw.x, 0x07060302u),
+                 __builtin_amdgcn_perm(raw.w, raw.z, 0x05040100u), __builtin_amdgcn_perm(raw.w, raw.z, 0x07060302u)};
+}
+
+// The run's share of the group sums in the layout kLayout.
 template <int kLayout>
-__device__ __forceinline__ void stage_x8(const u32x4 raw, int v8, uint32_t* xp, float* sx) {
-    if constexpr (kLayout == kPlain) {
-        *reinterpret_cast<u32x4*>(xp + (size_t)v8 * 4) = raw;
-        return;
-    }
-    u32x4 perm;
-    perm.x = __builtin_amdgcn_perm(raw.y, raw.x, 0x05040100u);
-    perm.y = __builtin_amdgcn_perm(raw.y, raw.x, 0x07060302u);
-    perm.z = __builtin_amdgcn_perm(raw.w, raw.z, 0x05040100u);
-    perm.w = __builtin_amdgcn_perm(raw.w, raw.z, 0x07060302u);
-    *reinterpret_cast<u32x4*>(xp + (size_t)v8 * 4) = perm;
+__device__ __forceinline__ void stage_sums8(const u32x4 raw, int v8, float* sx, float scale = 1.f) {
     float s = 0.f;
     s += h2f(raw.x & 0xffffu) + h2f(raw.x >> 16);
     s += h2f(raw.y & 0xffffu) + h2f(raw.y >> 16);
@@ -68,7 +64,7 @@ __device__ __forceinline__ void stage_x8(const u32x4 raw, int v8, uint32_t* xp, 
         // four consecutive threads hold one 32-value group
         s += dpp<kDppXor1>(s);
         s += dpp<kDppXor2>(s);
-        if ((v8 & 3) == 0) sx[v8 >> 2] = s;
+        if ((v8 & 3) == 0) sx[v8 >> 2] = s * scale;
     } else {
         // two consecutive threads hold one 16-value slice
         s += dpp<kDppXor1>(s);
@@ -76,8 +72,20 @@ __device__ __forceinline__ void stage_x8(const u32x4 raw, int v8, uint32_t* xp, 
             const int v = v8 * 8;
             const int b = v >> 8, in = v & 255;
             const int h = in >> 7, k = (in & 127) >> 5, ih = (in & 31) >> 4;
-            sx[b * 16 + h * 8 + ih * 4 + k] = s;
+            sx[b * 16 + h * 8 + ih * 4 + k] = s * scale;
         }
+    }
+}
+
+// Permutes one run of eight x values into LDS and writes its share of the
+// group sums in the layout kLayout.
+template <int kLayout>
+__device__ __forceinline__ void stage_x8(const u32x4 raw, int v8, uint32_t* xp, float* sx) {
+    if constexpr (kLayout == kPlain) {
+        *reinterpret_cast<u32x4*>(xp + (size_t)v8 * 4) = raw;
+    } else {
+        *reinterpret_cast<u32x4*>(xp + (size_t)v8 * 4) = permute_x8(raw);
+        stage_sums8<kLayout>(raw, v8, sx);
     }
 }
 
@@ -180,7 +188,6 @@ struct Q4K {
     static constexpr int kLanesPerSb = 4;
     static constexpr int kSbPerStep = kWave / kLanesPerSb;
     static constexpr int kHoistSteps = 4;   // x held in registers for rows of up to this many steps
-    static constexpr int kMaxSteps = 7;     // longest row a wave streams (K = 25600)
     struct Frag { u32x4 hdr, q0, q1; };
 
     __device__ static __forceinline__ Frag load(const uint8_t* sb, int j) {
@@ -210,18 +217,14 @@ struct Q4K {
         return dot(f, j, xload(xp, sx, j, b));
     }
 
-    // Contribution of lane j (group pair 2j, 2j+1) of a super-block.
-    __device__ static __forceinline__ float dot(const Frag& f, int j, const XRegs& x) {
-        // no fused multiply-adds: every kernel that inlines this computes the
-        // same bits (the fused launches equal the plain ones)
-#pragma clang fp contract(off)
+    // The 6-bit (scale, min) codes of groups 2j and 2j + 1, one byte each.
+    __device__ static __forceinline__ void scale_codes(const Frag& f, int j, uint32_t& sc, uint32_t& mn) {
         // 6-bit (scale, min) codes of groups 2j, 2j+1 (kernels.cu:174-186):
         // work on the two bytes k, k+1 of each 4-byte scale word at once.
         const uint32_t sh = (uint32_t)((2 * j) & 3) * 8u;
         const uint32_t a = (f.hdr.y >> sh) & 0xffffu;   // scales[k], [k+1]
         const uint32_t bq = (f.hdr.z >> sh) & 0xffffu;  // scales[k+4], [k+5]
         const uint32_t c = (f.hdr.w >> sh) & 0xffffu;   // scales[k+8], [k+9]
-        uint32_t sc, mn;
         if (j < 2) {
             sc = a & 0x3f3fu;
             mn = bq & 0x3f3fu;
@@ -229,9 +232,17 @@ struct Q4K {
             sc = (c & 0x0f0fu) | ((a >> 2) & 0x3030u);
             mn = ((c >> 4) & 0x0f0fu) | ((bq >> 2) & 0x3030u);
         }
+    }
+
+    // Contribution of lane j (group pair 2j, 2j+1) of a super-block.
+    __device__ static __forceinline__ float dot(const Frag& f, int j, const XRegs& x) {
+        // no fused multiply-adds: every kernel that inlines this computes the
+        // same bits (the fused launches equal the plain ones)
+#pragma clang fp contract(off)
+        uint32_t sc, mn;
+        scale_codes(f, j, sc, mn);
         const float d = h2f(f.hdr.x & 0xffffu);
         const float dmin = h2f(f.hdr.x >> 16);
-
         const u32x4 xl0 = x.l[0], xl1 = x.l[1], xl2 = x.l[2], xl3 = x.l[3];
         const u32x4 xh0 = x.h[0], xh1 = x.h[1], xh2 = x.h[2], xh3 = x.h[3];
         const uint32_t q[8] = {f.q0.x, f.q0.y, f.q0.z, f.q0.w, f.q1.x, f.q1.y, f.q1.z, f.q1.w};
@@ -268,7 +279,6 @@ struct Q6K {
     static constexpr int kLanesPerSb = 4;
     static constexpr int kSbPerStep = kWave / kLanesPerSb;
     static constexpr int kHoistSteps = 4;
-    static constexpr int kMaxSteps = 7;
     struct Frag { uint32_t wa[4], wb[4], u[4]; uint32_t s0, s1, dbits; };
 
     // lane_in_sb = 2*h + ih.  A 210-byte block starts on a 2-byte boundary;
@@ -310,47 +320,56 @@ struct Q6K {
         return dot(f, l4, xload(xp, sx, l4, b));
     }
 
+    // The 6-bit codes of the fragment's word t (four bytes) of every part p,
+    // as fp16 subnormals: bytes 0/2 in a[p], bytes 1/3 in b[p].
+    __device__ static __forceinline__ void codes(const Frag& f, int t, uint32_t (&a)[4], uint32_t (&b)[4]) {
+        const uint32_t wa = f.wa[t], wb = f.wb[t], u = f.u[t];
+        // low nibble (ql) | the slice's two qh bits << 4, one byte each; then
+        // bytes 0/2 and bytes 1/3 go to the two fp16 halves of an operand
+        // (one byte permute each, the other bytes zero).
+        const uint32_t k[4] = {(wa & 0x0f0f0f0fu) | ((u << 4) & 0x30303030u),
+                               (wb & 0x0f0f0f0fu) | ((u << 2) & 0x30303030u),
+                               ((wa >> 4) & 0x0f0f0f0fu) | (u & 0x30303030u),
+                               ((wb >> 4) & 0x0f0f0f0fu) | ((u >> 2) & 0x30303030u)};
+        constexpr uint32_t kEven = 0x0c020c00u, kOdd = 0x0c030c01u;   // 0x0c selects a zero byte
+#pragma unroll
+        for (int p = 0; p < 4; ++p) {
+            a[p] = __builtin_amdgcn_perm(0u, k[p], kEven);
+            b[p] = __builtin_amdgcn_perm(0u, k[p], kOdd);
+        }
+    }
+
+    // int8 scales sc[8h + ih + 2k], k = 0..3 (kernels.cu:166-167)
+    // (int8_t casts: the result must be converted as a signed value)
+    __device__ static __forceinline__ void scales(const Frag& f, int l4, float (&sc)[4]) {
+        const uint32_t sh = (uint32_t)(l4 & 1) * 8u;
+        sc[0] = (float)(int8_t)(f.s0 >> sh);
+        sc[1] = (float)(int8_t)(f.s0 >> (sh + 16u));
+        sc[2] = (float)(int8_t)(f.s1 >> sh);
+        sc[3] = (float)(int8_t)(f.s1 >> (sh + 16u));
+    }
+
     __device__ static __forceinline__ float dot(const Frag& f, int l4, const XRegs& x) {
 #pragma clang fp contract(off)   // the same bits in every kernel that inlines it
-        const int ih = l4 & 1;
         const float d = h2f((uint16_t)f.dbits);
-        // int8 scales sc[8h + ih + 2k], k = 0..3 (kernels.cu:166-167)
-        // (int8_t casts: the result must be converted as a signed value)
-        const uint32_t sh = (uint32_t)ih * 8u;
-        const float sc0 = (float)(int8_t)(f.s0 >> sh);
-        const float sc1 = (float)(int8_t)(f.s0 >> (sh + 16u));
-        const float sc2 = (float)(int8_t)(f.s1 >> sh);
-        const float sc3 = (float)(int8_t)(f.s1 >> (sh + 16u));
-
+        float sc[4];
+        scales(f, l4, sc);
         float p0 = 0.f, p1 = 0.f, p2 = 0.f, p3 = 0.f;
 #pragma unroll
         for (int t = 0; t < 4; ++t) {
-            const uint32_t wa = f.wa[t], wb = f.wb[t], u = f.u[t];
-            // 6-bit codes of the word's four bytes for each slice k: low
-            // nibble (ql) | the slice's two qh bits << 4, one byte each;
-            // then bytes 0/2 and bytes 1/3 go to the two fp16 halves of a
-            // dot2 operand (one byte permute each, the other bytes zero).
-            const uint32_t k0 = (wa & 0x0f0f0f0fu) | ((u << 4) & 0x30303030u);
-            const uint32_t k1 = (wb & 0x0f0f0f0fu) | ((u << 2) & 0x30303030u);
-            const uint32_t k2 = ((wa >> 4) & 0x0f0f0f0fu) | (u & 0x30303030u);
-            const uint32_t k3 = ((wb >> 4) & 0x0f0f0f0fu) | ((u >> 2) & 0x30303030u);
-            constexpr uint32_t kEven = 0x0c020c00u, kOdd = 0x0c030c01u;   // 0x0c selects a zero byte
-            const uint32_t c0a = __builtin_amdgcn_perm(0u, k0, kEven), c0b = __builtin_amdgcn_perm(0u, k0, kOdd);
-            const uint32_t c1a = __builtin_amdgcn_perm(0u, k1, kEven), c1b = __builtin_amdgcn_perm(0u, k1, kOdd);
-            const uint32_t c2a = __builtin_amdgcn_perm(0u, k2, kEven), c2b = __builtin_amdgcn_perm(0u, k2, kOdd);
-            const uint32_t c3a = __builtin_amdgcn_perm(0u, k3, kEven), c3b = __builtin_amdgcn_perm(0u, k3, kOdd);
-            const u32x2 x0 = x.v[0][t], x1 = x.v[1][t], x2 = x.v[2][t], x3 = x.v[3][t];
-            p0 = dot2(c0b, x0.y, dot2(c0a, x0.x, p0));
-            p1 = dot2(c1b, x1.y, dot2(c1a, x1.x, p1));
-            p2 = dot2(c2b, x2.y, dot2(c2a, x2.x, p2));
-            p3 = dot2(c3b, x3.y, dot2(c3a, x3.x, p3));
+            uint32_t a[4], b[4];
+            codes(f, t, a, b);
+            p0 = dot2(b[0], x.v[0][t].y, dot2(a[0], x.v[0][t].x, p0));
+            p1 = dot2(b[1], x.v[1][t].y, dot2(a[1], x.v[1][t].x, p1));
+            p2 = dot2(b[2], x.v[2][t].y, dot2(a[2], x.v[2][t].x, p2));
+            p3 = dot2(b[3], x.v[3][t].y, dot2(a[3], x.v[3][t].x, p3));
         }
         const f32x4 s = x.s;
         // sum (q6 - 32) x = 2^24 P - 32 S
-        const float t0 = sc0 * (p0 * 16777216.0f - 32.0f * s.x);
-        const float t1 = sc1 * (p1 * 16777216.0f - 32.0f * s.y);
-        const float t2 = sc2 * (p2 * 16777216.0f - 32.0f * s.z);
-        const float t3 = sc3 * (p3 * 16777216.0f - 32.0f * s.w);
+        const float t0 = sc[0] * (p0 * 16777216.0f - 32.0f * s.x);
+        const float t1 = sc[1] * (p1 * 16777216.0f - 32.0f * s.y);
+        const float t2 = sc[2] * (p2 * 16777216.0f - 32.0f * s.z);
+        const float t3 = sc[3] * (p3 * 16777216.0f - 32.0f * s.w);
         return d * ((t0 + t1) + (t2 + t3));
     }
 };
@@ -372,9 +391,6 @@ struct F16 {
     // a lane's x is 32 registers per step: rows of four steps read it from
     // LDS instead
     static constexpr int kHoistSteps = 3;
-    // 32 registers of weights per step in flight: longer rows take the flat
-    // kernel
-    static constexpr int kMaxSteps = 4;
     struct Frag { u32x4 v[8]; };
 
     __device__ static __forceinline__ Frag load(const uint8_t* sb, int j) {
@@ -751,6 +767,520 @@ __global__ __launch_bounds__(kBlock) void matvec_flat_kernel(const uint8_t* __re
     }
 }
 
+// ---------------------------------------------------------------------------
+// Tile kernels: Q4_K / Q6_K rows of any super-block count nb on the matrix
+// cores (v_mfma_f32_16x16x32_f16), for the counts that do not fill the wave
+// steps of the streaming kernels (see tile_length).
+//
+// A tile is up to 16 rows, MFMA columns; a wave's step is one super-block of
+// each of them, lane (row n = lane % 16, quarter g = lane / 16) holding
+// the 64 codes that lane g of a super-block holds in the streaming kernels.
+// The codes go in as the B operand (fp16 subnormals, exact, as in the dot2
+// form) and x as A, unchanged fp16 values: A row 4g + i is slot i of quarter
+// g and is non-zero only in lane group g, so lane (n, g) gets the sums of its
+// own codes with x slot i in accumulator i -- one sum per scale, no lane
+// moves.  Slots: the four 16-value parts of a Q6_K quarter, the first and
+// second half of the low and the high group of a Q4_K one.  Per 64 codes a
+// lane spends 40 (Q4_K) / 80 (Q6_K) bit operations and 8 MFMAs; the dot2 form
+// needs 32 dots more and a 64-lane sum per row.
+//
+// Each wave copies its steps' blocks, a piece of 144 / 210 bytes per row,
+// straight into a ring of kDepth LDS slots (global_load_lds_dwordx4, aligned
+// 16-byte pieces, so a Q6_K block's 2-byte alignment costs nothing before
+// LDS) and reads its fragments from there; the row pitch of 9 / 14 pieces
+// leaves the reads free of bank conflicts.  Read straight into registers in
+// this lane layout, a Q6_K matrix moved 4.5 TB/s against 6 here.
+//
+// The steps of a workgroup's tiles are dealt out to its eight waves in turn,
+// so no lane group or wave idles at any nb.  A step leaves its 16 row sums in
+// LDS; once a tile's steps are done one wave adds them in a fixed order.  A
+// row's result depends on nothing but its own blocks and x: every launch
+// form of a length gives the same bits.
+// ---------------------------------------------------------------------------
+typedef _Float16 half8 __attribute__((ext_vector_type(8)));
+
+constexpr int kTileCols = 16;
+constexpr int kTileWaves = 8;
+constexpr int kTileBlock = kTileWaves * kWave;
+constexpr int kZeroBytes = 128;   // what A lanes outside their quarter read (two 16-byte slots 64 bytes apart)
+
+__device__ __forceinline__ f32x4 mfma32(u32x4 a, u32x4 b, f32x4 c) {
+    return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(half8, a), __builtin_bit_cast(half8, b), c, 0, 0,
+                                                  0);
+}
+
+template <class QT>
+struct TileOps;
+
+template <>
+struct TileOps<Q4K> {
+    static constexpr int kPieces = 9;   // 16-byte pieces per block row
+    static constexpr int kRows = 14;    // rows of a tile
+    static constexpr float kSumScale = 1.f;
+    // 16-byte slot of run r (eight x values) of a super-block: [quarter][t][slot]
+    __device__ static __forceinline__ int slot(int r) {
+        const int grp = r >> 2, k = r & 3;   // 32-value group, run in it
+        return (grp >> 1) * 8 + (k & 1) * 4 + (grp & 1) + 2 * (k >> 1);
+    }
+    using Sums = f32x2;
+    __device__ static __forceinline__ Sums sums(const float* sx, int b, int g) {
+        return *reinterpret_cast<const f32x2*>(sx + b * 8 + 2 * g);
+    }
+    __device__ static __forceinline__ float dot(const Q4K::Frag& f, int g, u32x4 a0, u32x4 a1, Sums s) {
+#pragma clang fp contract(off)   // the same bits in every kernel that inlines it
+        const uint32_t q[8] = {f.q0.x, f.q0.y, f.q0.z, f.q0.w, f.q1.x, f.q1.y, f.q1.z, f.q1.w};
+        u32x4 lo[4], hi[4];
+#pragma unroll
+        for (int t = 0; t < 4; ++t) {
+            const uint32_t w0 = q[2 * t], w1 = q[2 * t + 1], v0 = w0 >> 8, v1 = w1 >> 8;
+            lo[t] = u32x4{w0 & 0x000f000fu, v0 & 0x000f000fu, w1 & 0x000f000fu, v1 & 0x000f000fu};   // q * 2^-24
+            hi[t] = u32x4{w0 & 0x00f000f0u, v0 & 0x00f000f0u, w1 & 0x00f000f0u, v1 & 0x00f000f0u};   // q * 2^-20
+        }
+        const f32x4 z = {0.f, 0.f, 0.f, 0.f};
+        f32x4 d0 = mfma32(a0, lo[0], z), d1 = mfma32(a0, hi[0], z), d2 = mfma32(a0, lo[2], z), d3 = mfma32(a0, hi[2], z);
+        d0 = mfma32(a1, lo[1], d0);
+        d1 = mfma32(a1, hi[1], d1);
+        d2 = mfma32(a1, lo[3], d2);
+        d3 = mfma32(a1, hi[3], d3);
+        uint32_t sc, mn;
+        Q4K::scale_codes(f, g, sc, mn);
+        const float d24 = h2f(f.hdr.x & 0xffffu) * 16777216.0f, dmin = h2f(f.hdr.x >> 16);
+        // d (sc_lo P_lo + sc_hi P_hi) - dmin (m_lo S_lo + m_hi S_hi)
+        const float p_hi = (float)((sc >> 8) & 0xffu) * (d1[1] + d3[3]);
+        const float p = fmaf((float)(sc & 0xffu), d0[0] + d2[2], p_hi * 0.0625f);
+        const float m = fmaf((float)(mn & 0xffu), s.x, (float)((mn >> 8) & 0xffu) * s.y);
+        return fmaf(d24, p, -(dmin * m));
+    }
+};
+
+template <>
+struct TileOps<Q6K> {
+    static constexpr int kPieces = 14;
+    static constexpr int kRows = 16;
+    static constexpr float kSumScale = 32.f / 16777216.f;   // 32 S in the units of the code sums
+    __device__ static __forceinline__ int slot(int r) {
+        const int h = r >> 4, part = (r >> 2) & 3, ih = (r >> 1) & 1, u = r & 1;
+        return (2 * h + ih) * 8 + u * 4 + part;
+    }
+    using Sums = f32x4;
+    __device__ static __forceinline__ Sums sums(const float* sx, int b, int g) {
+        return *reinterpret_cast<const f32x4*>(sx + b * 16 + 4 * g);
+    }
+    __device__ static __forceinline__ float dot(const Q6K::Frag& f, int g, u32x4 a0, u32x4 a1, Sums s) {
+#pragma clang fp contract(off)
+        u32x4 c[4][2];   // part, half of its 16 codes
+#pragma unroll
+        for (int t = 0; t < 4; ++t) {
+            uint32_t a[4], b[4];
+            Q6K::codes(f, t, a, b);
+#pragma unroll
+            for (int p = 0; p < 4; ++p) {
+                c[p][t >> 1][2 * (t & 1)] = a[p];
+                c[p][t >> 1][2 * (t & 1) + 1] = b[p];
+            }
+        }
+        const f32x4 z = {0.f, 0.f, 0.f, 0.f};
+        f32x4 d[4];
+#pragma unroll
+        for (int p = 0; p < 4; ++p) d[p] = mfma32(a0, c[p][0], z);
+#pragma unroll
+        for (int p = 0; p < 4; ++p) d[p] = mfma32(a1, c[p][1], d[p]);
+        float sc[4];
+        Q6K::scales(f, g, sc);
+        // d sum_p sc_p (P_p - 32 S_p), in units of 2^-24
+        float p = sc[0] * (d[0][0] - s.x);
+        p = fmaf(sc[1], d[1][1] - s.y, p);
+        p = fmaf(sc[2], d[2][2] - s.z, p);
+        p = fmaf(sc[3], d[3][3] - s.w, p);
+        return h2f((uint16_t)f.dbits) * 16777216.0f * p;
+    }
+};
+
+// A tile launch of type QT: tiles of kRows rows (columns past them repeat the
+// last one and are not stored), ring slots of kCopies copy instructions of 64
+// pieces.  Q4_K: 14 rows fill two copies (126 pieces); 16 rows in three
+// measured 6.39 against 5.51 us at 5120 x 5120 and 21.7 against 20.6 us for
+// gate/up 17408 x 5120.  Q6_K: 16 rows in four copies; 13 rows in three, 23.3
+// against 14.6 us at 3584 x 18944 (276 tiles on 256 CUs) and 81 against 69 us
+// at 151936 x 2560.
+template <class QT, int kMatrices>
+struct TileShape {
+    using Q = QT;
+    static constexpr int kMats = kMatrices;
+    static constexpr int kRows = TileOps<QT>::kRows, kPieces = TileOps<QT>::kPieces;
+    static constexpr int kCopies = (kRows * kPieces + kWave - 1) / kWave;
+    static constexpr int kDepth = 2;   // slots per wave; a third measured no faster
+    static constexpr int kSlot = kCopies * kWave * 16;
+    // LDS: x operands, x sums, norm scratch, zeros, the class sums of two
+    // tiles, the rings
+    __host__ __device__ static constexpr int sums(int nb) { return nb * kQK * 2; }
+    __host__ __device__ static constexpr int red(int nb) { return sums(nb) + nb * QT::kSxPerBlock * 4; }
+    __host__ __device__ static constexpr int zero(int nb) { return red(nb) + 16; }
+    __host__ __device__ static constexpr int part(int nb) { return zero(nb) + kZeroBytes; }
+    __host__ __device__ static constexpr int ring(int nb) { return part(nb) + 2 * kMats * kTileWaves * kTileCols * 4; }
+    __host__ __device__ static constexpr int bytes(int nb) { return ring(nb) + kTileWaves * kDepth * kSlot; }
+};
+
+// Waits until at most n of the wave's vector-memory operations are in flight.
+template <int n>
+__device__ __forceinline__ void wait_vm() {
+    static_assert(n < 64, "vmcnt");
+    __builtin_amdgcn_s_waitcnt(0x0f70 | (n & 15) | ((n >> 4) << 14));
+    asm volatile("" ::: "memory");
+}
+// LDS traffic of the wave done; copies in flight stay in flight.
+__device__ __forceinline__ void wait_lds() { asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory"); }
+__device__ __forceinline__ void tile_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
+
+__device__ __forceinline__ void copy16_to_lds(const uint8_t* src, uint8_t* dst_wave_base) {
+    __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)src,
+                                     (__attribute__((address_space(3))) void*)dst_wave_base, 16, 0, 0);
+}
+
+struct TileAt {
+    const uint8_t* w[2];
+    void* y;
+    int row, rows;   // first row and rows (up to 16) of the tile in its matrix
+};
+
+// The tiles wg, wg + wgs, ... of `tiles`.  tile_of(t): the matrix (its first
+// byte), first row and rows of tile t.  kMats = 2: a step list runs over the
+// blocks of the tile's rows in matrix 0, then in matrix 1 (gate and up, the
+// same rows of both).  finish(t, row, sums[kMats]): called by one lane per
+// row.  kNormIters: 0, or the input is the residual add + RMSNorm of x with at
+// most that many runs per thread (256 threads).
+template <class SH, int kNormIters, class TileOf, class Finish>
+__device__ __forceinline__ void tile_rows(const uint16_t* __restrict__ x, int nb, uint8_t* smem, int wg, int wgs,
+                                          int tiles, const NormIn& nrm, TileOf tile_of, Finish finish) {
+    using QT = typename SH::Q;
+    using OP = TileOps<QT>;
+    constexpr int kPieces = OP::kPieces, kCopies = SH::kCopies, kDepth = SH::kDepth, kMats = SH::kMats;
+    uint32_t* xp = reinterpret_cast<uint32_t*>(smem);
+    float* sx = reinterpret_cast<float*>(smem + SH::sums(nb));
+    float* red = reinterpret_cast<float*>(smem + SH::red(nb));
+    float* part = reinterpret_cast<float*>(smem + SH::part(nb));
+
+    const int lane = threadIdx.x & (kWave - 1);
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+    const int n = lane & 15, g = lane >> 4;
+    uint8_t* ring = smem + SH::ring(nb) + wave * kDepth * SH::kSlot;
+    const int row_bytes = nb * QT::kBytes;
+    int my_tiles = 0;   // at least one: wg < wgs <= tiles
+    for (int t = wg; t < tiles; t += wgs) ++my_tiles;
+    const int total = my_tiles * kMats * nb;
+    const int my_steps = wave < total ? (total - wave + kTileWaves - 1) / kTileWaves : 0;
+
+    // Copy identity: piece c * 64 + lane of a slot is 16-byte piece pc of row
+    // lr (lanes past the last piece repeat it; their LDS bytes are not read).
+    // rel: the row's offset in the tile, the last row's for rows past it.
+    int lr[kCopies], pc16[kCopies], rel[kCopies];
+#pragma unroll
+    for (int c = 0; c < kCopies; ++c) {
+        const int p = min(c * kWave + lane, SH::kRows * kPieces - 1);
+        lr[c] = p / kPieces;
+        pc16[c] = (p - lr[c] * kPieces) * 16;
+    }
+
+    // The steps of the workgroup in one list, unit (tile, matrix) by unit and
+    // block by block; wave w takes steps w, w + 8, ...  A unit's blocks that
+    // fall to one wave are the class b % 8 of its first one.
+    struct Walk { int u, b; };
+    auto first = [&]() {
+        Walk s{0, min(wave, total - 1)};
+        while (s.b >= nb) {
+            s.b -= nb;
+            ++s.u;
+        }
+        return s;
+    };
+    auto advance = [&](Walk& s) {
+        s.b += kTileWaves;
+        while (s.b >= nb) {
+            s.b -= nb;
+            ++s.u;
+        }
+    };
+    // The block rows of a step into a ring slot.  Every piece holds bytes of
+    // its block, so an aligned piece never reaches past the page of one.
+    const uint8_t* unit_base = nullptr;
+    int unit = -1;
+    auto copy = [&](const Walk& s, int slot) {
+        if (s.u != unit) {   // wave-uniform
+            unit = s.u;
+            const TileAt t = tile_of(wg + (unit / kMats) * wgs);
+            unit_base = (kMats == 2 && (unit & 1) ? t.w[1] : t.w[0]) + (size_t)t.row * row_bytes;
+#pragma unroll
+            for (int c = 0; c < kCopies; ++c) {
+                rel[c] = min(lr[c], t.rows - 1) * row_bytes;
+                if (QT::kBytes % 16 == 0) rel[c] += pc16[c];
+            }
+        }
+        const uint8_t* base = unit_base + s.b * QT::kBytes;
+        uint8_t* dst = ring + slot * SH::kSlot;
+        if constexpr (QT::kBytes % 16 == 0) {
+#pragma unroll
+            for (int c = 0; c < kCopies; ++c) copy16_to_lds(base + (uint32_t)rel[c], dst + c * kWave * 16);
+        } else {
+            const int skew = (int)((uintptr_t)base & 15);
+            base -= skew;
+#pragma unroll
+            for (int c = 0; c < kCopies; ++c)
+                copy16_to_lds(base + (uint32_t)(((rel[c] + skew) & ~15) + pc16[c]), dst + c * kWave * 16);
+        }
+    };
+
+    // x first (it arrives first), then the rings' first slots
+    constexpr int kIters = kNormIters ? kNormIters : 1;
+    u32x4 raw[kIters], dr[kIters], wr[kIters];
+    const int runs = nb * (kQK / 8);
+    if constexpr (kNormIters != 0) {
+        // by every wave, though only waves 0-3 use them: loads in a branch
+        // would make the wait for them cover the rings' copies too
+        const uint16_t* dp = nrm.d ? nrm.d : x;
+#pragma unroll
+        for (int i = 0; i < kIters; ++i) {
+            const size_t r = (size_t)staged_run(runs, i, (int)threadIdx.x & (kBlock - 1)) * 8;
+            raw[i] = *reinterpret_cast<const u32x4*>(x + r);
+            dr[i] = *reinterpret_cast<const u32x4*>(dp + r);
+            wr[i] = *reinterpret_cast<const u32x4*>(nrm.w + r);
+        }
+    } else {
+        for (int r0 = wave * kWave; r0 < runs; r0 += kTileBlock)
+            if (r0 + lane < runs) copy16_to_lds(reinterpret_cast<const uint8_t*>(x) + (size_t)(r0 + lane) * 16, smem + r0 * 16);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    // unconditional (a wave with fewer steps repeats its last one), so that
+    // the copies in flight are known.  With the norm, the compiler's wait for
+    // its register loads covers every copy issued before: one slot goes
+    // before it, the others right behind it, in flight over the norm.
+    Walk ahead = first();
+    constexpr int kBefore = kNormIters ? 1 : kDepth;
+    auto copy_first = [&](int from, int to) {
+#pragma unroll
+        for (int d = from; d < to; ++d) {
+            copy(ahead, d);
+            if (d + 1 < my_steps) advance(ahead);
+        }
+    };
+    copy_first(0, kBefore);
+    if constexpr (kNormIters != 0) {
+        // an empty asm that needs every loaded value
+#pragma unroll
+        for (int i = 0; i < kIters; ++i) asm volatile("" : "+v"(raw[i]), "+v"(dr[i]), "+v"(wr[i]));
+        copy_first(kBefore, kDepth);
+        __builtin_amdgcn_sched_barrier(0);
+    }
+    int issued = kDepth;
+    if ((int)threadIdx.x < kZeroBytes / 4) reinterpret_cast<uint32_t*>(smem + SH::zero(nb))[threadIdx.x] = 0u;
+
+    auto put = [&](u32x4 v, int r) {
+        *reinterpret_cast<u32x4*>(xp + (size_t)((r & ~31) + OP::slot(r & 31)) * 4) = permute_x8(v);
+        stage_sums8<QT::kSumLayout>(v, r, sx, OP::kSumScale);
+    };
+    if constexpr (kNormIters != 0) {
+        if (wave < kWavesPerBlock) {
+            // the order of norm_block_sum's callers (256 threads)
+            const bool has_d = nrm.d != nullptr;
+            float s = 0.f;
+#pragma unroll
+            for (int i = 0; i < kIters; ++i) {
+                const bool own = i * kBlock + (int)threadIdx.x < runs;
+                raw[i] = add_run(raw[i], dr[i], has_d);
+                if (!own) raw[i] = u32x4{0u, 0u, 0u, 0u};   // adds nothing
+                s = sq_run(raw[i], s);
+            }
+            if (nrm.xs_out && wg == 0) {
+#pragma unroll
+                for (int i = 0; i < kIters; ++i) {
+                    const int r = i * kBlock + (int)threadIdx.x;
+                    if (r < runs) *reinterpret_cast<u32x4*>(nrm.xs_out + (size_t)r * 8) = raw[i];
+                }
+            }
+            s = wave_sum(s);
+            if (lane == 0) red[wave] = s;
+            tile_barrier();
+            const float inv = rsqrtf((((red[0] + red[1]) + red[2]) + red[3]) / (float)(runs * 8) + nrm.eps);
+#pragma unroll
+            for (int i = 0; i < kIters; ++i) {
+                const int r = i * kBlock + (int)threadIdx.x;
+                if (r < runs) put(norm_run(raw[i], wr[i], inv), r);
+            }
+        } else {
+            tile_barrier();
+        }
+    } else {
+        // this wave's runs are in LDS once only the ring copies are in flight
+        // (a wave's 64 runs are two whole super-blocks, permuted in place:
+        // every lane has read before any lane writes)
+        wait_vm<kDepth * kCopies>();
+        for (int r0 = wave * kWave; r0 < runs; r0 += kTileBlock) {
+            const int r = r0 + lane;
+            u32x4 v = {0u, 0u, 0u, 0u};
+            if (r < runs) v = *reinterpret_cast<const u32x4*>(xp + (size_t)r * 4);
+            wait_lds();
+            __builtin_amdgcn_wave_barrier();
+            if (r < runs) put(v, r);
+        }
+    }
+    tile_barrier();
+
+    // A operand address: slot lane & 3 of this lane group's quarter, or zeros
+    const bool a_live = ((lane & 15) >> 2) == g;
+    const int a_off = a_live ? g * 128 + (lane & 3) * 16 : SH::zero(nb);
+    const int a_mask = a_live ? -1 : 0;
+    Walk cur = first();
+    int done = 0, slot = 0;
+    for (int k = 0; k < my_tiles; ++k) {
+        const TileAt t = tile_of(wg + k * wgs);
+        const int col = min(n, t.rows - 1);
+        float* pt = part + (k & 1) * kMats * kTileWaves * kTileCols;
+#pragma unroll
+        for (int m = 0; m < kMats; ++m) {
+            if (done >= my_steps || cur.u != k * kMats + m) continue;   // wave-uniform
+            // low address bits of the lane's row (a Q6_K block's offset in its first piece)
+            const uint32_t row_at = QT::kBytes % 16 ? (uint32_t)(uintptr_t)t.w[m] + (uint32_t)(t.row + col) * (uint32_t)row_bytes : 0u;
+            const int cls = cur.b;
+            float acc = 0.f;
+            do {
+                const int b = cur.b;
+                const int later = issued - done - 1;   // steps in flight behind this one
+                if (later >= kDepth - 1) wait_vm<(kDepth - 1) * kCopies>();
+                else wait_vm<0>();
+                const uint8_t* sb = ring + slot * SH::kSlot + col * kPieces * 16;
+                if (QT::kBytes % 16) sb += (row_at + (uint32_t)(b * QT::kBytes)) & 15u;
+                const typename QT::Frag f = QT::load(sb, g);
+                const int a_at = ((b * kQK * 2) & a_mask) | a_off;
+                const u32x4 a0 = *reinterpret_cast<const u32x4*>(smem + a_at);
+                const u32x4 a1 = *reinterpret_cast<const u32x4*>(smem + a_at + 64);
+                const typename OP::Sums xs = OP::sums(sx, b, g);
+                wait_lds();
+                __builtin_amdgcn_sched_barrier(0);
+                if (issued < my_steps) {   // the slot is read: refill it
+                    copy(ahead, slot);
+                    advance(ahead);
+                    ++issued;
+                }
+                __builtin_amdgcn_sched_barrier(0);
+                acc += OP::dot(f, g, a0, a1, xs);
+                slot = slot + 1 == kDepth ? 0 : slot + 1;
+                ++done;
+                advance(cur);
+            } while (done < my_steps && cur.u == k * kMats + m);
+            acc = sum32(sum16(acc));   // the row's four quarters
+            if (g == 0) pt[(m * kTileWaves + cls) * kTileCols + n] = acc;
+        }
+        tile_barrier();   // the tile's class sums are in LDS
+        if (wave == (k & (kTileWaves - 1))) {
+            float sum[kMats];
+#pragma unroll
+            for (int m = 0; m < kMats; ++m) {
+                // classes g and g + 4 of the row, then the lane groups
+                const float* c = pt + m * kTileWaves * kTileCols + n;
+                const float v0 = g < nb ? c[g * kTileCols] : 0.f, v1 = g + 4 < nb ? c[(g + 4) * kTileCols] : 0.f;
+                sum[m] = sum32(sum16(v0 + v1));
+            }
+            if (g == 0 && n < t.rows) finish(t, t.row + n, sum);
+        }
+    }
+    wait_vm<0>();   // no copy outlives the workgroup's LDS
+}
+
+// Tiles of up to three matrices of one type that read the same x: tile t
+// belongs to the first matrix s with t < end[s].
+struct TileSet {
+    RowSet rs;
+    int end[3];
+};
+template <class QT>
+constexpr int tiles_of(int rows) { return (rows + TileOps<QT>::kRows - 1) / TileOps<QT>::kRows; }
+template <class QT>
+TileSet make_tile_set(const RowSet& rs) {
+    TileSet ts{rs, {}};
+    for (int i = 0, rows = 0, tiles = 0; i < 3; ++i) {
+        tiles += tiles_of<QT>(rs.end[i] - rows);
+        rows = rs.end[i];
+        ts.end[i] = tiles;
+    }
+    return ts;
+}
+// The value of entry 0, 1 or 2.  As assignments, since a conditional
+// expression of three members is an lvalue: the compiler selects the address
+// and keeps the struct in scratch memory.
+template <typename T>
+__device__ __forceinline__ T pick3(bool s1, bool s2, T v0, T v1, T v2) {
+    T r = v0;
+    if (s1) r = v1;
+    if (s2) r = v2;
+    return r;
+}
+
+// tile t of a set, in registers
+template <int kRows>
+struct SetTiles {
+    const uint8_t *w0, *w1, *w2;
+    void *y0, *y1, *y2;
+    int e0, e1, n0, n1, n2;
+    __device__ __forceinline__ explicit SetTiles(const TileSet& ts)
+        : w0(ts.rs.w[0]), w1(ts.rs.w[1]), w2(ts.rs.w[2]), y0(ts.rs.y[0]), y1(ts.rs.y[1]), y2(ts.rs.y[2]),
+          e0(ts.end[0]), e1(ts.end[1]), n0(ts.rs.end[0]), n1(ts.rs.end[1] - ts.rs.end[0]),
+          n2(ts.rs.end[2] - ts.rs.end[1]) {}
+    __device__ __forceinline__ TileAt operator()(int t) const {
+        const bool s1 = t >= e0, s2 = t >= e1;
+        const uint8_t* w = pick3(s1, s2, w0, w1, w2);
+        const int row = (t - pick3(s1, s2, 0, e0, e1)) * kRows;
+        return TileAt{{w, w}, pick3(s1, s2, y0, y1, y2), row, min(kRows, pick3(s1, s2, n0, n1, n2) - row)};
+    }
+};
+
+template <class SH, int kNormIters>
+__device__ __forceinline__ void tile_set(const TileSet& ts, const uint16_t* x, int nb, int f32, uint8_t* smem, int wg,
+                                         int wgs, const NormIn& nrm) {
+    tile_rows<SH, kNormIters>(x, nb, smem, wg, wgs, ts.end[2], nrm, SetTiles<SH::kRows>(ts),
+                              [f32](const TileAt& t, int row, const float (&s)[1]) {
+                                  if (f32) store_y<true>(t.y, row, s[0]);
+                                  else store_y<false>(t.y, row, s[0]);
+                              });
+}
+
+template <class SH, int kNormIters>
+__global__ __launch_bounds__(kTileBlock, 4) void matvec_tile_kernel(TileSet ts, const uint16_t* __restrict__ x, int nb,
+                                                                    int f32, NormIn nrm) {
+    extern __shared__ __align__(16) uint8_t smem[];
+    tile_set<SH, kNormIters>(ts, x, nb, f32, smem, blockIdx.x, gridDim.x, nrm);
+}
+
+// Q4_K tiles on blocks [0, blocks_a), Q6_K tiles on the rest.
+template <class SA, class SB, int kNormIters>
+__global__ __launch_bounds__(kTileBlock, 4) void matvec_tile_group_kernel(TileSet a, TileSet b, int blocks_a,
+                                                                          const uint16_t* __restrict__ x, int nb,
+                                                                          NormIn nrm) {
+    extern __shared__ __align__(16) uint8_t smem[];
+    if ((int)blockIdx.x < blocks_a) {
+        tile_set<SA, kNormIters>(a, x, nb, 0, smem, blockIdx.x, blocks_a, nrm);
+    } else {
+        NormIn no_sum = nrm;   // the Q4_K blocks store the residual sum
+        no_sum.xs_out = nullptr;
+        tile_set<SB, kNormIters>(b, x, nb, 0, smem, blockIdx.x - blocks_a, gridDim.x - blocks_a, no_sum);
+    }
+}
+
+// ffn_gate, ffn_up and SwiGLU: a tile's steps run over both matrices.
+template <class SH, int kNormIters>
+__global__ __launch_bounds__(kTileBlock, 4) void matvec_tile_gate_up_kernel(const uint8_t* __restrict__ wg,
+                                                                            const uint8_t* __restrict__ wu,
+                                                                            const uint16_t* __restrict__ x,
+                                                                            uint16_t* __restrict__ act, int nb,
+                                                                            int tiles, int N, NormIn nrm) {
+    extern __shared__ __align__(16) uint8_t smem[];
+    tile_rows<SH, kNormIters>(
+        x, nb, smem, blockIdx.x, gridDim.x, tiles, nrm,
+        [=](int t) { return TileAt{{wg, wu}, nullptr, t * SH::kRows, min(SH::kRows, N - t * SH::kRows)}; },
+        [=](const TileAt&, int row, const float (&s)[2]) {
+            const float g = h2f(f2h_rne(s[0])), u = h2f(f2h_rne(s[1]));
+            act[row] = f2h_rne(g / (1.0f + expf(-g)) * u);
+        });
+}
+
 int device_cus() {
     static int cus = 0;
     if (!cus) {
@@ -792,6 +1322,105 @@ void launch_rows_once(const RowSet& rs, const uint16_t* x, size_t lds, const Nor
     const int grid = (units + M * kWavesPerBlock - 1) / (M * kWavesPerBlock);
     launch_kernel((matvec_stream_kernel<QT, kF32, 1, M, kSegs, false, kNorm, NB>), dim3(grid), dim3(kBlock), lds,
                   stream, rs, x, K, nrm);
+}
+
+// Super-block counts whose Q4_K / Q6_K rows go through the tile kernels: 20
+// (hidden 5120) and every count without a streaming instantiation.  Measured
+// against the streaming kernels (us, streaming -> tile, back-to-back launches
+// over rotated weights): 20 blocks Q4_K 5120 rows 7.6 -> 5.8, gate/up with the
+// norm 2 x 17408 24.2 -> 19.9 and 2 x 25600 30.4 -> 29.0, grouped q/k/v 9.9 ->
+// 10.3; against the flat walk over super-blocks that served other counts:
+// Q4_K 18944 x 3584 13.2 -> 10.2, 3584 x 3584 5.4 -> 4.1, 512 x 3584 4.6 ->
+// 3.4, Q6_K 3584 x 18944 22.6 -> 14.4.  The streaming kernels stay where they
+// were faster: 10 blocks (grouped q/k/v 6.1 against 8.1, though gate/up 9.7
+// against 8.8), 12 and 24 (Q6_K 1024 rows 3.2 against 4.7, 2048 rows 5.4
+// against 6.9), 38 (8.8 against 9.0), 68 and 100 (5120 rows 18.1 against 22.2
+// and 24.9 against 31: 320 tiles on 256 CUs).
+__host__ __device__ constexpr bool tile_length(int nb) {
+    switch (nb) {
+        case 4: case 8: case 10: case 12: case 16: case 24: case 32: case 38: case 48: case 64: case 68: case 100: return false;
+        default: return true;
+    }
+}
+
+constexpr int kLdsPerCu = 160 * 1024;
+
+// More than 64 KB of LDS is asked for per kernel and device, once.
+template <typename Kernel>
+hipError_t allow_lds(Kernel kernel) {
+    static std::atomic<uint64_t> done{0};
+    int dev = 0;
+    hipError_t e = hipGetDevice(&dev);
+    if (e != hipSuccess) return e;
+    const uint64_t bit = (uint64_t)1 << (dev & 63);
+    if (done.load(std::memory_order_acquire) & bit) return hipSuccess;
+    e = hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, kLdsPerCu);
+    if (e == hipSuccess) done.fetch_or(bit, std::memory_order_release);
+    return e;
+}
+
+// Two workgroups per CU where the LDS of two fits, never more than tiles.
+int tile_grid(int tiles, int lds) { return std::min(tiles, device_cus() * (2 * lds <= kLdsPerCu ? 2 : 1)); }
+
+// kNormIters: the norm prologue's runs of eight inputs per thread of 256, 3
+// for its only tile length (20 blocks), 0 without it
+template <bool kNorm, typename F>
+hipError_t with_norm_iters(int nb, F f) {
+    if constexpr (!kNorm) return f(std::integral_constant<int, 0>{});
+    else if (nb == 20) return f(std::integral_constant<int, 3>{});
+    else return hipErrorInvalidValue;
+}
+
+template <class QT, bool kNorm>
+hipError_t launch_tile(int nb, const RowSet& rs, const uint16_t* x, bool f32, const NormIn& nrm, hipStream_t stream) {
+    return with_norm_iters<kNorm>(nb, [&](auto it) {
+        using SH = TileShape<QT, 1>;
+        auto kernel = matvec_tile_kernel<SH, decltype(it)::value>;
+        const hipError_t e = allow_lds(kernel);
+        if (e != hipSuccess) return e;
+        const TileSet ts = make_tile_set<QT>(rs);
+        const int lds = SH::bytes(nb);
+        launch_kernel(kernel, dim3(tile_grid(ts.end[2], lds)), dim3(kTileBlock), (size_t)lds, stream, ts, x, nb,
+                      (int)f32, nrm);
+        return hipGetLastError();
+    });
+}
+
+template <bool kNorm>
+hipError_t launch_tile_mixed(int nb, const RowSet& a, const RowSet& b, const uint16_t* x, const NormIn& nrm,
+                             hipStream_t stream) {
+    using SA = TileShape<Q4K, 1>;
+    using SB = TileShape<Q6K, 1>;
+    const TileSet ta = make_tile_set<Q4K>(a), tb = make_tile_set<Q6K>(b);
+    const int lds = std::max(SA::bytes(nb), SB::bytes(nb));
+    const int grid = std::max(2, tile_grid(ta.end[2] + tb.end[2], lds));
+    // blocks split in proportion to the bytes each set streams
+    const double wa = (double)a.end[2] * Q4K::kBytes, wb = (double)b.end[2] * Q6K::kBytes;
+    int ga = (int)(grid * wa / (wa + wb) + 0.5);
+    ga = std::max(1, std::min(ga, std::min(grid - 1, ta.end[2])));
+    const int gb = std::max(1, std::min(grid - ga, tb.end[2]));
+    return with_norm_iters<kNorm>(nb, [&](auto it) {
+        auto kernel = matvec_tile_group_kernel<SA, SB, decltype(it)::value>;
+        const hipError_t e = allow_lds(kernel);
+        if (e != hipSuccess) return e;
+        launch_kernel(kernel, dim3(ga + gb), dim3(kTileBlock), (size_t)lds, stream, ta, tb, ga, x, nb, nrm);
+        return hipGetLastError();
+    });
+}
+
+template <class QT, bool kNorm>
+hipError_t launch_tile_gate_up(const uint8_t* wg, const uint8_t* wu, const uint16_t* x, uint16_t* act, int nb, int N,
+                               const NormIn& nrm, hipStream_t stream) {
+    return with_norm_iters<kNorm>(nb, [&](auto it) {
+        using SH = TileShape<QT, 2>;
+        auto kernel = matvec_tile_gate_up_kernel<SH, decltype(it)::value>;
+        const hipError_t e = allow_lds(kernel);
+        if (e != hipSuccess) return e;
+        const int lds = SH::bytes(nb), tiles = tiles_of<QT>(N);
+        launch_kernel(kernel, dim3(tile_grid(tiles, lds)), dim3(kTileBlock), (size_t)lds, stream, wg, wu, x, act, nb,
+                      tiles, N, nrm);
+        return hipGetLastError();
+    });
 }
 
 // Rows ending in a partial wave step (NB blocks, not a multiple of 16).
@@ -843,24 +1472,30 @@ bool launch_stream_for(int nb, const RowSet& rs, const uint16_t* x, size_t lds, 
         case 64: launch_stream<QT, kF32, 4, 1, kSegs, kNorm>(rs, x, lds, nrm, stream); return true;
         // the other Qwen3 row lengths: hidden 1024 / 2048 / 2560 / 5120, FFN
         // 3072 / 6144 / 9728 / 17408 / 25600 (the last two without the norm
-        // prologue, which only hidden-sized inputs take)
+        // prologue, which only hidden-sized inputs take); 20 blocks here only
+        // as fp16 (Q4_K / Q6_K: the tile kernels), 68 and 100 only quantized
+        // (fp16: 32 registers of weights per step in flight)
         case 4: launch_partial<QT, kF32, kSegs, kNorm, 4>(rs, x, lds, nrm, stream); return true;
         case 8: launch_partial<QT, kF32, kSegs, kNorm, 8>(rs, x, lds, nrm, stream); return true;
         case 10: launch_partial<QT, kF32, kSegs, kNorm, 10>(rs, x, lds, nrm, stream); return true;
         case 12: launch_partial<QT, kF32, kSegs, kNorm, 12>(rs, x, lds, nrm, stream); return true;
-        case 20: launch_partial<QT, kF32, kSegs, kNorm, 20>(rs, x, lds, nrm, stream); return true;
         case 24: launch_partial<QT, kF32, kSegs, kNorm, 24>(rs, x, lds, nrm, stream); return true;
         case 38: launch_partial<QT, kF32, kSegs, kNorm, 38>(rs, x, lds, nrm, stream); return true;
-        case 68:
-            if constexpr (kNorm || 5 > QT::kMaxSteps) return false;
-            else launch_partial<QT, kF32, kSegs, kNorm, 68>(rs, x, lds, nrm, stream);
-            return true;
-        case 100:
-            if constexpr (kNorm || 7 > QT::kMaxSteps) return false;
-            else launch_partial<QT, kF32, kSegs, kNorm, 100>(rs, x, lds, nrm, stream);
-            return true;
-        default: return false;
+        default: break;
     }
+    if constexpr (std::is_same<QT, F16>::value) {
+        if (nb == 20) {
+            launch_partial<QT, kF32, kSegs, kNorm, 20>(rs, x, lds, nrm, stream);
+            return true;
+        }
+    } else if constexpr (!kNorm) {
+        switch (nb) {
+            case 68: launch_partial<QT, kF32, kSegs, kNorm, 68>(rs, x, lds, nrm, stream); return true;
+            case 100: launch_partial<QT, kF32, kSegs, kNorm, 100>(rs, x, lds, nrm, stream); return true;
+            default: break;
+        }
+    }
+    return false;
 }
 
 // staged x (fp16 pairs), the x-sum table and 4 floats of reduction scratch
@@ -874,16 +1509,20 @@ constexpr NormIn kNoNorm{nullptr, nullptr, nullptr, 0.f};
 template <class QT, bool kF32>
 hipError_t launch_matvec(const uint8_t* w, const uint16_t* x, void* y, int K, int N, hipStream_t stream) {
     const int nb = K / kQK;
-    const size_t lds = lds_bytes<QT>(K);
     const RowSet rs{{w, w, w}, {y, y, y}, {N, N, N}};
+    if constexpr (!std::is_same<QT, F16>::value) {
+        if (tile_length(nb)) return launch_tile<QT, false>(nb, rs, x, kF32, kNoNorm, stream);
+    }
+    const size_t lds = lds_bytes<QT>(K);
     if (!launch_stream_for<QT, kF32, 1>(nb, rs, x, lds, kNoNorm, stream)) {
-        // any other length: flat walk over the super-blocks of 4 rows
+        if constexpr (!std::is_same<QT, F16>::value) return hipErrorInvalidValue;   // not reached: tile_length
+        // any other fp16 length: flat walk over the 256-value blocks of 4 rows
         constexpr int kRows = 4;
         // floor(f / nb) == (f * magic) >> 32 for every f < 2^20 (nb <= 112)
         const uint64_t magic = ((uint64_t)1 << 32) / (uint64_t)nb + 1u;
         const int rows_per_block = kRows * kWavesPerBlock;
         const int grid = (N + rows_per_block - 1) / rows_per_block;
-        launch_kernel((matvec_flat_kernel<QT, kF32, kRows>), dim3(grid), dim3(kBlock), lds, stream, w, x, y, K,
+        launch_kernel((matvec_flat_kernel<F16, kF32, kRows>), dim3(grid), dim3(kBlock), lds, stream, w, x, y, K,
                       N, magic);
     }
     return hipGetLastError();
@@ -893,7 +1532,11 @@ template <class QT, bool kF32>
 hipError_t launch_matvec_prologue(const uint8_t* w, const uint16_t* x, const NormIn& nrm, void* y, int K, int N,
                                   hipStream_t stream) {
     const RowSet rs{{w, w, w}, {y, y, y}, {N, N, N}};
-    if (!launch_stream_for<QT, kF32, 1, true>(K / kQK, rs, x, lds_bytes<QT>(K), nrm, stream))
+    const int nb = K / kQK;
+    if constexpr (!std::is_same<QT, F16>::value) {
+        if (tile_length(nb)) return launch_tile<QT, true>(nb, rs, x, kF32, nrm, stream);
+    }
+    if (!launch_stream_for<QT, kF32, 1, true>(nb, rs, x, lds_bytes<QT>(K), nrm, stream))
         return hipErrorInvalidValue;
     return hipGetLastError();
 }
@@ -928,48 +1571,63 @@ void launch_group_mixed(const RowSet& a, const RowSet& b, const uint16_t* x, int
 }
 
 template <bool kNorm>
-bool launch_group(int nb, RowSet (&set)[2], const int (&cnt)[2], bool f16, const uint16_t* x, int K,
-                  const NormIn& nrm, hipStream_t s) {
-    if (f16) return launch_stream_for<F16, false, 3, kNorm>(nb, set[0], x, lds_bytes<F16>(K), nrm, s);
-    if (cnt[1] == 0) return launch_stream_for<Q4K, false, 3, kNorm>(nb, set[0], x, lds_bytes<Q4K>(K), nrm, s);
-    if (cnt[0] == 0) return launch_stream_for<Q6K, false, 3, kNorm>(nb, set[1], x, lds_bytes<Q6K>(K), nrm, s);
-    switch (nb) {
-        case 16: launch_group_mixed<1, 1, kNorm>(set[0], set[1], x, K, nrm, s); return true;
-        case 32: launch_group_mixed<2, 1, kNorm>(set[0], set[1], x, K, nrm, s); return true;
-        case 48: launch_group_mixed<3, 1, kNorm>(set[0], set[1], x, K, nrm, s); return true;
-        case 64: launch_group_mixed<4, 1, kNorm>(set[0], set[1], x, K, nrm, s); return true;
-        case 4: launch_group_mixed<1, 1, kNorm, 4>(set[0], set[1], x, K, nrm, s); return true;
-        case 8: launch_group_mixed<1, 1, kNorm, 8>(set[0], set[1], x, K, nrm, s); return true;
-        case 10: launch_group_mixed<1, 1, kNorm, 10>(set[0], set[1], x, K, nrm, s); return true;
-        case 12: launch_group_mixed<1, 1, kNorm, 12>(set[0], set[1], x, K, nrm, s); return true;
-        case 20: launch_group_mixed<2, 1, kNorm, 20>(set[0], set[1], x, K, nrm, s); return true;
-        case 24: launch_group_mixed<2, 1, kNorm, 24>(set[0], set[1], x, K, nrm, s); return true;
-        case 38: launch_group_mixed<3, 1, kNorm, 38>(set[0], set[1], x, K, nrm, s); return true;
-        default: return false;
+hipError_t launch_group(int nb, RowSet (&set)[2], const int (&cnt)[2], bool f16, const uint16_t* x, int K,
+                        const NormIn& nrm, hipStream_t s) {
+    if (!f16 && tile_length(nb)) {
+        if (cnt[1] == 0) return launch_tile<Q4K, kNorm>(nb, set[0], x, false, nrm, s);
+        if (cnt[0] == 0) return launch_tile<Q6K, kNorm>(nb, set[1], x, false, nrm, s);
+        return launch_tile_mixed<kNorm>(nb, set[0], set[1], x, nrm, s);
     }
+    bool ok = true;
+    if (f16) ok = launch_stream_for<F16, false, 3, kNorm>(nb, set[0], x, lds_bytes<F16>(K), nrm, s);
+    else if (cnt[1] == 0) ok = launch_stream_for<Q4K, false, 3, kNorm>(nb, set[0], x, lds_bytes<Q4K>(K), nrm, s);
+    else if (cnt[0] == 0) ok = launch_stream_for<Q6K, false, 3, kNorm>(nb, set[1], x, lds_bytes<Q6K>(K), nrm, s);
+    else
+        switch (nb) {
+            case 16: launch_group_mixed<1, 1, kNorm>(set[0], set[1], x, K, nrm, s); break;
+            case 32: launch_group_mixed<2, 1, kNorm>(set[0], set[1], x, K, nrm, s); break;
+            case 48: launch_group_mixed<3, 1, kNorm>(set[0], set[1], x, K, nrm, s); break;
+            case 64: launch_group_mixed<4, 1, kNorm>(set[0], set[1], x, K, nrm, s); break;
+            case 4: launch_group_mixed<1, 1, kNorm, 4>(set[0], set[1], x, K, nrm, s); break;
+            case 8: launch_group_mixed<1, 1, kNorm, 8>(set[0], set[1], x, K, nrm, s); break;
+            case 10: launch_group_mixed<1, 1, kNorm, 10>(set[0], set[1], x, K, nrm, s); break;
+            case 12: launch_group_mixed<1, 1, kNorm, 12>(set[0], set[1], x, K, nrm, s); break;
+            case 24: launch_group_mixed<2, 1, kNorm, 24>(set[0], set[1], x, K, nrm, s); break;
+            case 38: launch_group_mixed<3, 1, kNorm, 38>(set[0], set[1], x, K, nrm, s); break;
+            default: ok = false;
+        }
+    return ok ? hipGetLastError() : hipErrorInvalidValue;
 }
 
 template <class QT, bool kNorm>
 hipError_t launch_gate_up_t(const uint8_t* wg, const uint8_t* wu, const uint16_t* x, uint16_t* act, int K, int N,
                           const NormIn& nrm, hipStream_t stream) {
+    const int nb = K / kQK;
+    if constexpr (!std::is_same<QT, F16>::value) {
+        if (tile_length(nb)) return launch_tile_gate_up<QT, kNorm>(wg, wu, x, act, nb, N, nrm, stream);
+    }
     const size_t lds = lds_bytes<QT>(K) + sizeof(int);   // + the unit counter
     int grid = device_cus();
-    const int nb = K / kQK;
     const int per_unit = pack_rows(nb, QT::kSbPerStep);
     const int units = (N + per_unit - 1) / per_unit;
     const int need = (units + kGateUpWaves - 1) / kGateUpWaves;
     if (grid > need) grid = need;
     const dim3 g(grid), b(kGateUpBlock);
-    switch (K / kQK) {
+    switch (nb) {
         case 16: launch_kernel((matvec_gate_up_kernel<QT, 1, kNorm>), g, b, lds, stream, wg, wu, x, act, K, N, nrm); break;
         case 32: launch_kernel((matvec_gate_up_kernel<QT, 2, kNorm>), g, b, lds, stream, wg, wu, x, act, K, N, nrm); break;
         // rows shorter than one wave step (Qwen3-0.6B: hidden 1024; 1.7B: 2048;
-        // 4B: 2560), and hidden 5120 (Qwen3-14B / 32B)
+        // 4B: 2560), and hidden 5120 (Qwen3-14B / 32B) as fp16
         case 4: launch_kernel((matvec_gate_up_kernel<QT, 1, kNorm, 4>), g, b, lds, stream, wg, wu, x, act, K, N, nrm); break;
         case 8: launch_kernel((matvec_gate_up_kernel<QT, 1, kNorm, 8>), g, b, lds, stream, wg, wu, x, act, K, N, nrm); break;
         case 12: launch_kernel((matvec_gate_up_kernel<QT, 1, kNorm, 12>), g, b, lds, stream, wg, wu, x, act, K, N, nrm); break;
         case 10: launch_kernel((matvec_gate_up_kernel<QT, 1, kNorm, 10>), g, b, lds, stream, wg, wu, x, act, K, N, nrm); break;
-        case 20: launch_kernel((matvec_gate_up_kernel<QT, 2, kNorm, 20>), g, b, lds, stream, wg, wu, x, act, K, N, nrm); break;
+        case 20:
+            if constexpr (std::is_same<QT, F16>::value) {
+                launch_kernel((matvec_gate_up_kernel<QT, 2, kNorm, 20>), g, b, lds, stream, wg, wu, x, act, K, N, nrm);
+                break;
+            }
+            return hipErrorInvalidValue;   // not reached: tile_length
         default: return hipErrorInvalidValue;
     }
     return hipGetLastError();
@@ -1057,9 +1715,8 @@ hipError_t launch_matvec_group(int count, const int* kinds, const uint8_t* const
             set[t].end[j] = set[t].end[j - 1];
         }
     const int nb = K / kQK;
-    const bool ok = norm ? launch_group<true>(nb, set, cnt, f16 != 0, x, K, *norm, s)
-                         : launch_group<false>(nb, set, cnt, f16 != 0, x, K, kNoNorm, s);
-    return ok ? hipGetLastError() : hipErrorInvalidValue;
+    return norm ? launch_group<true>(nb, set, cnt, f16 != 0, x, K, *norm, s)
+                : launch_group<false>(nb, set, cnt, f16 != 0, x, K, kNoNorm, s);
 }
 
 // kind 4: Q4_K, 6: Q6_K, 1: fp16; in_features 1024, 2048, 3072, 4096 or

@@ -184,3 +184,36 @@ def test_rows_permute_with_weights(hip):
     y = dy.download(np.float32, n)
     hip.device.matvec("q6k", hip.DeviceArray.from_numpy(np.ascontiguousarray(w[perm])), dx, dy, k, n, f32_out=True)
     np.testing.assert_array_equal(dy.download(np.float32, n), y[perm])
+
+
+# Rows of the block counts that run on the tile kernels (tiles of 14 Q4_K or
+# 16 Q6_K rows, blocks dealt to eight waves): row counts around a tile and its
+# neighbours, block counts below, at and beyond the eight waves and up to the
+# largest, many tiles per workgroup.
+TILE_ROWS = [1, 13, 14, 15, 16, 17, 33]
+TILE_K = [256, 768, 1792, 2304, 5120, 18944, 28416]
+
+
+@pytest.mark.parametrize("kind", ["q4k", "q6k"])
+@pytest.mark.parametrize("k", TILE_K)
+def test_tile_rows_match_oracle(hip, orc, kind, k):
+    for n in TILE_ROWS + ([20011] if k == 768 else []):
+        print(f"[tile matvec] kind={kind} n={n} k={k}", flush=True)
+        w, x = _inputs(hip, kind, n, k, seed=3 * n + k)
+        # Q6_K weights are 4-byte aligned, so try an offset inside a 16-byte piece
+        off = 4 if kind == "q6k" and n % 2 else 0
+        dw = hip.DeviceArray.from_numpy(np.concatenate([np.zeros(off, np.uint8), w]))
+        dx = hip.DeviceArray.from_numpy(x)
+        dy = hip.DeviceArray(n * 4 + 64)
+        dy.zero()
+        hip.device.matvec(kind, dw.at(off), dx, dy, k, n, f32_out=True)
+        got = dy.download(np.float32, n + 16)
+        assert not got[n:].any(), "wrote past the last row"
+        ref = orc.matvec(kind, w, x, k, n)
+        # fp32 sums of k products: a few ulps per addition level of the terms
+        wf = np.abs(orc.dequant_f32(kind, w, n * k).reshape(n, k).astype(np.float64))
+        bound = 2.0 ** -20 * (wf @ np.abs(x.view(np.float16).astype(np.float64))) + 1e-6
+        assert np.all(np.abs(got[:n] - ref) <= bound), float(np.max(np.abs(got[:n] - ref) / bound))
+        # the fp16 form stores the same sums, rounded
+        hip.device.matvec(kind, dw.at(off), dx, dy, k, n)
+        assert np.array_equal(dy.download(np.uint16, n), got[:n].astype(np.float16).view(np.uint16))
