@@ -11,16 +11,11 @@
 //  * One workgroup (4 waves) per (position chunk, kv head, sequence); it
 //    serves every query head of the GQA group, so K and V are read from HBM
 //    once per kv head (the reference re-reads them per query head).
-//  * Each wave streams tiles of positions: coalesced 128-bit loads of the K
-//    and V rows into registers, staged through a wave-private LDS tile, with
-//    the next tile's loads issued before the current tile is consumed.
-//  * Scores: lane = (position, head); q of the lane's head lives in VGPRs as
-//    fp16 pairs and v_dot2_f32_f16 accumulates in fp32.  The running max and
-//    sum of the online softmax are butterflies over the lanes of one head.
+//  * Each wave streams tiles of positions with the next tile's loads issued
+//    before the current one is consumed; both products run on the matrix
+//    cores, for every head_dim and group (the padding columns cost nothing
+//    that bounds the kernel: it waits for memory and LDS, not for MFMA).
 //    Exponentials are taken in base 2 with log2(e) folded into the scale.
-//  * Values: lane = (position group, 8-dim slice) accumulating every head of
-//    the group, so each staged V row is read from LDS once per lane group;
-//    p * V accumulates in fp32 and the groups are summed in the final merge.
 //  * The four waves merge in LDS; a chunk writes (max, sum, acc[head_dim])
 //    per head and a second kernel merges the chunks of each query head by
 //    log-sum-exp.  A sequence that fits one chunk is written directly.
@@ -41,35 +36,6 @@ constexpr int kBlock = 256;
 constexpr int kWaves = kBlock / kWave;
 constexpr int kMaxSplits = 512;   // plan_attention never makes more chunks
 
-template <int HD, int GP>
-struct Cfg {
-    static_assert(HD == 64 || HD == 128, "head_dim");
-    static_assert(GP == 1 || GP == 2 || GP == 4 || GP == 8, "group");
-    static constexpr int kChunks = HD / 8;                 // 16-byte slices per row
-    static constexpr int kTP = (64 / GP) < 32 ? 64 / GP : 32;   // positions per tile
-    static constexpr int kStride = HD + 8;                 // padded LDS row (halves)
-    static constexpr int kRowsPerLoad = kWave / kChunks;
-    static constexpr int kLoads = kTP / kRowsPerLoad;      // per tile, for K and for V
-    // value phase: lane = (position group, 8-dim slice), every head of the group
-    static constexpr int kVGroups = kWave / kChunks;
-    static constexpr int kVPerLane = kTP / kVGroups;       // positions per lane per tile
-    static constexpr int kTileHalves = kTP * kStride;
-    // wave-private region: K tile, V tile, p[kTP][GP], alpha[GP]; 16-byte multiple
-    static constexpr size_t kWaveLds =
-        (((size_t)kTileHalves * 2 * 2 + (size_t)GP * kTP * 4 + (size_t)GP * 4) + 15) & ~(size_t)15;
-    // workgroup merge: (max, sum)[kWaves][GP], then acc[kWaves * kVGroups][GP][HD]
-    static constexpr size_t kMlFloats = ((size_t)kWaves * GP * 2 + 3) & ~(size_t)3;
-    static constexpr size_t kMergeLds = (kMlFloats + (size_t)kWaves * kVGroups * GP * HD) * sizeof(float);
-    static_assert(kLoads >= 1 && kVPerLane >= 1 && kTP % kVGroups == 0, "tile");
-};
-
-template <int HD, int GP>
-size_t split_lds_bytes() {
-    using C = Cfg<HD, GP>;
-    const size_t tiles = C::kWaveLds * kWaves;
-    return tiles > C::kMergeLds ? tiles : C::kMergeLds;
-}
-
 // Positions a sequence covers and its chunk count.  A position at or beyond
 // the caller's bound `max_len` is cut there, so neither the cache reads nor
 // the chunk index leave their buffers.
@@ -83,242 +49,30 @@ __device__ __forceinline__ SeqSpan seq_span(const int32_t* positions, int positi
     return {L, L > 0 ? (L + chunk - 1) / chunk : 0};
 }
 
-// Grid: (chunk, kv_head, seq).  `positions` (device, per sequence) or the
-// scalar `position` gives the last cached position of each sequence.
-template <int HD, int GP, int kDepth>
-__global__ __launch_bounds__(kBlock) void attn_split_kernel(
-    const uint16_t* __restrict__ q, const uint16_t* __restrict__ k_cache, const uint16_t* __restrict__ v_cache,
-    long long seq_stride, const int32_t* __restrict__ positions, int position, int max_len, int heads,
-    int kv_heads, int group, int chunk, float scale_log2, float* __restrict__ part, int n_splits,
-    uint16_t* __restrict__ out) {
-    using C = Cfg<HD, GP>;
-    extern __shared__ __align__(16) uint8_t smem[];
-
-    const int split = blockIdx.x, kvh = blockIdx.y, seq = blockIdx.z;
-    const SeqSpan span = seq_span(positions, position, seq, chunk, max_len);
-    const int L = span.len, n_valid = span.n_valid;
-    const int b0 = split * chunk;
-    if (b0 >= L) return;
-    const int b1 = min(L, b0 + chunk);
-
-    const int lane = threadIdx.x & (kWave - 1);
-    const int wave = threadIdx.x / kWave;
-    // the chunk's positions split over the four waves in whole tiles (a
-    // short sequence's only chunk still occupies every wave)
-    const int sub = (((b1 - b0 + kWaves - 1) / kWaves + C::kTP - 1) / C::kTP) * C::kTP;
-    const int w0 = min(b1, b0 + wave * sub);
-    const int w1 = min(b1, w0 + sub);
-
-    uint8_t* wl = smem + (size_t)wave * C::kWaveLds;
-    uint16_t* kt = reinterpret_cast<uint16_t*>(wl);
-    uint16_t* vt = kt + C::kTileHalves;
-    float* pt = reinterpret_cast<float*>(vt + C::kTileHalves);   // [kTP][GP]
-    float* at = pt + GP * C::kTP;                                 // [GP]
-
-    const uint16_t* kbase = k_cache + (size_t)seq * seq_stride + (size_t)kvh * HD;
-    const uint16_t* vbase = v_cache + (size_t)seq * seq_stride + (size_t)kvh * HD;
-    const size_t row_step = (size_t)kv_heads * HD;
-
-    // scores-phase identity
-    const int sh = lane % GP, sp = lane / GP;
-    const bool s_head_ok = sh < group;
-    const bool s_lane_ok = sp < C::kTP;
-    // q of the lane's head in VGPRs.  Unconditional loads (a padding head
-    // reads the group's last head and is zeroed) keep every global load
-    // outside branches, so the compiler's load counting stays exact and the
-    // waits below never cover the tiles still in flight.
-    uint32_t qv[HD / 2];
-    {
-        const int hq = kvh * group + (s_head_ok ? sh : group - 1);
-        const uint16_t* qh = q + ((size_t)seq * heads + hq) * HD;
-        const uint32_t keep = s_head_ok ? 0xffffffffu : 0u;
-#pragma unroll
-        for (int c = 0; c < C::kChunks; ++c) {
-            const u32x4 v = *reinterpret_cast<const u32x4*>(qh + c * 8);
-            qv[4 * c + 0] = v.x & keep; qv[4 * c + 1] = v.y & keep;
-            qv[4 * c + 2] = v.z & keep; qv[4 * c + 3] = v.w & keep;
-        }
-    }
-    // value-phase identity: lane = (position group vg, 8-dim slice vc)
-    const int vc = lane % C::kChunks, vg = lane / C::kChunks;
-    float acc[GP][8];
-#pragma unroll
-    for (int h = 0; h < GP; ++h)
-#pragma unroll
-        for (int k = 0; k < 8; ++k) acc[h][k] = 0.f;
-
-    float m_run = -INFINITY, l_run = 0.f;   // per scores lane (head sh)
-
-    // load identity; kDepth tiles of K and V rows in flight per wave
-    const int lrow = lane / C::kChunks, lc = lane % C::kChunks;
-    u32x4 kr[kDepth][C::kLoads], vr[kDepth][C::kLoads];
-    auto load_tile = [&](u32x4 (&kd)[C::kLoads], u32x4 (&vd)[C::kLoads], int t0) {
-#pragma unroll
-        for (int i = 0; i < C::kLoads; ++i) {
-            // branch-free: rows past the range re-read the last one (never used)
-            const int pos = min(t0 + i * C::kRowsPerLoad + lrow, w1 - 1);
-            kd[i] = *reinterpret_cast<const u32x4*>(kbase + (size_t)pos * row_step + lc * 8);
-            vd[i] = *reinterpret_cast<const u32x4*>(vbase + (size_t)pos * row_step + lc * 8);
-        }
-    };
-
-    // One staged tile; with nv <= 0 it changes nothing (scores -inf, weights 0).
-    auto process_tile = [&](int t0) {
-        const int nv = min(C::kTP, w1 - t0);
-
-        // ---- scores + online softmax (lane = position sp, head sh) ----
-        float s2 = -INFINITY;
-        if (s_lane_ok && s_head_ok && sp < nv) {
-            const uint16_t* kr_row = kt + sp * C::kStride;
-            float a0 = 0.f, a1 = 0.f;
-#pragma unroll
-            for (int c = 0; c < C::kChunks; ++c) {
-                const u32x4 kk = *reinterpret_cast<const u32x4*>(kr_row + c * 8);
-                a0 = dot2(qv[4 * c + 0], kk.x, a0);
-                a1 = dot2(qv[4 * c + 1], kk.y, a1);
-                a0 = dot2(qv[4 * c + 2], kk.z, a0);
-                a1 = dot2(qv[4 * c + 3], kk.w, a1);
-            }
-            s2 = (a0 + a1) * scale_log2;
-        }
-        const float mt = column_max<GP>(s2);
-        const float m_new = fmaxf(m_run, mt);
-        const bool live = m_new != -INFINITY;
-        const float alpha = live ? __builtin_amdgcn_exp2f(m_run - m_new) : 1.f;
-        const float pw = live ? __builtin_amdgcn_exp2f(s2 - m_new) : 0.f;
-        const float ps = column_sum<GP>(pw);
-        l_run = l_run * alpha + ps;
-        m_run = m_new;
-        if (s_lane_ok) pt[lane] = pw;   // lane = sp * GP + sh
-        if (sp == 0) at[sh] = alpha;
-        wave_lds_sync();
-
-        // ---- values: every head for kVPerLane positions of this lane ----
-        float al[GP];
-        load_floats<GP>(at, al);
-#pragma unroll
-        for (int h = 0; h < GP; ++h)
-#pragma unroll
-            for (int k = 0; k < 8; ++k) acc[h][k] *= al[h];
-        // rows past nv hold finite copies of a valid row and weight 0
-#pragma unroll
-        for (int j = 0; j < C::kVPerLane; ++j) {
-            const int p = vg + j * C::kVGroups;
-            const u32x4 vv = *reinterpret_cast<const u32x4*>(vt + p * C::kStride + vc * 8);
-            float pp[GP];
-            load_floats<GP>(pt + p * GP, pp);
-            const float v8[8] = {h2f(vv.x & 0xffffu), h2f(vv.x >> 16), h2f(vv.y & 0xffffu), h2f(vv.y >> 16),
-                                 h2f(vv.z & 0xffffu), h2f(vv.z >> 16), h2f(vv.w & 0xffffu), h2f(vv.w >> 16)};
-#pragma unroll
-            for (int h = 0; h < GP; ++h)
-#pragma unroll
-                for (int k = 0; k < 8; ++k) acc[h][k] = fmaf(pp[h], v8[k], acc[h][k]);
-        }
-        wave_lds_sync();
-    };
-
-    // kDepth tiles in flight: tile t is consumed while tiles t+1 .. t+kDepth-1
-    // load, and its slot is refilled with tile t+kDepth right away.  Loads
-    // are unconditional (past the range they re-read row w1 - 1, in bounds
-    // even for an empty range since w1 = b1 >= 1 there) and a tile past the
-    // range is a no-op, so no load sits in a branch.
-    // The issue order is pinned (sched_barrier): the slots must be issued in
-    // the same order as the loop refills them, or the wait before a slot's
-    // first use covers the later slots too.
-    __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-    for (int d = 0; d < kDepth; ++d) {
-        load_tile(kr[d], vr[d], w0 + d * C::kTP);
-        __builtin_amdgcn_sched_barrier(0);
-    }
-    for (int t0 = w0; t0 < w1; t0 += kDepth * C::kTP) {
-#pragma unroll
-        for (int d = 0; d < kDepth; ++d) {
-            const int tt = t0 + d * C::kTP;
-            // every row is stored: rows past the range hold a copy of row
-            // w1 - 1 (finite) and get weight 0
-#pragma unroll
-            for (int i = 0; i < C::kLoads; ++i) {
-                const int r = i * C::kRowsPerLoad + lrow;
-                *reinterpret_cast<u32x4*>(kt + r * C::kStride + lc * 8) = kr[d][i];
-                *reinterpret_cast<u32x4*>(vt + r * C::kStride + lc * 8) = vr[d][i];
-            }
-            wave_lds_sync();
-            __builtin_amdgcn_sched_barrier(0);
-            load_tile(kr[d], vr[d], tt + kDepth * C::kTP);
-            __builtin_amdgcn_sched_barrier(0);
-            process_tile(tt);
-        }
-    }
-
-    // ---- merge the position groups and the four waves in LDS ----
-    __syncthreads();   // every wave is done with its tiles
-    float* ml = reinterpret_cast<float*>(smem);   // [kWaves][GP] (max, sum)
-    float* ms = ml + C::kMlFloats;                // [kWaves * kVGroups][GP][HD]
-    if (sp == 0) {
-        ml[(wave * GP + sh) * 2] = m_run;
-        ml[(wave * GP + sh) * 2 + 1] = l_run;
-    }
-#pragma unroll
-    for (int h = 0; h < GP; ++h) {
-        f32x4* e = reinterpret_cast<f32x4*>(ms + ((size_t)(wave * C::kVGroups + vg) * GP + h) * HD + vc * 8);
-        e[0] = f32x4{acc[h][0], acc[h][1], acc[h][2], acc[h][3]};
-        e[1] = f32x4{acc[h][4], acc[h][5], acc[h][6], acc[h][7]};
-    }
-    __syncthreads();
-
-    for (int idx = threadIdx.x; idx < group * HD; idx += kBlock) {
-        const int h = idx / HD, d = idx - h * HD;
-        float M = -INFINITY;
-#pragma unroll
-        for (int w = 0; w < kWaves; ++w) M = fmaxf(M, ml[(w * GP + h) * 2]);
-        float Ls = 0.f, A = 0.f;
-#pragma unroll
-        for (int w = 0; w < kWaves; ++w) {
-            const float mw = ml[(w * GP + h) * 2];
-            const float f = mw == -INFINITY ? 0.f : exp2f(mw - M);
-            Ls += ml[(w * GP + h) * 2 + 1] * f;
-            float a = 0.f;
-#pragma unroll
-            for (int g = 0; g < C::kVGroups; ++g) a += ms[((size_t)(w * C::kVGroups + g) * GP + h) * HD + d];
-            A += a * f;
-        }
-        const int hq = kvh * group + h;
-        if (n_valid == 1) {
-            out[((size_t)seq * heads + hq) * HD + d] = f2h_rne(A / Ls);
-        } else {
-            float* pe = part + (((size_t)seq * heads + hq) * n_splits + split) * (HD + 4);
-            pe[d] = A;
-            if (d == 0) {
-                pe[HD] = M;
-                pe[HD + 1] = Ls;
-            }
-        }
-    }
-}
-
 // ---------------------------------------------------------------------------
-// head_dim 128, GQA group 2..8: the same chunk / merge structure with both
-// products on the matrix cores (v_mfma_f32_16x16x16f16).  The group's heads
-// are the 16 MFMA columns (padding heads have q = 0 and are never written).
-// Per wave, a tile of 16 positions, one tile's loads in flight:
+// Chunk kernel, both products on the matrix cores (v_mfma_f32_16x16x16f16).
+// The group's heads are the 16 MFMA columns (padding heads have q = 0 and are
+// never written).  Per wave, a tile of 16 (head_dim 128) or 32 (64) positions,
+// 4 KB of K and of V, one tile's loads in flight:
 //  * loads, two forms (kRows, chosen by the plan):
-//    - direct: lane = (row col, 64-byte slab grp), 16 rows x 64 bytes per
-//      instruction, K straight into the A operand, V into an LDS tile; the
-//      refill is issued once the scores are in;
+//    - direct: lane = (row col, 16-byte slices grp, grp + 4, ...), 16 rows x
+//      64 bytes per instruction, K straight into the A operand, V into an LDS
+//      tile; the refill is issued once the scores are in;
 //    - rows (launches of more than two workgroups per CU, where HBM
-//      saturates): each nontemporal instruction reads four whole 256-byte
-//      rows (lane = row 4u + grp, 16-byte slice col), which a probe of the
-//      same shape reads at ~7 TB/s against ~5.9 for 16 rows x 64 bytes;
-//      K and V go to wave-private LDS rows, the refill is issued at once
-//      and K is read back in the A operand layout.
+//      saturates): each nontemporal instruction reads whole rows, four of 256
+//      or eight of 128 bytes, which a probe of the 256-byte shape reads at
+//      ~7 TB/s against ~5.9 for 16 rows x 64 bytes; K and V go to
+//      wave-private LDS rows, the refill is issued at once and K is read back
+//      in the A operand layout.
 //  * scores S[pos][head] = K[pos][:] . q[head][:]: the A operand is K row
-//    `col` (lane = row `col`, a 64-byte slab `grp` of it; the 128
-//    dims in 8 steps of 16, dim 32t + 8grp + 4h + j of step (t, h) being
-//    operand k = 4grp + j), q is the B operand in the same dim order; lane
-//    (col, grp) gets the scores of positions 4grp + i for head col.
+//    `col` of 16 positions (lane = row `col`, dims 32t + 8grp + 4h + j of step
+//    (t, h) being operand k = 4grp + j), q is the B operand in the same dim
+//    order; lane (col, grp) gets the scores of positions 4grp + i for head
+//    col.
 //  * online softmax per head column (max and sum over the column's four lane
-//    groups by permlane swaps), exponentials in base 2 as the VALU kernel.
+//    groups by permlane swaps), exponentials in base 2.  At head_dim 64 one
+//    softmax step covers 32 positions, so its cost per byte of cache is that
+//    of head_dim 128.
 //  * out^T[dim][head] += V^T[dim][pos] P^T[pos][head]: the scores' lane
 //    layout is the B operand P^T as it stands, so every accumulator of a
 //    lane belongs to the lane's head column and the online-softmax rescale
@@ -329,16 +83,26 @@ __global__ __launch_bounds__(kBlock) void attn_split_kernel(
 //    output block 4c + e, rows 4grp + i of which are dims 64c + 16grp + 4i + e).
 // ---------------------------------------------------------------------------
 typedef _Float16 half4 __attribute__((ext_vector_type(4)));
-constexpr int kMTile = 16;                     // positions per MFMA tile
-constexpr int kMStride = 128 + 8;              // K / V tile row in LDS (halves)
-constexpr size_t kMWaveLds = (size_t)kMTile * kMStride * 2;
-// merge: (max, sum)[NW][8], acc[NW][8 blocks][8 heads][4 lane groups][4]
-// tiles: per wave a V tile, and with row loads a K tile, kMWaveLds each
-template <int NW, bool kRows>
+template <int HD>
+struct AttnTile {
+    static_assert(HD == 64 || HD == 128, "head_dim");
+    static constexpr int kSubs = 128 / HD;         // MFMA row blocks of 16 positions
+    static constexpr int kPos = 16 * kSubs;        // positions per tile
+    static constexpr int kStride = HD + 8;         // K / V tile row in LDS (halves)
+    static constexpr size_t kBytes = (size_t)kPos * kStride * 2;
+    static constexpr int kSlices = HD / 8;         // 16-byte slices per row
+    static constexpr int kRowsPerLoad = kWave / kSlices;
+    static constexpr int kSteps = HD / 32;         // score steps (two MFMAs each) per 16 positions
+    static constexpr int kOut = HD / 16;           // output blocks
+};
+// merge: (max, sum)[NW][8], acc[NW][kOut blocks][8 heads][4 lane groups][4]
+// tiles: per wave a V tile, and with row loads a K tile
+template <int HD, int NW, bool kRows>
 struct MfmaLds {
+    using T = AttnTile<HD>;
     static constexpr size_t kMlFloats = (size_t)NW * 8 * 2;
-    static constexpr size_t kMerge = (kMlFloats + (size_t)NW * 2 * 8 * 16 * 4) * sizeof(float);
-    static constexpr size_t kTiles = (kRows ? 2 : 1) * kMWaveLds * NW;
+    static constexpr size_t kMerge = (kMlFloats + (size_t)NW * T::kOut * 8 * 16) * sizeof(float);
+    static constexpr size_t kTiles = (kRows ? 2 : 1) * T::kBytes * NW;
     static constexpr size_t kBytes = kMerge > kTiles ? kMerge : kTiles;
     // with the q/k prologue: q' of up to 8 heads, then per wave k' and v of the step
     static constexpr size_t kQs = kBytes;
@@ -366,14 +130,16 @@ __device__ __forceinline__ half4 as_half4(uint32_t lo, uint32_t hi) {
 // serves launches of many workgroups per CU and is asked for four waves (it
 // fits in 124-128 VGPRs, no spill); the direct form runs at most two
 // workgroups per CU and keeps the allocation it schedules best with.
-template <int GP, bool kRows, int NW, bool kPrep>
+template <int HD, int GP, bool kRows, int NW, bool kPrep>
 __global__ __launch_bounds__(NW * kWave, kRows ? 4 : 1) void attn_mfma_kernel(
     const uint16_t* __restrict__ q, const uint16_t* __restrict__ k_cache, const uint16_t* __restrict__ v_cache,
     long long seq_stride, const int32_t* __restrict__ positions, int position, int max_len, int heads,
     int kv_heads, int group, int chunk, float scale_log2, float* __restrict__ part, int n_splits,
     uint16_t* __restrict__ out, QkPrep prep) {
-    constexpr int HD = 128;
-    static_assert(GP >= 2 && GP <= 8, "group");
+    using T = AttnTile<HD>;
+    constexpr int kTile = T::kPos, kStride = T::kStride;
+    static_assert(GP >= 1 && GP <= 8, "group");
+    static_assert(!kPrep || (HD == 128 && GP >= 2), "the q/k prologue is built for head_dim 128 with GQA");
     extern __shared__ __align__(16) uint8_t smem[];
 
     const int split = blockIdx.x, kvh = blockIdx.y, seq = blockIdx.z;
@@ -386,7 +152,7 @@ __global__ __launch_bounds__(NW * kWave, kRows ? 4 : 1) void attn_mfma_kernel(
     const int lane = threadIdx.x & (kWave - 1);
     const int wave = threadIdx.x / kWave;
     const int col = lane & 15, grp = lane >> 4;
-    const int sub = (((b1 - b0 + NW - 1) / NW + kMTile - 1) / kMTile) * kMTile;
+    const int sub = (((b1 - b0 + NW - 1) / NW + kTile - 1) / kTile) * kTile;
     const int w0 = min(b1, b0 + wave * sub);
     const int w1 = min(b1, w0 + sub);
 
@@ -396,12 +162,12 @@ __global__ __launch_bounds__(NW * kWave, kRows ? 4 : 1) void attn_mfma_kernel(
     const int pos_row = L - 1;
     const bool has_pos = kPrep && p_raw >= 0 && p_raw < max_len && w0 <= pos_row && pos_row < w1;
 
-    using Lds = MfmaLds<NW, kRows>;
-    uint16_t* vt = reinterpret_cast<uint16_t*>(smem + (size_t)wave * (kRows ? 2 : 1) * kMWaveLds);
-    uint16_t* kt = vt + kMTile * kMStride;   // row loads only
-    // direct: lane = (row col, 64-byte slab grp); rows: lane = (row 4u + grp,
-    // 16-byte slice col of the kv head's 256-byte row)
-    const int lane_off = kRows ? 8 * col : 8 * grp;
+    using Lds = MfmaLds<HD, NW, kRows>;
+    uint16_t* vt = reinterpret_cast<uint16_t*>(smem + (size_t)wave * (kRows ? 2 : 1) * T::kBytes);
+    uint16_t* kt = vt + kTile * kStride;   // row loads only
+    // row loads: lane = (row lrow of an instruction's rows, 16-byte slice lsl)
+    const int lsl = lane % T::kSlices, lrow = lane / T::kSlices;
+    const int lane_off = kRows ? 8 * lsl : 8 * grp;
     const uint16_t* kbase = k_cache + (size_t)seq * seq_stride + (size_t)kvh * HD + lane_off;
     const uint16_t* vbase = v_cache + (size_t)seq * seq_stride + (size_t)kvh * HD + lane_off;
     const size_t row_step = (size_t)kv_heads * HD;
@@ -410,7 +176,7 @@ __global__ __launch_bounds__(NW * kWave, kRows ? 4 : 1) void attn_mfma_kernel(
     // + j; loaded here, turned into operands after the first tiles' loads are
     // issued, so that q's round trip overlaps theirs
     const bool q_ok = col < group;
-    u32x4 q_raw[4];
+    u32x4 q_raw[T::kSteps];
     // kPrep: raw q of the heads this wave forms (dims lane, lane + 64), the
     // step's k and v of this kv head, the norm weights; all loads
     // unconditional (a missing weight reads q and is not used)
@@ -438,30 +204,31 @@ __global__ __launch_bounds__(NW * kWave, kRows ? 4 : 1) void attn_mfma_kernel(
     } else {
         const uint16_t* qh = q + ((size_t)seq * heads + kvh * group + (q_ok ? col : group - 1)) * HD + 8 * grp;
 #pragma unroll
-        for (int t = 0; t < 4; ++t) q_raw[t] = *reinterpret_cast<const u32x4*>(qh + 32 * t);
+        for (int t = 0; t < T::kSteps; ++t) q_raw[t] = *reinterpret_cast<const u32x4*>(qh + 32 * t);
     }
-    half4 qb[4][2];
-    f32x4 o[8];   // o[4c + e][i]: dim 64c + 16grp + 4i + e of head col
+    half4 qb[T::kSteps][2];
+    f32x4 o[T::kOut];   // o[4c + e][i]: dim 64c + 16grp + 4i + e of head col
 #pragma unroll
-    for (int b = 0; b < 8; ++b) o[b] = f32x4{0.f, 0.f, 0.f, 0.f};
+    for (int b = 0; b < T::kOut; ++b) o[b] = f32x4{0.f, 0.f, 0.f, 0.f};
     float m_run = -INFINITY, l_run = 0.f;   // head col
 
     // One tile of K and V rows in flight; branch-free (rows past the range
     // re-read row w1 - 1, in bounds also for an empty range).  Slot u of a
-    // lane: direct, row t0 + col, dims 32u + 8grp .. + 7; rows, row
-    // t0 + 4u + grp, dims 8col .. + 7.
+    // lane: direct, row t0 + 16 (u / kSteps) + col, dims 32 (u % kSteps) +
+    // 8grp .. + 7; rows, row t0 + kRowsPerLoad u + lrow, dims 8lsl .. + 7.
+    auto slot_row = [&](int u) { return kRows ? T::kRowsPerLoad * u + lrow : 16 * (u / T::kSteps) + col; };
+    auto slot_dim = [&](int u) { return kRows ? 0 : 32 * (u % T::kSteps); };   // beyond lane_off
     u32x4 kr[4], vr[4];
     auto load_tile = [&](int t0) {
 #pragma unroll
         for (int u = 0; u < 4; ++u) {
+            const size_t at = (size_t)min(t0 + slot_row(u), w1 - 1) * row_step + slot_dim(u);
             if constexpr (kRows) {
-                const size_t pos = (size_t)min(t0 + 4 * u + grp, w1 - 1);
-                kr[u] = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(kbase + pos * row_step));
-                vr[u] = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(vbase + pos * row_step));
+                kr[u] = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(kbase + at));
+                vr[u] = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(vbase + at));
             } else {
-                const size_t pos = (size_t)min(t0 + col, w1 - 1);
-                kr[u] = *reinterpret_cast<const u32x4*>(kbase + pos * row_step + 32 * u);
-                vr[u] = *reinterpret_cast<const u32x4*>(vbase + pos * row_step + 32 * u);
+                kr[u] = *reinterpret_cast<const u32x4*>(kbase + at);
+                vr[u] = *reinterpret_cast<const u32x4*>(vbase + at);
             }
         }
     };
@@ -472,61 +239,72 @@ __global__ __launch_bounds__(NW * kWave, kRows ? 4 : 1) void attn_mfma_kernel(
             // the step's row comes from the prologue's k' and v in LDS
 #pragma unroll
             for (int u = 0; u < 4; ++u) {
-                const int row = kRows ? t0 + 4 * u + grp : t0 + col;
-                if (has_pos && min(row, w1 - 1) == pos_row) {
-                    const int dim = kRows ? 8 * col : 32 * u + 8 * grp;
+                if (has_pos && min(t0 + slot_row(u), w1 - 1) == pos_row) {
+                    const int dim = lane_off + slot_dim(u);
                     kr[u] = *reinterpret_cast<const u32x4*>(kv_new + dim);
                     vr[u] = *reinterpret_cast<const u32x4*>(kv_new + HD + dim);
                 }
             }
         }
-        f32x4 s = f32x4{0.f, 0.f, 0.f, 0.f};
+        f32x4 s[T::kSubs];
+#pragma unroll
+        for (int b = 0; b < T::kSubs; ++b) s[b] = f32x4{0.f, 0.f, 0.f, 0.f};
         if constexpr (kRows) {
             // both tiles into LDS rows; the slot is then free: refill it with
             // the next tile, in flight over this tile's whole computation
 #pragma unroll
             for (int u = 0; u < 4; ++u) {
-                *reinterpret_cast<u32x4*>(vt + (4 * u + grp) * kMStride + 8 * col) = vr[u];
-                *reinterpret_cast<u32x4*>(kt + (4 * u + grp) * kMStride + 8 * col) = kr[u];
+                *reinterpret_cast<u32x4*>(vt + slot_row(u) * kStride + lane_off) = vr[u];
+                *reinterpret_cast<u32x4*>(kt + slot_row(u) * kStride + lane_off) = kr[u];
             }
             __builtin_amdgcn_sched_barrier(0);
-            load_tile(t0 + kMTile);
+            load_tile(t0 + kTile);
             __builtin_amdgcn_sched_barrier(0);
             wave_lds_sync();   // the K and V rows stored above
-            // K row col, dims 32t + 8grp .. + 7: the A operand layout
+            // K row 16b + col, dims 32t + 8grp .. + 7: the A operand layout
             u32x4 kk[4];
 #pragma unroll
-            for (int t = 0; t < 4; ++t) kk[t] = *reinterpret_cast<const u32x4*>(kt + col * kMStride + 32 * t + 8 * grp);
+            for (int u = 0; u < 4; ++u)
+                kk[u] = *reinterpret_cast<const u32x4*>(kt + (16 * (u / T::kSteps) + col) * kStride +
+                                                        32 * (u % T::kSteps) + 8 * grp);
 #pragma unroll
-            for (int t = 0; t < 4; ++t) {
-                s = mfma16(as_half4(kk[t].x, kk[t].y), qb[t][0], s);
-                s = mfma16(as_half4(kk[t].z, kk[t].w), qb[t][1], s);
+            for (int u = 0; u < 4; ++u) {
+                f32x4& sb = s[u / T::kSteps];
+                sb = mfma16(as_half4(kk[u].x, kk[u].y), qb[u % T::kSteps][0], sb);
+                sb = mfma16(as_half4(kk[u].z, kk[u].w), qb[u % T::kSteps][1], sb);
             }
         } else {
 #pragma unroll
-            for (int t = 0; t < 4; ++t) *reinterpret_cast<u32x4*>(vt + col * kMStride + 32 * t + 8 * grp) = vr[t];
+            for (int u = 0; u < 4; ++u)
+                *reinterpret_cast<u32x4*>(vt + slot_row(u) * kStride + lane_off + slot_dim(u)) = vr[u];
 #pragma unroll
-            for (int t = 0; t < 4; ++t) {
-                s = mfma16(as_half4(kr[t].x, kr[t].y), qb[t][0], s);
-                s = mfma16(as_half4(kr[t].z, kr[t].w), qb[t][1], s);
+            for (int u = 0; u < 4; ++u) {
+                f32x4& sb = s[u / T::kSteps];
+                sb = mfma16(as_half4(kr[u].x, kr[u].y), qb[u % T::kSteps][0], sb);
+                sb = mfma16(as_half4(kr[u].z, kr[u].w), qb[u % T::kSteps][1], sb);
             }
             // the slot is consumed: refill it with the next tile (the address
             // waits for the scores, so the load is issued after them)
-            load_tile(issue_after(t0 + kMTile, s[0], s[3]));
+            load_tile(issue_after(t0 + kTile, s[0][0], s[T::kSubs - 1][3]));
             __builtin_amdgcn_sched_barrier(0);
         }
 
-        float sv[4];
+        float sv[4 * T::kSubs];   // position t0 + 16 (i / 4) + 4grp + i % 4
+        float mt = -INFINITY;
 #pragma unroll
-        for (int i = 0; i < 4; ++i) sv[i] = t0 + 4 * grp + i < w1 ? s[i] * scale_log2 : -INFINITY;
-        const float mt = column_max<16>(fmaxf(fmaxf(sv[0], sv[1]), fmaxf(sv[2], sv[3])));
+        for (int i = 0; i < 4 * T::kSubs; ++i)
+            sv[i] = t0 + 16 * (i / 4) + 4 * grp + i % 4 < w1 ? s[i / 4][i % 4] * scale_log2 : -INFINITY;
+#pragma unroll
+        for (int b = 0; b < T::kSubs; ++b)
+            mt = fmaxf(mt, fmaxf(fmaxf(sv[4 * b], sv[4 * b + 1]), fmaxf(sv[4 * b + 2], sv[4 * b + 3])));
+        mt = column_max<16>(mt);
         const float m_new = fmaxf(m_run, mt);
         const bool live = m_new != -INFINITY;
         const float alpha = live ? __builtin_amdgcn_exp2f(m_run - m_new) : 1.f;
-        float pv[4];
+        float pv[4 * T::kSubs];
         float ps = 0.f;
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
+        for (int i = 0; i < 4 * T::kSubs; ++i) {
             pv[i] = live ? __builtin_amdgcn_exp2f(sv[i] - m_new) : 0.f;
             ps += pv[i];
         }
@@ -541,38 +319,42 @@ __global__ __launch_bounds__(NW * kWave, kRows ? 4 : 1) void attn_mfma_kernel(
         if constexpr (kPrep) {
             if (t0 != w0 && __builtin_amdgcn_ballot_w64(alpha != 1.f) != 0) {
 #pragma unroll
-                for (int b = 0; b < 8; ++b) o[b] *= alpha;
+                for (int b = 0; b < T::kOut; ++b) o[b] *= alpha;
             }
         } else if constexpr (!decltype(first_tile)::value) {
 #pragma unroll
-            for (int b = 0; b < 8; ++b) o[b] *= alpha;
+            for (int b = 0; b < T::kOut; ++b) o[b] *= alpha;
         }
-        half4 ph, pl;
+        half4 ph[T::kSubs], pl[T::kSubs];
 #pragma unroll
-        for (int j = 0; j < 4; ++j) {
+        for (int j = 0; j < 4 * T::kSubs; ++j) {
             const _Float16 h = (_Float16)pv[j];
-            ph[j] = h;
-            pl[j] = (_Float16)(pv[j] - (float)h);
+            ph[j / 4][j % 4] = h;
+            pl[j / 4][j % 4] = (_Float16)(pv[j] - (float)h);
         }
         if constexpr (!kRows) wave_lds_sync();   // the V rows stored above
 #pragma unroll
-        for (int c = 0; c < 2; ++c) {
-            uint32_t w[4][2];   // rows 4grp + j, dims 64c + 4col .. + 3
+        for (int b = 0; b < T::kSubs; ++b) {
 #pragma unroll
-            for (int j = 0; j < 4; ++j) {
-                const u32x2 x = *reinterpret_cast<const u32x2*>(vt + (4 * grp + j) * kMStride + 64 * c + 4 * col);
-                w[j][0] = x.x;
-                w[j][1] = x.y;
-            }
+            for (int c = 0; c < HD / 64; ++c) {
+                uint32_t w[4][2];   // rows 16b + 4grp + j, dims 64c + 4col .. + 3
 #pragma unroll
-            for (int e = 0; e < 4; ++e) {
-                const uint32_t sel = (e & 1) ? 0x07060302u : 0x05040100u;
-                const half4 vb = as_half4(__builtin_amdgcn_perm(w[1][e >> 1], w[0][e >> 1], sel),
-                                          __builtin_amdgcn_perm(w[3][e >> 1], w[2][e >> 1], sel));
-                // V^T P^T: dims x heads, so a lane's accumulators belong to
-                // one head (its column) and the rescale needs no lane moves
-                o[4 * c + e] = mfma16(vb, ph, o[4 * c + e]);
-                o[4 * c + e] = mfma16(vb, pl, o[4 * c + e]);
+                for (int j = 0; j < 4; ++j) {
+                    const u32x2 x =
+                        *reinterpret_cast<const u32x2*>(vt + (16 * b + 4 * grp + j) * kStride + 64 * c + 4 * col);
+                    w[j][0] = x.x;
+                    w[j][1] = x.y;
+                }
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    const uint32_t sel = (e & 1) ? 0x07060302u : 0x05040100u;
+                    const half4 vb = as_half4(__builtin_amdgcn_perm(w[1][e >> 1], w[0][e >> 1], sel),
+                                              __builtin_amdgcn_perm(w[3][e >> 1], w[2][e >> 1], sel));
+                    // V^T P^T: dims x heads, so a lane's accumulators belong to
+                    // one head (its column) and the rescale needs no lane moves
+                    o[4 * c + e] = mfma16(vb, ph[b], o[4 * c + e]);
+                    o[4 * c + e] = mfma16(vb, pl[b], o[4 * c + e]);
+                }
             }
         }
         wave_lds_sync();   // before the next tile overwrites the rows
@@ -630,7 +412,7 @@ __global__ __launch_bounds__(NW * kWave, kRows ? 4 : 1) void attn_mfma_kernel(
         const uint16_t* qh = qs + (q_ok ? col : 0) * HD + 8 * grp;
         const uint32_t keep = q_ok ? 0xffffffffu : 0u;
 #pragma unroll
-        for (int t = 0; t < 4; ++t) {
+        for (int t = 0; t < T::kSteps; ++t) {
             const u32x4 v = *reinterpret_cast<const u32x4*>(qh + 32 * t);
             qb[t][0] = as_half4(v.x & keep, v.y & keep);
             qb[t][1] = as_half4(v.z & keep, v.w & keep);
@@ -638,38 +420,38 @@ __global__ __launch_bounds__(NW * kWave, kRows ? 4 : 1) void attn_mfma_kernel(
     } else {
         const uint32_t keep = q_ok ? 0xffffffffu : 0u;
 #pragma unroll
-        for (int t = 0; t < 4; ++t) {
+        for (int t = 0; t < T::kSteps; ++t) {
             qb[t][0] = as_half4(q_raw[t].x & keep, q_raw[t].y & keep);
             qb[t][1] = as_half4(q_raw[t].z & keep, q_raw[t].w & keep);
         }
     }
     if constexpr (kPrep) {
-        for (int t0 = w0; t0 < w1; t0 += kMTile) process(t0, std::false_type{});
+        for (int t0 = w0; t0 < w1; t0 += kTile) process(t0, std::false_type{});
     } else {
         if (w0 < w1) process(w0, std::true_type{});
-        for (int t0 = w0 + kMTile; t0 < w1; t0 += kMTile) process(t0, std::false_type{});
+        for (int t0 = w0 + kTile; t0 < w1; t0 += kTile) process(t0, std::false_type{});
     }
 
     // ---- merge the waves in LDS ----
     __syncthreads();   // every wave is done with its V tile
     float* ml = reinterpret_cast<float*>(smem);   // [NW][8] (max, sum)
-    float* ms = ml + Lds::kMlFloats;              // [NW][8 b][8 heads][4 grp][4 i]
+    float* ms = ml + Lds::kMlFloats;              // [NW][kOut b][8 heads][4 grp][4 i]
     if (grp == 0 && col < GP) {
         ml[(wave * 8 + col) * 2] = m_run;
         ml[(wave * 8 + col) * 2 + 1] = l_run;
     }
     if (col < GP) {
 #pragma unroll
-        for (int b = 0; b < 8; ++b)
-            *reinterpret_cast<f32x4*>(ms + ((((size_t)wave * 8 + b) * 8 + col) * 4 + grp) * 4) = o[b];
+        for (int b = 0; b < T::kOut; ++b)
+            *reinterpret_cast<f32x4*>(ms + ((((size_t)wave * T::kOut + b) * 8 + col) * 4 + grp) * 4) = o[b];
     }
     __syncthreads();
 
-    // Thread t merges dims kPer*t .. + kPer - 1 of one head (kPer divides HD):
-    // the head's max, wave factors and sum are formed once, and every LDS
-    // read is issued before the arithmetic.
-    constexpr int kPer = GP * HD / (NW * kWave);
-    static_assert(kPer >= 1 && HD % kPer == 0 && kPer * NW * kWave == GP * HD, "merge split");
+    // Thread t merges dims kPer*t .. + kPer - 1 of one head (kPer divides HD;
+    // with fewer dims than threads, one each): the head's max, wave factors and
+    // sum are formed once, and every LDS read is issued before the arithmetic.
+    constexpr int kPer = GP * HD <= NW * kWave ? 1 : GP * HD / (NW * kWave);
+    static_assert(HD % kPer == 0 && kPer * NW * kWave >= GP * HD, "merge split");
     const int base = (int)threadIdx.x * kPer;
     if (base >= group * HD) return;
     const int h = base / HD, dim0 = base - h * HD;
@@ -683,7 +465,7 @@ __global__ __launch_bounds__(NW * kWave, kRows ? 4 : 1) void attn_mfma_kernel(
             // dim = 64c + 16g + 4i + e lives in o[4c + e][i] of lane group g
             const int dim = dim0 + j;
             const int b = 4 * (dim >> 6) + (dim & 3), g4 = (dim >> 4) & 3, i4 = (dim >> 2) & 3;
-            acc[w][j] = ms[((((size_t)w * 8 + b) * 8 + h) * 4 + g4) * 4 + i4];
+            acc[w][j] = ms[((((size_t)w * T::kOut + b) * 8 + h) * 4 + g4) * 4 + i4];
         }
     }
     float M = -INFINITY;
@@ -830,63 +612,39 @@ void launch_merge(const AttnArgs& a, const AttnPlan& p, hipStream_t stream) {
     }
 }
 
-template <int HD, int GP, int kDepth>
-hipError_t launch_split(const AttnArgs& a, const AttnPlan& p, hipStream_t stream) {
-    const size_t lds = split_lds_bytes<HD, GP>();
+template <int HD, int GP, bool kRows, bool kPrep>
+hipError_t launch_chunks(const AttnArgs& a, const AttnPlan& p, const QkPrep& prep, hipStream_t stream) {
+    using Lds = MfmaLds<HD, kWaves, kRows>;
     const float scale_log2 = (float)(1.4426950408889634 / sqrt((double)HD));
-    launch_kernel_in_call(p.n_splits <= 1, (attn_split_kernel<HD, GP, kDepth>), dim3(p.n_splits, a.kv_heads, a.nseq),
-                          dim3(kBlock), lds, stream, a.q, a.k_cache, a.v_cache, a.seq_stride, a.positions,
-                          a.position, a.max_len, a.heads, a.kv_heads, a.heads / a.kv_heads, p.chunk, scale_log2,
-                          a.workspace, p.n_splits, a.out);
+    launch_kernel_in_call(p.n_splits <= 1, (attn_mfma_kernel<HD, GP, kRows, kWaves, kPrep>),
+                          dim3(p.n_splits, a.kv_heads, a.nseq), dim3(kBlock), kPrep ? Lds::kPrepBytes : Lds::kBytes,
+                          stream, a.q, a.k_cache, a.v_cache, a.seq_stride, a.positions, a.position, a.max_len, a.heads,
+                          a.kv_heads, a.heads / a.kv_heads, p.chunk, scale_log2, a.workspace, p.n_splits, a.out, prep);
     const hipError_t e = hipGetLastError();
     if (e != hipSuccess || p.n_splits <= 1) return e;
     launch_merge<HD>(a, p, stream);
     return hipGetLastError();
 }
 
-template <int GP, bool kRows, int NW = kWaves>
-hipError_t launch_mfma(const AttnArgs& a, const AttnPlan& p, hipStream_t stream) {
-    const float scale_log2 = (float)(1.4426950408889634 / sqrt(128.0));
-    const dim3 grid(p.n_splits, a.kv_heads, a.nseq);
-    if (a.prep != nullptr) {
-        launch_kernel_in_call(p.n_splits <= 1, (attn_mfma_kernel<GP, kRows, NW, true>), grid, dim3(NW * kWave),
-                              MfmaLds<NW, kRows>::kPrepBytes, stream, a.q, a.k_cache, a.v_cache, a.seq_stride, a.positions,
-                              a.position, a.max_len, a.heads, a.kv_heads, a.heads / a.kv_heads, p.chunk, scale_log2,
-                              a.workspace, p.n_splits, a.out, *a.prep);
-    } else {
-        launch_kernel_in_call(p.n_splits <= 1, (attn_mfma_kernel<GP, kRows, NW, false>), grid, dim3(NW * kWave),
-                              MfmaLds<NW, kRows>::kBytes, stream, a.q, a.k_cache, a.v_cache, a.seq_stride, a.positions,
-                              a.position, a.max_len, a.heads, a.kv_heads, a.heads / a.kv_heads, p.chunk, scale_log2,
-                              a.workspace, p.n_splits, a.out, QkPrep{});
-    }
-    const hipError_t e = hipGetLastError();
-    if (e != hipSuccess || p.n_splits <= 1) return e;
-    launch_merge<128>(a, p, stream);
-    return hipGetLastError();
-}
-
 template <int HD, int GP>
-hipError_t launch_depth(const AttnArgs& a, const AttnPlan& p, hipStream_t s) {
-    if constexpr (HD == 128 && GP >= 2) {
-        // one tile in flight per wave; the plan picks the load form
-        if (p.depth != 1) return hipErrorInvalidValue;
-        return p.rows ? launch_mfma<GP, true>(a, p, s) : launch_mfma<GP, false>(a, p, s);
+hipError_t launch_group(const AttnArgs& a, const AttnPlan& p, hipStream_t s) {
+    if (a.prep != nullptr) {
+        if constexpr (HD == 128 && GP >= 2)
+            return p.rows ? launch_chunks<HD, GP, true, true>(a, p, *a.prep, s)
+                          : launch_chunks<HD, GP, false, true>(a, p, *a.prep, s);
+        return hipErrorInvalidValue;   // the q/k prologue is not built for this shape
     }
-    if (a.prep != nullptr) return hipErrorInvalidValue;   // the q/k prologue exists only in the MFMA kernel
-    switch (p.depth) {
-        case 1: return launch_split<HD, GP, 1>(a, p, s);
-        case 2: return launch_split<HD, GP, 2>(a, p, s);
-        default: return hipErrorInvalidValue;
-    }
+    return p.rows ? launch_chunks<HD, GP, true, false>(a, p, QkPrep{}, s)
+                  : launch_chunks<HD, GP, false, false>(a, p, QkPrep{}, s);
 }
 
 template <int HD>
 hipError_t launch_hd(const AttnArgs& a, const AttnPlan& p, hipStream_t s) {
     switch (p.gp) {
-        case 1: return launch_depth<HD, 1>(a, p, s);
-        case 2: return launch_depth<HD, 2>(a, p, s);
-        case 4: return launch_depth<HD, 4>(a, p, s);
-        case 8: return launch_depth<HD, 8>(a, p, s);
+        case 1: return launch_group<HD, 1>(a, p, s);
+        case 2: return launch_group<HD, 2>(a, p, s);
+        case 4: return launch_group<HD, 4>(a, p, s);
+        case 8: return launch_group<HD, 8>(a, p, s);
         default: return hipErrorInvalidValue;
     }
 }
@@ -905,21 +663,21 @@ int attention_plan_length(int length, int max_context) {
 
 // Work split: enough chunks for about `target_blocks` workgroups over all
 // (sequence, kv head) units, within a range of chunk lengths that keeps the
-// per-workgroup set-up and the partial write amortised -- for the
-// matrix-core kernel (head_dim 128, group >= 2) 64 positions up to 1024 with
-// at most 16 units, 512 with more; 256..512 for the other kernel (measured
-// on MI355X: one sequence at 512..32768 positions, 16 sequences of
-// 4096..32768); the chunk a multiple of 4 tiles, and at most kMaxSplits
-// chunks (bounds the merge's per-thread loop and the partials workspace).
+// per-workgroup set-up and the partial write amortised -- at head_dim 128
+// with GQA 64 positions up to 1024 with at most 16 units, 512 with more;
+// 256..512 at head_dim 64 and without GQA, whose bytes per position of one
+// launch unit are fewer (measured on MI355X: one sequence at 512..32768
+// positions, 16 sequences of 4096..32768); the chunk a multiple of a few
+// tiles, and at most kMaxSplits chunks (bounds the merge's per-thread loop
+// and the partials workspace).
 AttnPlan plan_attention(int max_len, int nseq, int kv_heads, int heads, int head_dim, int target_blocks) {
     AttnPlan p{};
     const int group = heads / kv_heads;
     p.gp = group <= 1 ? 1 : group <= 2 ? 2 : group <= 4 ? 4 : 8;
-    const bool mfma = head_dim == 128 && p.gp >= 2;
-    const int tp = mfma ? kMTile : (64 / p.gp) < 32 ? 64 / p.gp : 32;
-    const int quantum = tp * kWaves;
+    const bool gqa128 = head_dim == 128 && p.gp >= 2;
+    const int quantum = gqa128 ? 64 : (64 / p.gp) < 32 ? 64 / p.gp * kWaves : 32 * kWaves;
     const long long units = (long long)nseq * kv_heads;
-    const long long lo = mfma ? 64 : 256, hi = mfma ? (units <= 16 ? 1024 : 512) : 512;
+    const long long lo = gqa128 ? 64 : 256, hi = gqa128 ? (units <= 16 ? 1024 : 512) : 512;
     long long chunk = ((long long)max_len * units + target_blocks - 1) / target_blocks;
     chunk = chunk < lo ? lo : chunk > hi ? hi : chunk;
     const long long min_chunk = ((long long)max_len + kMaxSplits - 1) / kMaxSplits;
@@ -927,13 +685,11 @@ AttnPlan plan_attention(int max_len, int nseq, int kv_heads, int heads, int head
     chunk = ((chunk + quantum - 1) / quantum) * quantum;
     p.chunk = (int)chunk;
     p.n_splits = (int)((max_len + chunk - 1) / chunk);
-    // one tile in flight per wave: deeper rings measured no faster on
-    // gfx950 (the per-tile work, not the load latency, bounds a wave)
-    p.depth = 1;
     // whole-row loads once the launch holds more than two workgroups per CU
-    // (HBM saturates; measured at config 4: 251 against 298-308 us), direct
-    // loads below (latency-bound launches: 0.1-0.2 us faster)
-    p.rows = mfma && units * p.n_splits > 2LL * target_blocks;
+    // (HBM saturates; measured at 16 sequences of 4096..32768 positions, 32/8
+    // heads of 128: 251 against 298-308 us), direct loads below (latency-bound
+    // launches: 0.1-0.2 us faster)
+    p.rows = units * p.n_splits > 2LL * target_blocks;
     return p;
 }
 

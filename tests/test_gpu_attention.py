@@ -275,3 +275,36 @@ def test_batched_position_past_bound_is_cut_at_bound(hip):
         hip.device.attention_batched(dq, dk, dv, stride, dpos, bound, nseq, heads, kv, hd, dws, ws_bytes, do)
         outs.append(do.download(np.uint16))
     assert np.array_equal(outs[0], outs[1])
+
+
+@pytest.mark.parametrize("heads,kv,hd", [(4, 4, 64), (8, 4, 64), (12, 4, 64), (28, 4, 64), (32, 4, 64), (4, 4, 128)])
+@pytest.mark.parametrize("nseq,bound", [(2, 300), (56, 1300)])
+def test_batched_other_shapes_tile_edges(hip, orc, heads, kv, hd, nseq, bound):
+    """head_dim 64 (tiles of 32 positions) and no GQA on the matrix-core chunk
+    kernel: groups 1, 2, 3, 7 and 8, both load forms (2 sequences of up to
+    300 positions plan direct loads, 56 of up to 1300 whole-row loads), lengths
+    around tiles, waves and chunks; positions past a length hold NaN."""
+    chunk, splits = hip.device.attention_plan_info(bound, nseq, heads, kv, hd)
+    assert (nseq * kv * splits > 512) == (nseq == 56)
+    rng = hip.synth.Rng(9 + heads + nseq + hd)
+    edges = [1, bound, 15, 16, 17, 31, 32, 33, 63, 65, 127, 128, 129, 255, 256, 257, 511, 513, chunk, chunk + 1]
+    lens = [min(e, bound) for e in (edges * 3)[:nseq]]
+    stride = bound * kv * hd
+    k = hip.synth.normal_f16(rng, nseq * stride).reshape(nseq, bound, -1)
+    v = hip.synth.normal_f16(rng, nseq * stride).reshape(nseq, bound, -1)
+    for s, n in enumerate(lens):
+        k[s, n:], v[s, n:] = 0x7e00, 0x7e00
+    q = hip.synth.normal_f16(rng, nseq * heads * hd)
+    ws_bytes = hip.device.attention_workspace_bytes(bound, nseq, heads, kv, hd)
+    dws = hip.DeviceArray(max(ws_bytes, 16))
+    dq, dk, dv = (hip.DeviceArray.from_numpy(a) for a in (q, k, v))
+    dpos = hip.DeviceArray.from_numpy(np.array([n - 1 for n in lens], np.int32))
+    do = hip.DeviceArray(nseq * heads * hd * 2)
+    print(f"[attention edges] heads={heads} kv={kv} hd={hd} nseq={nseq} bound={bound}", flush=True)
+    hip.device.attention_batched(dq, dk, dv, stride, dpos, bound, nseq, heads, kv, hd, dws, ws_bytes, do)
+    got = do.download(np.uint16).view(np.float16).astype(np.float64).reshape(nseq, heads * hd)
+    for s, n in enumerate(lens[:len(edges)]):   # the rest repeat the lengths
+        ref = orc.attention(q[s * heads * hd:(s + 1) * heads * hd], k[s].reshape(-1), v[s].reshape(-1), n - 1, heads,
+                            kv, hd)
+        # one fp16 rounding of the output plus fp32 noise
+        assert np.all(np.abs(got[s] - ref) <= np.abs(ref) * 2 ** -10 + 1e-4), (n, np.abs(got[s] - ref).max())
