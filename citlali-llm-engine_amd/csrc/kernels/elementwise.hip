@@ -136,6 +136,44 @@ __global__ __launch_bounds__(kNormThreads) void add_rms_norm_kernel(uint16_t* __
         }
 }
 
+// Both of the above for whole runs of eight values, 16-byte aligned: thread t
+// holds its kRuns runs in registers (the order of the scalar forms: runs t,
+// t + 256, ...; a run past the end adds nothing), all loads issued together,
+// so the kernel is one memory round trip and one barrier.  Bound by that
+// latency; the scalar forms make three dependent passes of 2-byte loads.
+template <int kRuns, bool kAdd>
+__global__ __launch_bounds__(kNormThreads) void rms_norm_runs_kernel(const uint16_t* x, const uint16_t* d,
+                                                                     const uint16_t* w, uint16_t* sum, uint16_t* out,
+                                                                     int n, float eps) {
+    __shared__ float red[4];
+    const int runs = n >> 3;
+    u32x4 v[kRuns], dv[kAdd ? kRuns : 1], wv[kRuns];
+#pragma unroll
+    for (int i = 0; i < kRuns; ++i) {
+        const size_t at = (size_t)min(i * kNormThreads + (int)threadIdx.x, runs - 1) * 8;
+        v[i] = *reinterpret_cast<const u32x4*>(x + at);
+        if constexpr (kAdd) dv[i] = *reinterpret_cast<const u32x4*>(d + at);
+        wv[i] = *reinterpret_cast<const u32x4*>(w + at);
+    }
+    float s = 0.f;
+#pragma unroll
+    for (int i = 0; i < kRuns; ++i) {
+        const int r = i * kNormThreads + (int)threadIdx.x;
+        if constexpr (kAdd) v[i] = add_run(v[i], dv[i], true);
+        if (r < runs) {
+            s = sq_run(v[i], s);
+            if constexpr (kAdd) *reinterpret_cast<u32x4*>(sum + (size_t)r * 8) = v[i];
+        }
+    }
+    s = norm_block_sum(s, red);
+    const float inv = rsqrtf(s / (float)n + eps);
+#pragma unroll
+    for (int i = 0; i < kRuns; ++i) {
+        const int r = i * kNormThreads + (int)threadIdx.x;
+        if (r < runs) *reinterpret_cast<u32x4*>(out + (size_t)r * 8) = norm_run(v[i], wv[i], inv);
+    }
+}
+
 // Per-head RMSNorm of q and k (when their weights are given), NeoX RoPE of
 // both, and the store of this position's k and v rows into the caches: the
 // reference's launch_rms_norm_heads x2, launch_rope x2 and launch_store_kv
@@ -373,8 +411,34 @@ hipError_t launch_add_inplace(uint16_t* t, const uint16_t* d, int n, hipStream_t
     return hipGetLastError();
 }
 
+namespace {
+bool aligned16(const void* p) { return ((uintptr_t)p & 15u) == 0; }
+
+// The norm in runs of eight: whole runs at 16-byte aligned addresses, up to
+// eight runs per thread.  The residual is read by the thread that writes it, so
+// x and sum may be one buffer (and out may be x or d, as in the scalar form,
+// each run being read before it is written).
+template <bool kAdd>
+bool launch_norm_runs(const uint16_t* x, const uint16_t* d, const uint16_t* w, uint16_t* sum, uint16_t* out, int n,
+                      float eps, hipStream_t s) {
+    if (n % 8 != 0 || n > 8 * 8 * kNormThreads || !aligned16(x) || !aligned16(w) || !aligned16(out) ||
+        (kAdd && !aligned16(d)))
+        return false;
+    auto go = [&](auto kernel) {
+        launch_kernel(kernel, dim3(1), dim3(kNormThreads), 0, s, x, d, w, sum, out, n, eps);
+    };
+    const int per = (n / 8 + kNormThreads - 1) / kNormThreads;
+    if (per <= 1) go(rms_norm_runs_kernel<1, kAdd>);
+    else if (per <= 2) go(rms_norm_runs_kernel<2, kAdd>);
+    else if (per <= 4) go(rms_norm_runs_kernel<4, kAdd>);
+    else go(rms_norm_runs_kernel<8, kAdd>);
+    return true;
+}
+}  // namespace
+
 hipError_t launch_rms_norm(const uint16_t* in, const uint16_t* w, uint16_t* out, int n, float eps, hipStream_t s) {
-    launch_kernel(rms_norm_vec_kernel, dim3(1), dim3(kNormThreads), 0, s, in, w, out, n, eps);
+    if (!launch_norm_runs<false>(in, nullptr, w, nullptr, out, n, eps, s))
+        launch_kernel(rms_norm_vec_kernel, dim3(1), dim3(kNormThreads), 0, s, in, w, out, n, eps);
     return hipGetLastError();
 }
 
@@ -386,7 +450,8 @@ hipError_t launch_rms_norm_heads(const uint16_t* in, const uint16_t* w, uint16_t
 
 hipError_t launch_add_rms_norm(uint16_t* x, const uint16_t* d, const uint16_t* w, uint16_t* out, int n, float eps,
                                hipStream_t s) {
-    launch_kernel(add_rms_norm_kernel, dim3(1), dim3(kNormThreads), 0, s, x, d, w, out, n, eps);
+    if (!launch_norm_runs<true>(x, d, w, x, out, n, eps, s))
+        launch_kernel(add_rms_norm_kernel, dim3(1), dim3(kNormThreads), 0, s, x, d, w, out, n, eps);
     return hipGetLastError();
 }
 

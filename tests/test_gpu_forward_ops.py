@@ -344,3 +344,32 @@ def test_large_host_to_device_copies_are_exact(hip, nbytes, offset):
     got = dev.download(np.uint8, offset + nbytes + 4096)
     assert np.array_equal(got[offset:offset + nbytes], src)
     assert (got[:offset] == 0xA5).all() and (got[offset + nbytes:] == 0xA5).all()
+
+
+@pytest.mark.parametrize("n", [8, 1024, 2040, 2048, 2056, 3584, 8192, 8200, 16384, 16392, 1021])
+def test_norms_in_runs_equal_scalar_forms(hip, n):
+    """rms_norm and add_rms_norm on 16-byte aligned buffers (runs of eight in
+    registers where n is a multiple of 8 up to 16384) give the bits of the
+    same call at 2-byte aligned addresses (the scalar forms), also in place."""
+    rng = hip.synth.Rng(n)
+    x, d, w = (hip.synth.normal_f16(rng, n, s) for s in (2.0, 1.0, 1.0))
+
+    def run(off, add, in_place):
+        pad = np.full(off, 0x7e00, np.uint16)
+        dx, dd, dw = (up(hip, np.concatenate([pad, a, pad])) for a in (x, d, w))
+        do = up(hip, np.full(n + 2 * off + 8, 0x1234, np.uint16))
+        at = lambda b: b.at(2 * off)
+        out = dx if in_place else do
+        if add:
+            hip.device.add_rms_norm(at(dx), at(dd), at(dw), at(out), n, 1e-6)
+        else:
+            hip.device.rms_norm(at(dx), at(dw), at(out), n, 1e-6)
+        if not in_place:
+            tail = do.download(np.uint16)
+            assert np.all(tail[:off] == 0x1234) and np.all(tail[off + n:] == 0x1234)
+        return [b.download(np.uint16, n, 2 * off) for b in (out, dx)]
+
+    for add in (False, True):
+        for in_place in (False, True):
+            for g, r in zip(run(0, add, in_place), run(1, add, in_place)):
+                assert np.array_equal(g, r), (add, in_place)
