@@ -58,8 +58,8 @@ __device__ __forceinline__ SeqSpan seq_span(const int32_t* positions, int positi
 //    - direct: lane = (row col, 16-byte slices grp, grp + 4, ...), 16 rows x
 //      64 bytes per instruction, K straight into the A operand, V into an LDS
 //      tile; the refill is issued once the scores are in;
-//    - rows (launches of more than two workgroups per CU, where HBM
-//      saturates): each nontemporal instruction reads whole rows, four of 256
+//    - rows (launches of long chunks or of more than two workgroups per
+//      CU): each nontemporal instruction reads whole rows, four of 256
 //      or eight of 128 bytes, which a probe of the 256-byte shape reads at
 //      ~7 TB/s against ~5.9 for 16 rows x 64 bytes; K and V go to
 //      wave-private LDS rows, the refill is issued at once and K is read back
@@ -687,9 +687,13 @@ AttnPlan plan_attention(int max_len, int nseq, int kv_heads, int heads, int head
     p.n_splits = (int)((max_len + chunk - 1) / chunk);
     // whole-row loads once the launch holds more than two workgroups per CU
     // (HBM saturates; measured at 16 sequences of 4096..32768 positions, 32/8
-    // heads of 128: 251 against 298-308 us), direct loads below (latency-bound
-    // launches: 0.1-0.2 us faster)
-    p.rows = units * p.n_splits > 2LL * target_blocks;
+    // heads of 128: 207 against 241 us) or a wave streams eight tiles and more
+    // (split + merge, us, rows against direct: one sequence of 16384 16.4 /
+    // 17.6, of 30011 25.5 / 26.8, 2 of 8192 16.3 / 17.4, 4 of 2000..8192 23.0 /
+    // 25.5, 16 of 100..1500 18.6 / 22.0); direct loads below, where a wave's few
+    // tiles wait for latency and the LDS round trip of K shows (8192 positions
+    // 10.6 against 11.3, 2048 7.2 against 7.8)
+    p.rows = chunk >= 512 || units * p.n_splits > 2LL * target_blocks;
     return p;
 }
 
