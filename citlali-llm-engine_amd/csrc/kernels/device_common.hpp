@@ -218,6 +218,14 @@ __device__ __forceinline__ float norm_block_sum(float s, float* red) {
     return ((red[0] + red[1]) + red[2]) + red[3];
 }
 
+// Run that thread `tid` loads in pass i of staging `runs` runs: its own, or
+// one that exists (not used) where it has none -- its first one, and with
+// fewer runs than threads (K = 1024: 128) the last one.
+__host__ __device__ constexpr int staged_run(int runs, int i, int tid) {
+    const int own = i * kNormThreads + tid;
+    return own < runs ? own : tid < runs ? tid : runs - 1;
+}
+
 // Head RMSNorm and NeoX RoPE pieces shared by the q/k norm + RoPE + store
 // kernel and the attention launch that does the same work in its prologue,
 // so both give the same bits.  rsqrt(mean(x^2) + eps) of a 128-dim head whose
@@ -269,6 +277,40 @@ __device__ __forceinline__ void wave_lds_sync() {
 __device__ __forceinline__ int issue_after(int v, float a, float b) {
     asm volatile("" : "+v"(v) : "v"(a), "v"(b));
     return v;
+}
+
+// The value of entry 0, 1 or 2.  As assignments, since a conditional
+// expression of three members is an lvalue: the compiler selects the address
+// and keeps the struct in scratch memory.
+template <typename T>
+__device__ __forceinline__ T pick3(bool s1, bool s2, T v0, T v1, T v2) {
+    T r = v0;
+    if (s1) r = v1;
+    if (s2) r = v2;
+    return r;
+}
+
+// ---- copies straight into LDS ---------------------------------------------
+// Waits until at most n of the wave's vector-memory operations are in flight.
+template <int n>
+__device__ __forceinline__ void wait_vm() {
+    static_assert(n < 64, "vmcnt");
+    __builtin_amdgcn_s_waitcnt(0x0f70 | (n & 15) | ((n >> 4) << 14));
+    asm volatile("" ::: "memory");
+}
+// LDS traffic of the wave done; copies in flight stay in flight.
+__device__ __forceinline__ void wait_lds() { asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory"); }
+// lds_barrier() as the compiler would not write it beside such copies: its
+// fences would wait for them.
+__device__ __forceinline__ void lds_only_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
+
+// 16 bytes per lane to LDS at dst_wave_base + 16 lane; kNontemporal for data
+// read once in whole cache lines.
+template <bool kNontemporal = false>
+__device__ __forceinline__ void copy16_to_lds(const uint8_t* src, uint8_t* dst_wave_base) {
+    __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)src,
+                                     (__attribute__((address_space(3))) void*)dst_wave_base, 16, 0,
+                                     kNontemporal ? 2 : 0);
 }
 
 }  // namespace citlali::hip

@@ -7,6 +7,7 @@
 #include <stddef.h>
 #include <stdint.h>
 
+#include <atomic>
 #include <vector>
 
 namespace citlali::hip {
@@ -58,6 +59,34 @@ inline void launch_kernel(Kernel kernel, dim3 grid, dim3 block, size_t lds, hipS
     launch_kernel_in_call(true, kernel, grid, block, lds, stream, args...);
 }
 
+constexpr int kLdsPerCu = 160 * 1024;
+
+inline int device_cus() {
+    static int cus = 0;
+    if (!cus) {
+        int dev = 0;
+        (void)hipGetDevice(&dev);
+        if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus <= 0)
+            cus = 256;
+    }
+    return cus;
+}
+
+// More than 64 KB of LDS is asked for per kernel and device, once.
+template <auto kKernel>
+inline hipError_t allow_lds(int lds) {
+    if (lds <= 64 * 1024) return hipSuccess;
+    static std::atomic<uint64_t> done{0};
+    int dev = 0;
+    hipError_t e = hipGetDevice(&dev);
+    if (e != hipSuccess) return e;
+    const uint64_t bit = (uint64_t)1 << (dev & 63);
+    if (done.load(std::memory_order_acquire) & bit) return hipSuccess;
+    e = hipFuncSetAttribute(reinterpret_cast<const void*>(kKernel), hipFuncAttributeMaxDynamicSharedMemorySize, kLdsPerCu);
+    if (e == hipSuccess) done.fetch_or(bit, std::memory_order_release);
+    return e;
+}
+
 // ---- fused dequant GEMV (matvec_kquant.hip) ----
 // kind: 4 = Q4_K, 6 = Q6_K, 1 = fp16 weights
 size_t matvec_lds_bytes(int kind, int K);
@@ -72,6 +101,10 @@ bool matvec_gate_up_length(int K);
 // through the streaming kernels of the K-quant GEMVs
 hipError_t launch_matvec_f16_blocks(const uint16_t* w, const uint16_t* x, void* y, bool f32_out, int K, int N,
                                     hipStream_t s);
+// fp16 weights [N][K] of any K that f16_rows_length takes (matvec_f16.hip)
+bool f16_rows_length(int K);
+hipError_t launch_matvec_f16_rows(const uint16_t* w, const uint16_t* x, void* y, bool f32_out, int K, int N,
+                                  hipStream_t s);
 hipError_t launch_matvec_q4k(const uint8_t* w, const uint16_t* x, void* y, bool f32_out, int K, int N,
                              hipStream_t s);
 hipError_t launch_matvec_q6k(const uint8_t* w, const uint16_t* x, void* y, bool f32_out, int K, int N,

@@ -37,7 +37,6 @@ constexpr int kWavesPerBlock = kBlock / kWave;
 constexpr int kSum32 = 0;     // Q4K: sum over each 32-value group, [b][g]
 constexpr int kSumQ6 = 1;     // Q6K: 16-value slices, [b][h][ih][k]
 constexpr int kPlain = 2;     // F16: x in its own order, no sums
-constexpr int kBatch = 4;        // wave steps whose loads are issued together
 // The streaming kernels run two workgroups per CU (two waves per SIMD):
 // their register budget is capped to keep both resident.
 constexpr int kWavesPerSimd = 2;
@@ -89,13 +88,6 @@ __device__ __forceinline__ void stage_x8(const u32x4 raw, int v8, uint32_t* xp, 
     }
 }
 
-// Run that thread `tid` loads in pass i of staging `runs` runs: its own, or
-// one that exists (not used) where it has none -- its first one, and with
-// fewer runs than threads (K = 1024: 128) the last one.
-__host__ __device__ constexpr int staged_run(int runs, int i, int tid) {
-    const int own = i * kBlock + tid;
-    return own < runs ? own : tid < runs ? tid : runs - 1;
-}
 constexpr bool staged_runs_exist(int runs) {
     for (int i = 0; i * kBlock < runs; ++i)
         for (int t = 0; t < kBlock; ++t)
@@ -166,17 +158,6 @@ struct XStage {
         lds_barrier();
     }
 };
-
-// Any K (a multiple of 256): every thread stages runs v8 = tid, tid + 256, ...
-// (a multiple of 4 runs per thread keeps each group's runs on consecutive
-// threads of one pass).
-template <int kLayout>
-__device__ __forceinline__ void stage_x(const uint16_t* __restrict__ x, int K, uint32_t* xp, float* sx) {
-    const int n8 = K >> 3;
-    for (int v8 = threadIdx.x; v8 < n8; v8 += kBlock)
-        stage_x8<kLayout>(*reinterpret_cast<const u32x4*>(x + (size_t)v8 * 8), v8, xp, sx);
-    lds_barrier();
-}
 
 // ---------------------------------------------------------------------------
 // Q4_K: d(f16) dmin(f16) scales[12] qs[128]   (weight_loader.cpp:150-161)
@@ -715,58 +696,6 @@ __global__ __launch_bounds__(kGateUpBlock, 2) void matvec_gate_up_kernel(const u
     }
 }
 
-// Any super-block count: a wave owns kRows rows and walks their super-blocks
-// as one flat list; a lane's row is found by multiply-high division.
-template <class QT, bool kF32, int kRows>
-__global__ __launch_bounds__(kBlock) void matvec_flat_kernel(const uint8_t* __restrict__ w,
-                                                             const uint16_t* __restrict__ x,
-                                                             void* __restrict__ y, int K, int N,
-                                                             uint64_t magic) {
-    extern __shared__ __align__(16) uint8_t smem[];
-    uint32_t* xp = reinterpret_cast<uint32_t*>(smem);
-    float* sx = reinterpret_cast<float*>(smem + (size_t)K * 2);
-    stage_x<QT::kSumLayout>(x, K, xp, sx);
-
-    const int lane = threadIdx.x & (kWave - 1);
-    const int wave = threadIdx.x / kWave;
-    const int l4 = lane % QT::kLanesPerSb;
-    const int sub = lane / QT::kLanesPerSb;
-    const int nb = K >> 8;
-    const int row0 = (blockIdx.x * kWavesPerBlock + wave) * kRows;
-    const int rows = min(kRows, N - row0);
-    const int nflat = rows > 0 ? rows * nb : 0;
-
-    float acc[kRows];
-#pragma unroll
-    for (int k = 0; k < kRows; ++k) acc[k] = 0.f;
-
-    for (int f0 = 0; f0 < nflat; f0 += kBatch * QT::kSbPerStep) {
-        typename QT::Frag fr[kBatch];
-        int rl[kBatch], bl[kBatch];
-#pragma unroll
-        for (int u = 0; u < kBatch; ++u) {
-            const uint32_t f = (uint32_t)(f0 + u * QT::kSbPerStep + sub);
-            const uint32_t r = (uint32_t)(((uint64_t)f * magic) >> 32);
-            rl[u] = (int)f < nflat ? (int)r : -1;
-            bl[u] = (int)(f - r * (uint32_t)nb);
-            if (rl[u] >= 0) fr[u] = QT::load(w + ((size_t)row0 * nb + f) * QT::kBytes, l4);
-        }
-#pragma unroll
-        for (int u = 0; u < kBatch; ++u) {
-            if (rl[u] >= 0) {
-                const float c = QT::dot(fr[u], l4, xp, sx, bl[u]);
-#pragma unroll
-                for (int k = 0; k < kRows; ++k) acc[k] += (rl[u] == k) ? c : 0.f;
-            }
-        }
-    }
-#pragma unroll
-    for (int k = 0; k < kRows; ++k) {
-        const float s = wave_sum(acc[k]);
-        if (lane == 0 && k < rows) store_y<kF32>(y, row0 + k, s);
-    }
-}
-
 // ---------------------------------------------------------------------------
 // Tile kernels: Q4_K / Q6_K rows of any super-block count nb on the matrix
 // cores (v_mfma_f32_16x16x32_f16), for the counts that do not fill the wave
@@ -920,22 +849,6 @@ struct TileShape {
     __host__ __device__ static constexpr int ring(int nb) { return part(nb) + 2 * kMats * kTileWaves * kTileCols * 4; }
     __host__ __device__ static constexpr int bytes(int nb) { return ring(nb) + kTileWaves * kDepth * kSlot; }
 };
-
-// Waits until at most n of the wave's vector-memory operations are in flight.
-template <int n>
-__device__ __forceinline__ void wait_vm() {
-    static_assert(n < 64, "vmcnt");
-    __builtin_amdgcn_s_waitcnt(0x0f70 | (n & 15) | ((n >> 4) << 14));
-    asm volatile("" ::: "memory");
-}
-// LDS traffic of the wave done; copies in flight stay in flight.
-__device__ __forceinline__ void wait_lds() { asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory"); }
-__device__ __forceinline__ void tile_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
-
-__device__ __forceinline__ void copy16_to_lds(const uint8_t* src, uint8_t* dst_wave_base) {
-    __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)src,
-                                     (__attribute__((address_space(3))) void*)dst_wave_base, 16, 0, 0);
-}
 
 struct TileAt {
     const uint8_t* w[2];
@@ -1098,7 +1011,7 @@ __device__ __forceinline__ void tile_rows(const uint16_t* __restrict__ x, int nb
             }
             s = wave_sum(s);
             if (lane == 0) red[wave] = s;
-            tile_barrier();
+            lds_only_barrier();
             const float inv = rsqrtf((((red[0] + red[1]) + red[2]) + red[3]) / (float)(runs * 8) + nrm.eps);
 #pragma unroll
             for (int i = 0; i < kIters; ++i) {
@@ -1106,7 +1019,7 @@ __device__ __forceinline__ void tile_rows(const uint16_t* __restrict__ x, int nb
                 if (r < runs) put(norm_run(raw[i], wr[i], inv), r);
             }
         } else {
-            tile_barrier();
+            lds_only_barrier();
         }
     } else {
         // this wave's runs are in LDS once only the ring copies are in flight
@@ -1122,7 +1035,7 @@ __device__ __forceinline__ void tile_rows(const uint16_t* __restrict__ x, int nb
             if (r < runs) put(v, r);
         }
     }
-    tile_barrier();
+    lds_only_barrier();
 
     // A operand address: slot lane & 3 of this lane group's quarter, or zeros
     const bool a_live = ((lane & 15) >> 2) == g;
@@ -1169,7 +1082,7 @@ __device__ __forceinline__ void tile_rows(const uint16_t* __restrict__ x, int nb
             acc = sum32(sum16(acc));   // the row's four quarters
             if (g == 0) pt[(m * kTileWaves + cls) * kTileCols + n] = acc;
         }
-        tile_barrier();   // the tile's class sums are in LDS
+        lds_only_barrier();   // the tile's class sums are in LDS
         if (wave == (k & (kTileWaves - 1))) {
             float sum[kMats];
 #pragma unroll
@@ -1203,17 +1116,6 @@ TileSet make_tile_set(const RowSet& rs) {
     }
     return ts;
 }
-// The value of entry 0, 1 or 2.  As assignments, since a conditional
-// expression of three members is an lvalue: the compiler selects the address
-// and keeps the struct in scratch memory.
-template <typename T>
-__device__ __forceinline__ T pick3(bool s1, bool s2, T v0, T v1, T v2) {
-    T r = v0;
-    if (s1) r = v1;
-    if (s2) r = v2;
-    return r;
-}
-
 // tile t of a set, in registers
 template <int kRows>
 struct SetTiles {
@@ -1281,17 +1183,6 @@ __global__ __launch_bounds__(kTileBlock, 4) void matvec_tile_gate_up_kernel(cons
         });
 }
 
-int device_cus() {
-    static int cus = 0;
-    if (!cus) {
-        int dev = 0;
-        (void)hipGetDevice(&dev);
-        if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus <= 0)
-            cus = 256;
-    }
-    return cus;
-}
-
 // `per_cu` workgroups per CU (two: two waves per SIMD), never more waves than
 // rows.
 int stream_grid(int rows, int per_cu = 2) {
@@ -1343,22 +1234,6 @@ __host__ __device__ constexpr bool tile_length(int nb) {
     }
 }
 
-constexpr int kLdsPerCu = 160 * 1024;
-
-// More than 64 KB of LDS is asked for per kernel and device, once.
-template <typename Kernel>
-hipError_t allow_lds(Kernel kernel) {
-    static std::atomic<uint64_t> done{0};
-    int dev = 0;
-    hipError_t e = hipGetDevice(&dev);
-    if (e != hipSuccess) return e;
-    const uint64_t bit = (uint64_t)1 << (dev & 63);
-    if (done.load(std::memory_order_acquire) & bit) return hipSuccess;
-    e = hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, kLdsPerCu);
-    if (e == hipSuccess) done.fetch_or(bit, std::memory_order_release);
-    return e;
-}
-
 // Two workgroups per CU where the LDS of two fits, never more than tiles.
 int tile_grid(int tiles, int lds) { return std::min(tiles, device_cus() * (2 * lds <= kLdsPerCu ? 2 : 1)); }
 
@@ -1375,11 +1250,11 @@ template <class QT, bool kNorm>
 hipError_t launch_tile(int nb, const RowSet& rs, const uint16_t* x, bool f32, const NormIn& nrm, hipStream_t stream) {
     return with_norm_iters<kNorm>(nb, [&](auto it) {
         using SH = TileShape<QT, 1>;
-        auto kernel = matvec_tile_kernel<SH, decltype(it)::value>;
-        const hipError_t e = allow_lds(kernel);
-        if (e != hipSuccess) return e;
+        constexpr auto kernel = matvec_tile_kernel<SH, decltype(it)::value>;
         const TileSet ts = make_tile_set<QT>(rs);
         const int lds = SH::bytes(nb);
+        const hipError_t e = allow_lds<kernel>(lds);
+        if (e != hipSuccess) return e;
         launch_kernel(kernel, dim3(tile_grid(ts.end[2], lds)), dim3(kTileBlock), (size_t)lds, stream, ts, x, nb,
                       (int)f32, nrm);
         return hipGetLastError();
@@ -1400,8 +1275,8 @@ hipError_t launch_tile_mixed(int nb, const RowSet& a, const RowSet& b, const uin
     ga = std::max(1, std::min(ga, std::min(grid - 1, ta.end[2])));
     const int gb = std::max(1, std::min(grid - ga, tb.end[2]));
     return with_norm_iters<kNorm>(nb, [&](auto it) {
-        auto kernel = matvec_tile_group_kernel<SA, SB, decltype(it)::value>;
-        const hipError_t e = allow_lds(kernel);
+        constexpr auto kernel = matvec_tile_group_kernel<SA, SB, decltype(it)::value>;
+        const hipError_t e = allow_lds<kernel>(lds);
         if (e != hipSuccess) return e;
         launch_kernel(kernel, dim3(ga + gb), dim3(kTileBlock), (size_t)lds, stream, ta, tb, ga, x, nb, nrm);
         return hipGetLastError();
@@ -1413,10 +1288,10 @@ hipError_t launch_tile_gate_up(const uint8_t* wg, const uint8_t* wu, const uint1
                                const NormIn& nrm, hipStream_t stream) {
     return with_norm_iters<kNorm>(nb, [&](auto it) {
         using SH = TileShape<QT, 2>;
-        auto kernel = matvec_tile_gate_up_kernel<SH, decltype(it)::value>;
-        const hipError_t e = allow_lds(kernel);
-        if (e != hipSuccess) return e;
+        constexpr auto kernel = matvec_tile_gate_up_kernel<SH, decltype(it)::value>;
         const int lds = SH::bytes(nb), tiles = tiles_of<QT>(N);
+        const hipError_t e = allow_lds<kernel>(lds);
+        if (e != hipSuccess) return e;
         launch_kernel(kernel, dim3(tile_grid(tiles, lds)), dim3(kTileBlock), (size_t)lds, stream, wg, wu, x, act, nb,
                       tiles, N, nrm);
         return hipGetLastError();
@@ -1515,15 +1390,10 @@ hipError_t launch_matvec(const uint8_t* w, const uint16_t* x, void* y, int K, in
     }
     const size_t lds = lds_bytes<QT>(K);
     if (!launch_stream_for<QT, kF32, 1>(nb, rs, x, lds, kNoNorm, stream)) {
-        if constexpr (!std::is_same<QT, F16>::value) return hipErrorInvalidValue;   // not reached: tile_length
-        // any other fp16 length: flat walk over the 256-value blocks of 4 rows
-        constexpr int kRows = 4;
-        // floor(f / nb) == (f * magic) >> 32 for every f < 2^20 (nb <= 112)
-        const uint64_t magic = ((uint64_t)1 << 32) / (uint64_t)nb + 1u;
-        const int rows_per_block = kRows * kWavesPerBlock;
-        const int grid = (N + rows_per_block - 1) / rows_per_block;
-        launch_kernel((matvec_flat_kernel<F16, kF32, kRows>), dim3(grid), dim3(kBlock), lds, stream, w, x, y, K,
-                      N, magic);
+        // fp16 rows of any other length (Q4_K / Q6_K: tile_length)
+        if constexpr (std::is_same<QT, F16>::value)
+            return launch_matvec_f16_rows(reinterpret_cast<const uint16_t*>(w), x, y, kF32, K, N, stream);
+        return hipErrorInvalidValue;
     }
     return hipGetLastError();
 }

@@ -373,3 +373,27 @@ def test_norms_in_runs_equal_scalar_forms(hip, n):
         for in_place in (False, True):
             for g, r in zip(run(0, add, in_place), run(1, add, in_place)):
                 assert np.array_equal(g, r), (add, in_place)
+
+
+@pytest.mark.parametrize("k", [8, 504, 512, 520, 1000, 1792, 3584, 17408, 28672])
+def test_matvec_fp16_other_lengths(hip, orc, k):
+    """fp16 rows of the lengths without a streaming instantiation (any
+    multiple of 8): below, at and just past whole 512-value steps, the longest;
+    rows around the four waves of a workgroup and several per wave.  The last
+    row is followed by NaN: a partial step must not count what lies behind it."""
+    for n in [1, 3, 4, 5, 9] + ([5003] if k in (504, 1792) else []):
+        print(f"[matvec fp16] n={n} k={k}", flush=True)
+        rng = hip.synth.Rng(n + k)
+        w, x = hip.synth.normal_f16(rng, n * k), hip.synth.normal_f16(rng, k)
+        dw = up(hip, np.concatenate([w, np.full(512, 0x7e00, np.uint16)]))
+        dx, dy = up(hip, np.concatenate([x, np.full(512, 0x7e00, np.uint16)])), hip.DeviceArray(n * 4 + 64)
+        dy.zero()
+        hip.device.matvec("fp16", dw, dx, dy, k, n, f32_out=True)
+        got = dy.download(np.float32, n + 16)
+        assert not got[n:].any(), "wrote past the last row"
+        wf, xf = vals(w).reshape(n, k).astype(np.float64), vals(x).astype(np.float64)
+        # fp32 sums of k exact products: a few ulps of the terms' magnitude
+        bound = 2.0 ** -21 * (np.abs(wf) @ np.abs(xf)) + 1e-7
+        assert np.all(np.abs(got[:n] - wf @ xf) <= bound)
+        hip.device.matvec("fp16", dw, dx, dy, k, n)
+        assert np.array_equal(dy.download(np.uint16, n), got[:n].astype(np.float16).view(np.uint16))
