@@ -20,9 +20,10 @@
 //    x pair and accumulates in fp32 -- no per-value int->float conversion.
 //  * The per-group offset terms (Q4_K "- dmin*m", Q6_K "- 32") need
 //    sum(x) over each group; the block computes those sums while staging x.
-//  * No MFMA: M = 1 is not a dense contraction.  The bound is HBM.
+//  * Rows that fill a wave's steps use no MFMA: M = 1 is not a dense
+//    contraction, and the bound is HBM.  The tile kernels below, for the
+//    other lengths, take rows as MFMA columns so that no lane idles.
 #include <algorithm>
-#include <atomic>
 #include <type_traits>
 
 #include "device_common.hpp"
