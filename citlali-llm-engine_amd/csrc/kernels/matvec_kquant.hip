@@ -20,9 +20,10 @@
 //    x pair and accumulates in fp32 -- no per-value int->float conversion.
 //  * The per-group offset terms (Q4_K "- dmin*m", Q6_K "- 32") need
 //    sum(x) over each group; the block computes those sums while staging x.
-//  * Rows that fill a wave's steps use no MFMA: M = 1 is not a dense
-//    contraction, and the bound is HBM.  The tile kernels below, for the
-//    other lengths, take rows as MFMA columns so that no lane idles.
+//  * No MFMA: M = 1 is not a dense contraction, and the bound is HBM.  (The
+//    tile kernels below took rows as MFMA columns for a while, 3-15% faster;
+//    the matrix cores' sums are not v_dot2_f32_f16's, and Q6_K rows were up
+//    to 4.7 times further from 64-bit sums.)
 #include <algorithm>
 #include <type_traits>
 
@@ -54,7 +55,7 @@ __device__ __forceinline__ u32x4 permute_x8(const u32x4 raw) {
 
 // The run's share of the group sums in the layout kLayout.
 template <int kLayout>
-__device__ __forceinline__ void stage_sums8(const u32x4 raw, int v8, float* sx, float scale = 1.f) {
+__device__ __forceinline__ void stage_sums8(const u32x4 raw, int v8, float* sx) {
     float s = 0.f;
     s += h2f(raw.x & 0xffffu) + h2f(raw.x >> 16);
     s += h2f(raw.y & 0xffffu) + h2f(raw.y >> 16);
@@ -64,7 +65,7 @@ __device__ __forceinline__ void stage_sums8(const u32x4 raw, int v8, float* sx, 
         // four consecutive threads hold one 32-value group
         s += dpp<kDppXor1>(s);
         s += dpp<kDppXor2>(s);
-        if ((v8 & 3) == 0) sx[v8 >> 2] = s * scale;
+        if ((v8 & 3) == 0) sx[v8 >> 2] = s;
     } else {
         // two consecutive threads hold one 16-value slice
         s += dpp<kDppXor1>(s);
@@ -72,7 +73,7 @@ __device__ __forceinline__ void stage_sums8(const u32x4 raw, int v8, float* sx, 
             const int v = v8 * 8;
             const int b = v >> 8, in = v & 255;
             const int h = in >> 7, k = (in & 127) >> 5, ih = (in & 31) >> 4;
-            sx[b * 16 + h * 8 + ih * 4 + k] = s * scale;
+            sx[b * 16 + h * 8 + ih * 4 + k] = s;
         }
     }
 }
@@ -705,21 +706,13 @@ __global__ __launch_bounds__(kGateUpBlock, 2) void matvec_gate_up_kernel(const u
 }
 
 // ---------------------------------------------------------------------------
-// Tile kernels: Q4_K / Q6_K rows of any super-block count nb on the matrix
-// cores (v_mfma_f32_16x16x32_f16), for the counts that do not fill the wave
-// steps of the streaming kernels (see tile_length).
+// Tile kernels: Q4_K / Q6_K rows of any super-block count nb, for the counts
+// that do not fill the wave steps of the streaming kernels (see tile_length).
 //
-// A tile is up to 16 rows, MFMA columns; a wave's step is one super-block of
-// each of them, lane (row n = lane % 16, quarter g = lane / 16) holding
-// the 64 codes that lane g of a super-block holds in the streaming kernels.
-// The codes go in as the B operand (fp16 subnormals, exact, as in the dot2
-// form) and x as A, unchanged fp16 values: A row 4g + i is slot i of quarter
-// g and is non-zero only in lane group g, so lane (n, g) gets the sums of its
-// own codes with x slot i in accumulator i -- one sum per scale, no lane
-// moves.  Slots: the four 16-value parts of a Q6_K quarter, the first and
-// second half of the low and the high group of a Q4_K one.  Per 64 codes a
-// lane spends 40 (Q4_K) / 80 (Q6_K) bit operations and 8 MFMAs; the dot2 form
-// needs 32 dots more and a 64-lane sum per row.
+// A tile is up to 16 rows; a wave's step is one super-block of each of them,
+// lane (row n = lane % 16, quarter g = lane / 16) holding the 64 codes that
+// lane g of a super-block holds in the streaming kernels and forming the same
+// dot with the same x.
 //
 // Each wave copies its steps' blocks, a piece of 144 / 210 bytes per row,
 // straight into a ring of kDepth LDS slots (global_load_lds_dwordx4, aligned
@@ -729,108 +722,31 @@ __global__ __launch_bounds__(kGateUpBlock, 2) void matvec_gate_up_kernel(const u
 // this lane layout, a Q6_K matrix moved 4.5 TB/s against 6 here.
 //
 // The steps of a workgroup's tiles are dealt out to its eight waves in turn,
-// so no lane group or wave idles at any nb.  A step leaves its 16 row sums in
-// LDS; once a tile's steps are done one wave adds them in a fixed order.  A
-// row's result depends on nothing but its own blocks and x: every launch
-// form of a length gives the same bits.
+// so no lane group or wave idles at any nb.  A wave adds its blocks b of one
+// residue b % 16 in increasing order and leaves the residue's 16 row sums in
+// LDS; once a tile's steps are done one wave adds the residues in the order
+// of wave_sum over the lanes (residue, quarter): the streaming kernels' order
+// of a row, so the two give the same bits.
 // ---------------------------------------------------------------------------
-typedef _Float16 half8 __attribute__((ext_vector_type(8)));
-
 constexpr int kTileCols = 16;
 constexpr int kTileWaves = 8;
 constexpr int kTileBlock = kTileWaves * kWave;
-constexpr int kZeroBytes = 128;   // what A lanes outside their quarter read (two 16-byte slots 64 bytes apart)
-
-__device__ __forceinline__ f32x4 mfma32(u32x4 a, u32x4 b, f32x4 c) {
-    return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(half8, a), __builtin_bit_cast(half8, b), c, 0, 0,
-                                                  0);
-}
+constexpr int kResidues = 16;   // QT::kSbPerStep
+// tile lengths whose rows are summed in the flat walk's order (every one
+// without a streaming instantiation)
+__host__ __device__ constexpr bool flat_order(int nb) { return nb != 20; }
 
 template <class QT>
 struct TileOps;
-
 template <>
 struct TileOps<Q4K> {
     static constexpr int kPieces = 9;   // 16-byte pieces per block row
     static constexpr int kRows = 14;    // rows of a tile
-    static constexpr float kSumScale = 1.f;
-    // 16-byte slot of run r (eight x values) of a super-block: [quarter][t][slot]
-    __device__ static __forceinline__ int slot(int r) {
-        const int grp = r >> 2, k = r & 3;   // 32-value group, run in it
-        return (grp >> 1) * 8 + (k & 1) * 4 + (grp & 1) + 2 * (k >> 1);
-    }
-    using Sums = f32x2;
-    __device__ static __forceinline__ Sums sums(const float* sx, int b, int g) {
-        return *reinterpret_cast<const f32x2*>(sx + b * 8 + 2 * g);
-    }
-    __device__ static __forceinline__ float dot(const Q4K::Frag& f, int g, u32x4 a0, u32x4 a1, Sums s) {
-#pragma clang fp contract(off)   // the same bits in every kernel that inlines it
-        const uint32_t q[8] = {f.q0.x, f.q0.y, f.q0.z, f.q0.w, f.q1.x, f.q1.y, f.q1.z, f.q1.w};
-        u32x4 lo[4], hi[4];
-#pragma unroll
-        for (int t = 0; t < 4; ++t) {
-            const uint32_t w0 = q[2 * t], w1 = q[2 * t + 1], v0 = w0 >> 8, v1 = w1 >> 8;
-            lo[t] = u32x4{w0 & 0x000f000fu, v0 & 0x000f000fu, w1 & 0x000f000fu, v1 & 0x000f000fu};   // q * 2^-24
-            hi[t] = u32x4{w0 & 0x00f000f0u, v0 & 0x00f000f0u, w1 & 0x00f000f0u, v1 & 0x00f000f0u};   // q * 2^-20
-        }
-        const f32x4 z = {0.f, 0.f, 0.f, 0.f};
-        f32x4 d0 = mfma32(a0, lo[0], z), d1 = mfma32(a0, hi[0], z), d2 = mfma32(a0, lo[2], z), d3 = mfma32(a0, hi[2], z);
-        d0 = mfma32(a1, lo[1], d0);
-        d1 = mfma32(a1, hi[1], d1);
-        d2 = mfma32(a1, lo[3], d2);
-        d3 = mfma32(a1, hi[3], d3);
-        uint32_t sc, mn;
-        Q4K::scale_codes(f, g, sc, mn);
-        const float d24 = h2f(f.hdr.x & 0xffffu) * 16777216.0f, dmin = h2f(f.hdr.x >> 16);
-        // d (sc_lo P_lo + sc_hi P_hi) - dmin (m_lo S_lo + m_hi S_hi)
-        const float p_hi = (float)((sc >> 8) & 0xffu) * (d1[1] + d3[3]);
-        const float p = fmaf((float)(sc & 0xffu), d0[0] + d2[2], p_hi * 0.0625f);
-        const float m = fmaf((float)(mn & 0xffu), s.x, (float)((mn >> 8) & 0xffu) * s.y);
-        return fmaf(d24, p, -(dmin * m));
-    }
 };
-
 template <>
 struct TileOps<Q6K> {
     static constexpr int kPieces = 14;
     static constexpr int kRows = 16;
-    static constexpr float kSumScale = 32.f / 16777216.f;   // 32 S in the units of the code sums
-    __device__ static __forceinline__ int slot(int r) {
-        const int h = r >> 4, part = (r >> 2) & 3, ih = (r >> 1) & 1, u = r & 1;
-        return (2 * h + ih) * 8 + u * 4 + part;
-    }
-    using Sums = f32x4;
-    __device__ static __forceinline__ Sums sums(const float* sx, int b, int g) {
-        return *reinterpret_cast<const f32x4*>(sx + b * 16 + 4 * g);
-    }
-    __device__ static __forceinline__ float dot(const Q6K::Frag& f, int g, u32x4 a0, u32x4 a1, Sums s) {
-#pragma clang fp contract(off)
-        u32x4 c[4][2];   // part, half of its 16 codes
-#pragma unroll
-        for (int t = 0; t < 4; ++t) {
-            uint32_t a[4], b[4];
-            Q6K::codes(f, t, a, b);
-#pragma unroll
-            for (int p = 0; p < 4; ++p) {
-                c[p][t >> 1][2 * (t & 1)] = a[p];
-                c[p][t >> 1][2 * (t & 1) + 1] = b[p];
-            }
-        }
-        const f32x4 z = {0.f, 0.f, 0.f, 0.f};
-        f32x4 d[4];
-#pragma unroll
-        for (int p = 0; p < 4; ++p) d[p] = mfma32(a0, c[p][0], z);
-#pragma unroll
-        for (int p = 0; p < 4; ++p) d[p] = mfma32(a1, c[p][1], d[p]);
-        float sc[4];
-        Q6K::scales(f, g, sc);
-        // d sum_p sc_p (P_p - 32 S_p), in units of 2^-24
-        float p = sc[0] * (d[0][0] - s.x);
-        p = fmaf(sc[1], d[1][1] - s.y, p);
-        p = fmaf(sc[2], d[2][2] - s.z, p);
-        p = fmaf(sc[3], d[3][3] - s.w, p);
-        return h2f((uint16_t)f.dbits) * 16777216.0f * p;
-    }
 };
 
 // A tile launch of type QT: tiles of kRows rows (columns past them repeat the
@@ -848,13 +764,12 @@ struct TileShape {
     static constexpr int kCopies = (kRows * kPieces + kWave - 1) / kWave;
     static constexpr int kDepth = 2;   // slots per wave; a third measured no faster
     static constexpr int kSlot = kCopies * kWave * 16;
-    // LDS: x operands, x sums, norm scratch, zeros, the class sums of two
-    // tiles, the rings
+    // LDS: x operands, x sums, norm scratch, the residue sums of two tiles,
+    // the rings
     __host__ __device__ static constexpr int sums(int nb) { return nb * kQK * 2; }
     __host__ __device__ static constexpr int red(int nb) { return sums(nb) + nb * QT::kSxPerBlock * 4; }
-    __host__ __device__ static constexpr int zero(int nb) { return red(nb) + 16; }
-    __host__ __device__ static constexpr int part(int nb) { return zero(nb) + kZeroBytes; }
-    __host__ __device__ static constexpr int ring(int nb) { return part(nb) + 2 * kMats * kTileWaves * kTileCols * 4; }
+    __host__ __device__ static constexpr int part(int nb) { return red(nb) + 16; }
+    __host__ __device__ static constexpr int ring(int nb) { return part(nb) + 2 * kMats * kResidues * kTileCols * 4; }
     __host__ __device__ static constexpr int bytes(int nb) { return ring(nb) + kTileWaves * kDepth * kSlot; }
 };
 
@@ -874,8 +789,7 @@ template <class SH, int kNormIters, class TileOf, class Finish>
 __device__ __forceinline__ void tile_rows(const uint16_t* __restrict__ x, int nb, uint8_t* smem, int wg, int wgs,
                                           int tiles, const NormIn& nrm, TileOf tile_of, Finish finish) {
     using QT = typename SH::Q;
-    using OP = TileOps<QT>;
-    constexpr int kPieces = OP::kPieces, kCopies = SH::kCopies, kDepth = SH::kDepth, kMats = SH::kMats;
+    constexpr int kPieces = TileOps<QT>::kPieces, kCopies = SH::kCopies, kDepth = SH::kDepth, kMats = SH::kMats;
     uint32_t* xp = reinterpret_cast<uint32_t*>(smem);
     float* sx = reinterpret_cast<float*>(smem + SH::sums(nb));
     float* red = reinterpret_cast<float*>(smem + SH::red(nb));
@@ -886,6 +800,9 @@ __device__ __forceinline__ void tile_rows(const uint16_t* __restrict__ x, int nb
     const int n = lane & 15, g = lane >> 4;
     uint8_t* ring = smem + SH::ring(nb) + wave * kDepth * SH::kSlot;
     const int row_bytes = nb * QT::kBytes;
+    // Where the streaming kernels have no instantiation, a row's residues start
+    // at lane (row % 4) nb % 16: the flat walk's, whose waves list four rows.
+    const int turn = flat_order(nb) ? nb & (kResidues - 1) : 0;
     int my_tiles = 0;   // at least one: wg < wgs <= tiles
     for (int t = wg; t < tiles; t += wgs) ++my_tiles;
     const int total = my_tiles * kMats * nb;
@@ -992,12 +909,6 @@ __device__ __forceinline__ void tile_rows(const uint16_t* __restrict__ x, int nb
         __builtin_amdgcn_sched_barrier(0);
     }
     int issued = kDepth;
-    if ((int)threadIdx.x < kZeroBytes / 4) reinterpret_cast<uint32_t*>(smem + SH::zero(nb))[threadIdx.x] = 0u;
-
-    auto put = [&](u32x4 v, int r) {
-        *reinterpret_cast<u32x4*>(xp + (size_t)((r & ~31) + OP::slot(r & 31)) * 4) = permute_x8(v);
-        stage_sums8<QT::kSumLayout>(v, r, sx, OP::kSumScale);
-    };
     if constexpr (kNormIters != 0) {
         if (wave < kWavesPerBlock) {
             // the order of norm_block_sum's callers (256 threads)
@@ -1024,56 +935,42 @@ __device__ __forceinline__ void tile_rows(const uint16_t* __restrict__ x, int nb
 #pragma unroll
             for (int i = 0; i < kIters; ++i) {
                 const int r = i * kBlock + (int)threadIdx.x;
-                if (r < runs) put(norm_run(raw[i], wr[i], inv), r);
+                if (r < runs) stage_x8<QT::kSumLayout>(norm_run(raw[i], wr[i], inv), r, xp, sx);
             }
         } else {
             lds_only_barrier();
         }
     } else {
-        // this wave's runs are in LDS once only the ring copies are in flight
-        // (a wave's 64 runs are two whole super-blocks, permuted in place:
-        // every lane has read before any lane writes)
+        // this wave's runs are in LDS once only the ring copies are in flight;
+        // each is permuted in place
         wait_vm<kDepth * kCopies>();
-        for (int r0 = wave * kWave; r0 < runs; r0 += kTileBlock) {
-            const int r = r0 + lane;
-            u32x4 v = {0u, 0u, 0u, 0u};
-            if (r < runs) v = *reinterpret_cast<const u32x4*>(xp + (size_t)r * 4);
-            wait_lds();
-            __builtin_amdgcn_wave_barrier();
-            if (r < runs) put(v, r);
-        }
+        for (int r = wave * kWave + lane; r < runs; r += kTileBlock)
+            stage_x8<QT::kSumLayout>(*reinterpret_cast<const u32x4*>(xp + (size_t)r * 4), r, xp, sx);
     }
     lds_only_barrier();
 
-    // A operand address: slot lane & 3 of this lane group's quarter, or zeros
-    const bool a_live = ((lane & 15) >> 2) == g;
-    const int a_off = a_live ? g * 128 + (lane & 3) * 16 : SH::zero(nb);
-    const int a_mask = a_live ? -1 : 0;
     Walk cur = first();
     int done = 0, slot = 0;
     for (int k = 0; k < my_tiles; ++k) {
         const TileAt t = tile_of(wg + k * wgs);
         const int col = min(n, t.rows - 1);
-        float* pt = part + (k & 1) * kMats * kTileWaves * kTileCols;
+        float* pt = part + (k & 1) * kMats * kResidues * kTileCols;
 #pragma unroll
         for (int m = 0; m < kMats; ++m) {
             if (done >= my_steps || cur.u != k * kMats + m) continue;   // wave-uniform
             // low address bits of the lane's row (a Q6_K block's offset in its first piece)
             const uint32_t row_at = QT::kBytes % 16 ? (uint32_t)(uintptr_t)t.w[m] + (uint32_t)(t.row + col) * (uint32_t)row_bytes : 0u;
-            const int cls = cur.b;
-            float acc = 0.f;
+            const int res = cur.b;   // 0..7: this wave's blocks have the residues res and res + 8, in turn
+            float even = 0.f, odd = 0.f;
             do {
                 const int b = cur.b;
+                const typename QT::XRegs xr = QT::xload(xp, sx, g, b);
                 const int later = issued - done - 1;   // steps in flight behind this one
                 if (later >= kDepth - 1) wait_vm<(kDepth - 1) * kCopies>();
                 else wait_vm<0>();
                 const uint8_t* sb = ring + slot * SH::kSlot + col * kPieces * 16;
                 if (QT::kBytes % 16) sb += (row_at + (uint32_t)(b * QT::kBytes)) & 15u;
                 const typename QT::Frag f = QT::load(sb, g);
-                const int a_at = ((b * kQK * 2) & a_mask) | a_off;
-                const u32x4 a0 = *reinterpret_cast<const u32x4*>(smem + a_at);
-                const u32x4 a1 = *reinterpret_cast<const u32x4*>(smem + a_at + 64);
-                const typename OP::Sums xs = OP::sums(sx, b, g);
                 wait_lds();
                 __builtin_amdgcn_sched_barrier(0);
                 if (issued < my_steps) {   // the slot is read: refill it
@@ -1082,23 +979,35 @@ __device__ __forceinline__ void tile_rows(const uint16_t* __restrict__ x, int nb
                     ++issued;
                 }
                 __builtin_amdgcn_sched_barrier(0);
-                acc += OP::dot(f, g, a0, a1, xs);
+                const float c = QT::dot(f, g, xr);
+                if ((b & 8) == 0) even += c;   // wave-uniform
+                else odd += c;
                 slot = slot + 1 == kDepth ? 0 : slot + 1;
                 ++done;
                 advance(cur);
             } while (done < my_steps && cur.u == k * kMats + m);
-            acc = sum32(sum16(acc));   // the row's four quarters
-            if (g == 0) pt[(m * kTileWaves + cls) * kTileCols + n] = acc;
+            even = sum32(sum16(even));   // the row's four quarters
+            odd = sum32(sum16(odd));
+            if (g == 0) {
+                pt[(m * kResidues + res) * kTileCols + n] = even;
+                pt[(m * kResidues + res + 8) * kTileCols + n] = odd;
+            }
         }
-        lds_only_barrier();   // the tile's class sums are in LDS
+        lds_only_barrier();   // the tile's residue sums are in LDS
         if (wave == (k & (kTileWaves - 1))) {
+            // lane group g: residues of the streaming lanes 4g .. 4g + 3
+            const int rot = ((t.row + n) & 3) * turn;
             float sum[kMats];
 #pragma unroll
             for (int m = 0; m < kMats; ++m) {
-                // classes g and g + 4 of the row, then the lane groups
-                const float* c = pt + m * kTileWaves * kTileCols + n;
-                const float v0 = g < nb ? c[g * kTileCols] : 0.f, v1 = g + 4 < nb ? c[(g + 4) * kTileCols] : 0.f;
-                sum[m] = sum32(sum16(v0 + v1));
+                const float* c = pt + m * kResidues * kTileCols + n;
+                float v[4];
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    const int res = (4 * g + i - rot) & (kResidues - 1);
+                    v[i] = res < nb ? c[res * kTileCols] : 0.f;
+                }
+                sum[m] = sum32(sum16((v[0] + v[3]) + (v[2] + v[1])));
             }
             if (g == 0 && n < t.rows) finish(t, t.row + n, sum);
         }
@@ -1226,15 +1135,10 @@ void launch_rows_once(const RowSet& rs, const uint16_t* x, size_t lds, const Nor
 // Super-block counts whose Q4_K / Q6_K rows go through the tile kernels: 20
 // (hidden 5120) and every count without a streaming instantiation.  Measured
 // against the streaming kernels (us, streaming -> tile, back-to-back launches
-// over rotated weights): 20 blocks Q4_K 5120 rows 7.6 -> 5.8, gate/up with the
-// norm 2 x 17408 24.2 -> 19.9 and 2 x 25600 30.4 -> 29.0, grouped q/k/v 9.9 ->
-// 10.3; against the flat walk over super-blocks that served other counts:
-// Q4_K 18944 x 3584 13.2 -> 10.2, 3584 x 3584 5.4 -> 4.1, 512 x 3584 4.6 ->
-// 3.4, Q6_K 3584 x 18944 22.6 -> 14.4.  The streaming kernels stay where they
-// were faster: 10 blocks (grouped q/k/v 6.1 against 8.1, though gate/up 9.7
-// against 8.8), 12 and 24 (Q6_K 1024 rows 3.2 against 4.7, 2048 rows 5.4
-// against 6.9), 38 (8.8 against 9.0), 68 and 100 (5120 rows 18.1 against 22.2
-// and 24.9 against 31: 320 tiles on 256 CUs).
+// over rotated weights): 20 blocks Q4_K 5120 rows 8.0 -> 6.8, gate/up with the
+// norm 2 x 17408 24.3 -> 21.3; against the flat walk over super-blocks that
+// served other counts: Q4_K 3584 x 3584 5.7 -> 4.8, 512 x 3584 5.0 -> 4.1,
+// 3584 x 18432 17.0 -> 10.5, Q6_K 3584 x 18432 21.9 -> 14.8.
 __host__ __device__ constexpr bool tile_length(int nb) {
     switch (nb) {
         case 4: case 8: case 10: case 12: case 16: case 24: case 32: case 38: case 48: case 64: case 68: case 100: return false;

@@ -217,3 +217,34 @@ def test_tile_rows_match_oracle(hip, orc, kind, k):
         # the fp16 form stores the same sums, rounded
         hip.device.matvec(kind, dw.at(off), dx, dy, k, n)
         assert np.array_equal(dy.download(np.uint16, n), got[:n].astype(np.float16).view(np.uint16))
+
+
+@pytest.mark.parametrize("kind", ["q4k", "q6k"])
+@pytest.mark.parametrize("nb", [1, 3, 9, 14, 17, 20, 28, 47])
+@pytest.mark.parametrize("n", [37, 9001])
+def test_every_length_sums_in_the_streaming_order(hip, kind, nb, n):
+    """A row's bits do not depend on the kernel that its length and the number
+    of rows choose: they are those of the streaming kernel of 16, 32, 48 or 64
+    blocks on the row padded with zero blocks.  Lengths without a streaming
+    instantiation keep the order of a walk over four rows in turn, in which
+    block b of row r falls to the lane of block (r % 4) nb + b: the same
+    number of zero blocks goes before the row."""
+    k = nb * 256
+    w, x = _inputs(hip, kind, n, k, seed=nb + n)
+    rows = w.reshape(n, -1)
+    dy = hip.DeviceArray(n * 4)
+    print(f"[sum order] {kind} {n} x {k}", flush=True)
+    hip.device.matvec(kind, hip.DeviceArray.from_numpy(w), hip.DeviceArray.from_numpy(x), dy, k, n, f32_out=True)
+    got = dy.download(np.float32, n)
+    per = rows.shape[1] // nb
+    for r in range(4):
+        before = 0 if nb == 20 else r * nb % 16
+        wide = -(-(before + nb) // 16) * 16
+        part = rows[r::4][:256]
+        wp = np.zeros((len(part), wide * per), np.uint8)
+        wp[:, before * per:(before + nb) * per] = part
+        xp = np.zeros(wide * 256, np.uint16)
+        xp[before * 256:before * 256 + k] = x
+        hip.device.matvec(kind, hip.DeviceArray.from_numpy(wp), hip.DeviceArray.from_numpy(xp), dy, wide * 256,
+                          len(part), f32_out=True)
+        np.testing.assert_array_equal(got[r::4][:256], dy.download(np.float32, len(part)))
