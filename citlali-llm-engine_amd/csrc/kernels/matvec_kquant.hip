@@ -39,6 +39,7 @@ constexpr int kWavesPerBlock = kBlock / kWave;
 constexpr int kSum32 = 0;     // Q4K: sum over each 32-value group, [b][g]
 constexpr int kSumQ6 = 1;     // Q6K: 16-value slices, [b][h][ih][k]
 constexpr int kPlain = 2;     // F16: x in its own order, no sums
+constexpr int kBatch = 4;        // wave steps of the flat walk whose loads are issued together
 // The streaming kernels run two workgroups per CU (two waves per SIMD):
 // their register budget is capped to keep both resident.
 constexpr int kWavesPerSimd = 2;
@@ -167,6 +168,17 @@ struct XStage {
         lds_barrier();
     }
 };
+
+// Any K (a multiple of 256): every thread stages runs v8 = tid, tid + 256, ...
+// (a multiple of 4 runs per thread keeps each group's runs on consecutive
+// threads of one pass).
+template <int kLayout>
+__device__ __forceinline__ void stage_x(const uint16_t* __restrict__ x, int K, uint32_t* xp, float* sx) {
+    const int n8 = K >> 3;
+    for (int v8 = threadIdx.x; v8 < n8; v8 += kBlock)
+        stage_x8<kLayout>(*reinterpret_cast<const u32x4*>(x + (size_t)v8 * 8), v8, xp, sx);
+    lds_barrier();
+}
 
 // ---------------------------------------------------------------------------
 // Q4_K: d(f16) dmin(f16) scales[12] qs[128]   (weight_loader.cpp:150-161)
@@ -705,9 +717,62 @@ __global__ __launch_bounds__(kGateUpBlock, 2) void matvec_gate_up_kernel(const u
     }
 }
 
+// Any super-block count, for the launches too small for the tile kernels below
+// (tile_wins): a wave owns kRows rows and walks their super-blocks as one flat
+// list; a lane's row is found by multiply-high division.
+template <class QT, bool kF32, int kRows>
+__global__ __launch_bounds__(kBlock) void matvec_flat_kernel(const uint8_t* __restrict__ w,
+                                                             const uint16_t* __restrict__ x,
+                                                             void* __restrict__ y, int K, int N,
+                                                             uint64_t magic) {
+    extern __shared__ __align__(16) uint8_t smem[];
+    uint32_t* xp = reinterpret_cast<uint32_t*>(smem);
+    float* sx = reinterpret_cast<float*>(smem + (size_t)K * 2);
+    stage_x<QT::kSumLayout>(x, K, xp, sx);
+
+    const int lane = threadIdx.x & (kWave - 1);
+    const int wave = threadIdx.x / kWave;
+    const int l4 = lane % QT::kLanesPerSb;
+    const int sub = lane / QT::kLanesPerSb;
+    const int nb = K >> 8;
+    const int row0 = (blockIdx.x * kWavesPerBlock + wave) * kRows;
+    const int rows = min(kRows, N - row0);
+    const int nflat = rows > 0 ? rows * nb : 0;
+
+    float acc[kRows];
+#pragma unroll
+    for (int k = 0; k < kRows; ++k) acc[k] = 0.f;
+
+    for (int f0 = 0; f0 < nflat; f0 += kBatch * QT::kSbPerStep) {
+        typename QT::Frag fr[kBatch];
+        int rl[kBatch], bl[kBatch];
+#pragma unroll
+        for (int u = 0; u < kBatch; ++u) {
+            const uint32_t f = (uint32_t)(f0 + u * QT::kSbPerStep + sub);
+            const uint32_t r = (uint32_t)(((uint64_t)f * magic) >> 32);
+            rl[u] = (int)f < nflat ? (int)r : -1;
+            bl[u] = (int)(f - r * (uint32_t)nb);
+            if (rl[u] >= 0) fr[u] = QT::load(w + ((size_t)row0 * nb + f) * QT::kBytes, l4);
+        }
+#pragma unroll
+        for (int u = 0; u < kBatch; ++u) {
+            if (rl[u] >= 0) {
+                const float c = QT::dot(fr[u], l4, xp, sx, bl[u]);
+#pragma unroll
+                for (int k = 0; k < kRows; ++k) acc[k] += (rl[u] == k) ? c : 0.f;
+            }
+        }
+    }
+#pragma unroll
+    for (int k = 0; k < kRows; ++k) {
+        const float s = wave_sum(acc[k]);
+        if (lane == 0 && k < rows) store_y<kF32>(y, row0 + k, s);
+    }
+}
+
 // ---------------------------------------------------------------------------
 // Tile kernels: Q4_K / Q6_K rows of any super-block count nb, for the counts
-// that do not fill the wave steps of the streaming kernels (see tile_length).
+// that do not fill the wave steps of the streaming kernels (see tile_wins).
 //
 // A tile is up to 16 rows; a wave's step is one super-block of each of them,
 // lane (row n = lane % 16, quarter g = lane / 16) holding the 64 codes that
@@ -732,9 +797,14 @@ constexpr int kTileCols = 16;
 constexpr int kTileWaves = 8;
 constexpr int kTileBlock = kTileWaves * kWave;
 constexpr int kResidues = 16;   // QT::kSbPerStep
-// tile lengths whose rows are summed in the flat walk's order (every one
-// without a streaming instantiation)
-__host__ __device__ constexpr bool flat_order(int nb) { return nb != 20; }
+// super-block counts with a streaming instantiation; rows of the others are
+// summed in the flat walk's order
+__host__ __device__ constexpr bool streaming_length(int nb) {
+    switch (nb) {
+        case 4: case 8: case 10: case 12: case 16: case 20: case 24: case 32: case 38: case 48: case 64: case 68: case 100: return true;
+        default: return false;
+    }
+}
 
 template <class QT>
 struct TileOps;
@@ -752,10 +822,10 @@ struct TileOps<Q6K> {
 // A tile launch of type QT: tiles of kRows rows (columns past them repeat the
 // last one and are not stored), ring slots of kCopies copy instructions of 64
 // pieces.  Q4_K: 14 rows fill two copies (126 pieces); 16 rows in three
-// measured 6.39 against 5.51 us at 5120 x 5120 and 21.7 against 20.6 us for
-// gate/up 17408 x 5120.  Q6_K: 16 rows in four copies; 13 rows in three, 23.3
-// against 14.6 us at 3584 x 18944 (276 tiles on 256 CUs) and 81 against 69 us
-// at 151936 x 2560.
+// measured 7.5 against 7.2 us at 5120 x 5120 and 21.8 against 20.6 us for
+// gate/up 17408 x 5120 (but 15.1 against 16.4 us at 20011 x 5120 with the
+// norm).  Q6_K: 16 rows in four copies; 13 rows in three, 23.0 against 14.6 us
+// at 3584 x 18432 (276 tiles on 256 CUs) and 61 against 53 us at 60000 x 5120.
 template <class QT, int kMatrices>
 struct TileShape {
     using Q = QT;
@@ -802,7 +872,7 @@ __device__ __forceinline__ void tile_rows(const uint16_t* __restrict__ x, int nb
     const int row_bytes = nb * QT::kBytes;
     // Where the streaming kernels have no instantiation, a row's residues start
     // at lane (row % 4) nb % 16: the flat walk's, whose waves list four rows.
-    const int turn = flat_order(nb) ? nb & (kResidues - 1) : 0;
+    const int turn = streaming_length(nb) ? 0 : nb & (kResidues - 1);
     int my_tiles = 0;   // at least one: wg < wgs <= tiles
     for (int t = wg; t < tiles; t += wgs) ++my_tiles;
     const int total = my_tiles * kMats * nb;
@@ -1068,21 +1138,6 @@ __global__ __launch_bounds__(kTileBlock, 4) void matvec_tile_kernel(TileSet ts, 
     tile_set<SH, kNormIters>(ts, x, nb, f32, smem, blockIdx.x, gridDim.x, nrm);
 }
 
-// Q4_K tiles on blocks [0, blocks_a), Q6_K tiles on the rest.
-template <class SA, class SB, int kNormIters>
-__global__ __launch_bounds__(kTileBlock, 4) void matvec_tile_group_kernel(TileSet a, TileSet b, int blocks_a,
-                                                                          const uint16_t* __restrict__ x, int nb,
-                                                                          NormIn nrm) {
-    extern __shared__ __align__(16) uint8_t smem[];
-    if ((int)blockIdx.x < blocks_a) {
-        tile_set<SA, kNormIters>(a, x, nb, 0, smem, blockIdx.x, blocks_a, nrm);
-    } else {
-        NormIn no_sum = nrm;   // the Q4_K blocks store the residual sum
-        no_sum.xs_out = nullptr;
-        tile_set<SB, kNormIters>(b, x, nb, 0, smem, blockIdx.x - blocks_a, gridDim.x - blocks_a, no_sum);
-    }
-}
-
 // ffn_gate, ffn_up and SwiGLU: a tile's steps run over both matrices.
 template <class SH, int kNormIters>
 __global__ __launch_bounds__(kTileBlock, 4) void matvec_tile_gate_up_kernel(const uint8_t* __restrict__ wg,
@@ -1132,18 +1187,31 @@ void launch_rows_once(const RowSet& rs, const uint16_t* x, size_t lds, const Nor
                   stream, rs, x, K, nrm);
 }
 
-// Super-block counts whose Q4_K / Q6_K rows go through the tile kernels: 20
-// (hidden 5120) and every count without a streaming instantiation.  Measured
-// against the streaming kernels (us, streaming -> tile, back-to-back launches
-// over rotated weights): 20 blocks Q4_K 5120 rows 8.0 -> 6.8, gate/up with the
-// norm 2 x 17408 24.3 -> 21.3; against the flat walk over super-blocks that
-// served other counts: Q4_K 3584 x 3584 5.7 -> 4.8, 512 x 3584 5.0 -> 4.1,
-// 3584 x 18432 17.0 -> 10.5, Q6_K 3584 x 18432 21.9 -> 14.8.
-__host__ __device__ constexpr bool tile_length(int nb) {
-    switch (nb) {
-        case 4: case 8: case 10: case 12: case 16: case 24: case 32: case 38: case 48: case 64: case 68: case 100: return false;
-        default: return true;
-    }
+// Whether `rows` rows of nb super-blocks go through the tile kernels.  The
+// bits of a row are the same either way, so the line lies where the time says
+// (us, back-to-back launches over rotated weights, other kernel / tile):
+//  * 20 blocks (hidden 5120), against the streaming kernels, which waste 12 of
+//    32 block slots but start sooner: Q4_K 1024 rows 4.2 / 4.6, 2048 rows 4.9 /
+//    4.6, 5120 rows 8.0 / 6.8; with the norm, in which every workgroup adds the
+//    residual and norms, 5120 rows 8.1 / 9.2, three matrices of 7168 rows 11.2 /
+//    9.8, 20011 rows 21.3 / 16.1, gate/up 2 x 17408 24.3 / 21.3; Q6_K
+//    2048 rows 6.0 / 6.6, 5120 rows 9.7 / 11.1, 12000 rows 17.3 / 14.8, gate/up
+//    with the norm 2 x 1000 9.4 / 10.1, 2 x 17408 42.1 / 34.4.  Launches of both
+//    types stay streaming (q/k/v of 5120, 1024 and 1024 rows with the norm 10.6
+//    / 11.3);
+//  * counts without a streaming instantiation, against the flat walk, whose
+//    x staging per 16 rows costs little for short rows: Q4_K 12000 x 768 4.2 /
+//    5.1, 5120 x 2304 5.8 / 4.9, 12000 x 1280 5.3 / 5.9, 40000 x 1536 12.1 / 12.7,
+//    12000 x 3584 9.6 / 9.1, 512 x 3584 5.0 / 4.1, 3584 x 18432 17.0 / 10.5; Q6_K
+//    12000 x 768 4.6 / 5.9, 3584 x 3584 6.5 / 6.6, 40000 x 1280 17.9 / 15.8, 512 x
+//    4352 5.9 / 5.1, 3584 x 18432 21.9 / 14.8.
+// The other streaming lengths stay with the streaming kernels.
+template <class QT>
+bool tile_wins(int nb, int rows, bool norm = false) {
+    constexpr bool q4 = std::is_same<QT, Q4K>::value;
+    if (nb == 20) return rows >= (!q4 ? 8192 : norm ? 6144 : 1536);
+    if (streaming_length(nb)) return false;
+    return q4 ? nb >= 12 || (nb >= 5 && rows < 8192) : nb > 16 || rows >= 32768;
 }
 
 // Two workgroups per CU where the LDS of two fits, never more than tiles.
@@ -1169,28 +1237,6 @@ hipError_t launch_tile(int nb, const RowSet& rs, const uint16_t* x, bool f32, co
         if (e != hipSuccess) return e;
         launch_kernel(kernel, dim3(tile_grid(ts.end[2], lds)), dim3(kTileBlock), (size_t)lds, stream, ts, x, nb,
                       (int)f32, nrm);
-        return hipGetLastError();
-    });
-}
-
-template <bool kNorm>
-hipError_t launch_tile_mixed(int nb, const RowSet& a, const RowSet& b, const uint16_t* x, const NormIn& nrm,
-                             hipStream_t stream) {
-    using SA = TileShape<Q4K, 1>;
-    using SB = TileShape<Q6K, 1>;
-    const TileSet ta = make_tile_set<Q4K>(a), tb = make_tile_set<Q6K>(b);
-    const int lds = std::max(SA::bytes(nb), SB::bytes(nb));
-    const int grid = std::max(2, tile_grid(ta.end[2] + tb.end[2], lds));
-    // blocks split in proportion to the bytes each set streams
-    const double wa = (double)a.end[2] * Q4K::kBytes, wb = (double)b.end[2] * Q6K::kBytes;
-    int ga = (int)(grid * wa / (wa + wb) + 0.5);
-    ga = std::max(1, std::min(ga, std::min(grid - 1, ta.end[2])));
-    const int gb = std::max(1, std::min(grid - ga, tb.end[2]));
-    return with_norm_iters<kNorm>(nb, [&](auto it) {
-        constexpr auto kernel = matvec_tile_group_kernel<SA, SB, decltype(it)::value>;
-        const hipError_t e = allow_lds<kernel>(lds);
-        if (e != hipSuccess) return e;
-        launch_kernel(kernel, dim3(ga + gb), dim3(kTileBlock), (size_t)lds, stream, ta, tb, ga, x, nb, nrm);
         return hipGetLastError();
     });
 }
@@ -1259,23 +1305,18 @@ bool launch_stream_for(int nb, const RowSet& rs, const uint16_t* x, size_t lds, 
         case 64: launch_stream<QT, kF32, 4, 1, kSegs, kNorm>(rs, x, lds, nrm, stream); return true;
         // the other Qwen3 row lengths: hidden 1024 / 2048 / 2560 / 5120, FFN
         // 3072 / 6144 / 9728 / 17408 / 25600 (the last two without the norm
-        // prologue, which only hidden-sized inputs take); 20 blocks here only
-        // as fp16 (Q4_K / Q6_K: the tile kernels), 68 and 100 only quantized
-        // (fp16: 32 registers of weights per step in flight)
+        // prologue, which only hidden-sized inputs take, and only quantized:
+        // an fp16 step has 32 registers of weights in flight)
         case 4: launch_partial<QT, kF32, kSegs, kNorm, 4>(rs, x, lds, nrm, stream); return true;
         case 8: launch_partial<QT, kF32, kSegs, kNorm, 8>(rs, x, lds, nrm, stream); return true;
         case 10: launch_partial<QT, kF32, kSegs, kNorm, 10>(rs, x, lds, nrm, stream); return true;
         case 12: launch_partial<QT, kF32, kSegs, kNorm, 12>(rs, x, lds, nrm, stream); return true;
+        case 20: launch_partial<QT, kF32, kSegs, kNorm, 20>(rs, x, lds, nrm, stream); return true;
         case 24: launch_partial<QT, kF32, kSegs, kNorm, 24>(rs, x, lds, nrm, stream); return true;
         case 38: launch_partial<QT, kF32, kSegs, kNorm, 38>(rs, x, lds, nrm, stream); return true;
         default: break;
     }
-    if constexpr (std::is_same<QT, F16>::value) {
-        if (nb == 20) {
-            launch_partial<QT, kF32, kSegs, kNorm, 20>(rs, x, lds, nrm, stream);
-            return true;
-        }
-    } else if constexpr (!kNorm) {
+    if constexpr (!std::is_same<QT, F16>::value && !kNorm) {
         switch (nb) {
             case 68: launch_partial<QT, kF32, kSegs, kNorm, 68>(rs, x, lds, nrm, stream); return true;
             case 100: launch_partial<QT, kF32, kSegs, kNorm, 100>(rs, x, lds, nrm, stream); return true;
@@ -1297,12 +1338,22 @@ template <class QT, bool kF32>
 hipError_t launch_matvec(const uint8_t* w, const uint16_t* x, void* y, int K, int N, hipStream_t stream) {
     const int nb = K / kQK;
     const RowSet rs{{w, w, w}, {y, y, y}, {N, N, N}};
-    if constexpr (!std::is_same<QT, F16>::value) {
-        if (tile_length(nb)) return launch_tile<QT, false>(nb, rs, x, kF32, kNoNorm, stream);
-    }
     const size_t lds = lds_bytes<QT>(K);
+    if constexpr (!std::is_same<QT, F16>::value) {
+        if (tile_wins<QT>(nb, N)) return launch_tile<QT, false>(nb, rs, x, kF32, kNoNorm, stream);
+        if (!streaming_length(nb)) {
+            constexpr int kRows = 4;
+            // floor(f / nb) == (f * magic) >> 32 for every f < 2^20 (nb <= 112)
+            const uint64_t magic = ((uint64_t)1 << 32) / (uint64_t)nb + 1u;
+            const int rows_per_block = kRows * kWavesPerBlock;
+            const int grid = (N + rows_per_block - 1) / rows_per_block;
+            launch_kernel((matvec_flat_kernel<QT, kF32, kRows>), dim3(grid), dim3(kBlock), lds, stream, w, x, y, K,
+                          N, magic);
+            return hipGetLastError();
+        }
+    }
     if (!launch_stream_for<QT, kF32, 1>(nb, rs, x, lds, kNoNorm, stream)) {
-        // fp16 rows of any other length (Q4_K / Q6_K: tile_length)
+        // fp16 rows of any other length
         if constexpr (std::is_same<QT, F16>::value)
             return launch_matvec_f16_rows(reinterpret_cast<const uint16_t*>(w), x, y, kF32, K, N, stream);
         return hipErrorInvalidValue;
@@ -1316,7 +1367,7 @@ hipError_t launch_matvec_prologue(const uint8_t* w, const uint16_t* x, const Nor
     const RowSet rs{{w, w, w}, {y, y, y}, {N, N, N}};
     const int nb = K / kQK;
     if constexpr (!std::is_same<QT, F16>::value) {
-        if (tile_length(nb)) return launch_tile<QT, true>(nb, rs, x, kF32, nrm, stream);
+        if (tile_wins<QT>(nb, N, true)) return launch_tile<QT, true>(nb, rs, x, kF32, nrm, stream);
     }
     if (!launch_stream_for<QT, kF32, 1, true>(nb, rs, x, lds_bytes<QT>(K), nrm, stream))
         return hipErrorInvalidValue;
@@ -1355,11 +1406,8 @@ void launch_group_mixed(const RowSet& a, const RowSet& b, const uint16_t* x, int
 template <bool kNorm>
 hipError_t launch_group(int nb, RowSet (&set)[2], const int (&cnt)[2], bool f16, const uint16_t* x, int K,
                         const NormIn& nrm, hipStream_t s) {
-    if (!f16 && tile_length(nb)) {
-        if (cnt[1] == 0) return launch_tile<Q4K, kNorm>(nb, set[0], x, false, nrm, s);
-        if (cnt[0] == 0) return launch_tile<Q6K, kNorm>(nb, set[1], x, false, nrm, s);
-        return launch_tile_mixed<kNorm>(nb, set[0], set[1], x, nrm, s);
-    }
+    if (!f16 && cnt[1] == 0 && tile_wins<Q4K>(nb, set[0].end[2], kNorm)) return launch_tile<Q4K, kNorm>(nb, set[0], x, false, nrm, s);
+    if (!f16 && cnt[0] == 0 && tile_wins<Q6K>(nb, set[1].end[2], kNorm)) return launch_tile<Q6K, kNorm>(nb, set[1], x, false, nrm, s);
     bool ok = true;
     if (f16) ok = launch_stream_for<F16, false, 3, kNorm>(nb, set[0], x, lds_bytes<F16>(K), nrm, s);
     else if (cnt[1] == 0) ok = launch_stream_for<Q4K, false, 3, kNorm>(nb, set[0], x, lds_bytes<Q4K>(K), nrm, s);
@@ -1374,6 +1422,7 @@ hipError_t launch_group(int nb, RowSet (&set)[2], const int (&cnt)[2], bool f16,
             case 8: launch_group_mixed<1, 1, kNorm, 8>(set[0], set[1], x, K, nrm, s); break;
             case 10: launch_group_mixed<1, 1, kNorm, 10>(set[0], set[1], x, K, nrm, s); break;
             case 12: launch_group_mixed<1, 1, kNorm, 12>(set[0], set[1], x, K, nrm, s); break;
+            case 20: launch_group_mixed<2, 1, kNorm, 20>(set[0], set[1], x, K, nrm, s); break;
             case 24: launch_group_mixed<2, 1, kNorm, 24>(set[0], set[1], x, K, nrm, s); break;
             case 38: launch_group_mixed<3, 1, kNorm, 38>(set[0], set[1], x, K, nrm, s); break;
             default: ok = false;
@@ -1386,7 +1435,7 @@ hipError_t launch_gate_up_t(const uint8_t* wg, const uint8_t* wu, const uint16_t
                           const NormIn& nrm, hipStream_t stream) {
     const int nb = K / kQK;
     if constexpr (!std::is_same<QT, F16>::value) {
-        if (tile_length(nb)) return launch_tile_gate_up<QT, kNorm>(wg, wu, x, act, nb, N, nrm, stream);
+        if (tile_wins<QT>(nb, 2 * N, kNorm)) return launch_tile_gate_up<QT, kNorm>(wg, wu, x, act, nb, N, nrm, stream);
     }
     const size_t lds = lds_bytes<QT>(K) + sizeof(int);   // + the unit counter
     int grid = device_cus();
@@ -1399,17 +1448,12 @@ hipError_t launch_gate_up_t(const uint8_t* wg, const uint8_t* wu, const uint16_t
         case 16: launch_kernel((matvec_gate_up_kernel<QT, 1, kNorm>), g, b, lds, stream, wg, wu, x, act, K, N, nrm); break;
         case 32: launch_kernel((matvec_gate_up_kernel<QT, 2, kNorm>), g, b, lds, stream, wg, wu, x, act, K, N, nrm); break;
         // rows shorter than one wave step (Qwen3-0.6B: hidden 1024; 1.7B: 2048;
-        // 4B: 2560), and hidden 5120 (Qwen3-14B / 32B) as fp16
+        // 4B: 2560), and hidden 5120 (Qwen3-14B / 32B)
         case 4: launch_kernel((matvec_gate_up_kernel<QT, 1, kNorm, 4>), g, b, lds, stream, wg, wu, x, act, K, N, nrm); break;
         case 8: launch_kernel((matvec_gate_up_kernel<QT, 1, kNorm, 8>), g, b, lds, stream, wg, wu, x, act, K, N, nrm); break;
         case 12: launch_kernel((matvec_gate_up_kernel<QT, 1, kNorm, 12>), g, b, lds, stream, wg, wu, x, act, K, N, nrm); break;
         case 10: launch_kernel((matvec_gate_up_kernel<QT, 1, kNorm, 10>), g, b, lds, stream, wg, wu, x, act, K, N, nrm); break;
-        case 20:
-            if constexpr (std::is_same<QT, F16>::value) {
-                launch_kernel((matvec_gate_up_kernel<QT, 2, kNorm, 20>), g, b, lds, stream, wg, wu, x, act, K, N, nrm);
-                break;
-            }
-            return hipErrorInvalidValue;   // not reached: tile_length
+        case 20: launch_kernel((matvec_gate_up_kernel<QT, 2, kNorm, 20>), g, b, lds, stream, wg, wu, x, act, K, N, nrm); break;
         default: return hipErrorInvalidValue;
     }
     return hipGetLastError();

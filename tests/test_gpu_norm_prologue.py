@@ -124,3 +124,81 @@ def test_norm_prologue_declines_other_lengths(hip):
     with pytest.raises(hip.CitlaliError, match="no fused kernel"):
         hip.device.matvec_gate_up_swiglu_norm("q4k", dw, dw, up(hip, x), up(hip, d), up(hip, w), None, 1e-6, y, k, n)
     assert (y.download(np.uint16, n) == 0x3c00).all()
+
+
+# Hidden 5120: the number of rows picks the streaming or the tile kernels, the
+# latter with several tiles per workgroup and a partial last one (17411 = 1243
+# tiles of 14 Q4_K rows and 9, 9001 = 562 of 16 Q6_K rows and 9, on 512
+# workgroups).  Every launch form of a matrix gives the plain launch's bits,
+# which one row order pins against the oracle.
+MANY = [("q4k", 17411), ("q4k", 500), ("q6k", 9001), ("q6k", 1000)]
+
+
+@pytest.mark.parametrize("kind,n", MANY)
+def test_hidden_5120_gate_up_forms_agree(hip, orc, kind, n):
+    k = 5120
+    rng, x, d, w = inputs(hip, k, n)
+    hg, hu = (hip.synth.quant_matrix(kind, rng, n, k) for _ in range(2))
+    wg, wu = up(hip, hg), up(hip, hu)
+    normed, resid = reference_norm(hip, x, d, w, k)
+    g, u, ref, plain, got, sum_out = *(hip.DeviceArray(n * 2) for _ in range(5)), hip.DeviceArray(k * 2)
+    print(f"[gate/up forms] {kind} {n} x {k}", flush=True)
+    hip.device.matvec(kind, wg, normed, g, k, n)
+    hip.device.matvec(kind, wu, normed, u, k, n)
+    hip.device.swiglu(g, u, ref, n)
+    hip.device.matvec_gate_up_swiglu(kind, wg, wu, normed, plain, k, n)
+    hip.device.matvec_gate_up_swiglu_norm(kind, wg, wu, up(hip, x), up(hip, d), up(hip, w), sum_out, 1e-6, got, k, n)
+    want = ref.download(np.uint16, n)
+    assert np.array_equal(plain.download(np.uint16, n), want)
+    assert np.array_equal(got.download(np.uint16, n), want)
+    assert np.array_equal(sum_out.download(np.uint16, k), resid)
+    # rows of the first, the last and two inner tiles against the oracle
+    rows = np.r_[0:20, n // 2:n // 2 + 20, n - 20:n]
+    xn = normed.download(np.uint16, k)
+    for h, y in ((hg, g), (hu, u)):
+        o = orc.matvec(kind, np.ascontiguousarray(h.reshape(n, -1)[rows]), xn, k, len(rows))
+        y = y.download(np.uint16, n)[rows].view(np.float16).astype(np.float64)
+        assert np.all(np.abs(y - o) <= 2.0 ** -11 * np.abs(o) + 2e-3)   # one fp16 rounding, fp32 sums
+
+
+@pytest.mark.parametrize("kind,n", [("q4k", 20011), ("q6k", 20011), ("q6k", 700)])
+def test_hidden_5120_matvec_norm_equals_plain(hip, orc, kind, n):
+    k = 5120
+    rng, x, d, w = inputs(hip, k, n)
+    hw = hip.synth.quant_matrix(kind, rng, n, k)
+    dw = up(hip, hw)
+    normed, resid = reference_norm(hip, x, d, w, k)
+    ref, got, sum_out = hip.DeviceArray(n * 4), hip.DeviceArray(n * 4), hip.DeviceArray(k * 2)
+    print(f"[matvec_norm] {kind} {n} x {k}", flush=True)
+    hip.device.matvec(kind, dw, normed, ref, k, n, f32_out=True)
+    hip.device.matvec_norm(kind, dw, up(hip, x), up(hip, d), up(hip, w), sum_out, 1e-6, got, k, n, f32_out=True)
+    got = got.download(np.float32, n)
+    assert np.array_equal(got, ref.download(np.float32, n))
+    assert np.array_equal(sum_out.download(np.uint16, k), resid)
+    rows = np.r_[0:20, n // 2:n // 2 + 20, n - 20:n]
+    o = orc.matvec(kind, np.ascontiguousarray(hw.reshape(n, -1)[rows]), normed.download(np.uint16, k), k, len(rows))
+    assert np.all(np.abs(got[rows] - o) <= 2e-3 + 1e-5 * np.abs(o))
+
+
+@pytest.mark.parametrize("kinds,rows", [
+    (("q4k", "q4k", "q4k"), (9001, 501, 3001)),   # tiles, the matrices' last ones partial
+    (("q6k", "q6k", "q6k"), (8192, 33, 1027)),
+    (("q4k", "q4k", "q6k"), (8001, 3, 3001)),     # two types: streaming
+])
+def test_hidden_5120_groups_equal_plain(hip, kinds, rows):
+    k = 5120
+    rng, x, d, w = inputs(hip, k, sum(rows))
+    ws = [up(hip, hip.synth.quant_matrix(kd, rng, n, k)) for kd, n in zip(kinds, rows)]
+    normed, resid = reference_norm(hip, x, d, w, k)
+    print(f"[groups] {kinds} {rows} x {k}", flush=True)
+    ref, plain, got = ([hip.DeviceArray(n * 2) for n in rows] for _ in range(3))
+    for kd, dw, y, n in zip(kinds, ws, ref, rows):
+        hip.device.matvec(kd, dw, normed, y, k, n)
+    hip.device.matvec_group(kinds, ws, normed, plain, rows, k)
+    sum_out = hip.DeviceArray(k * 2)
+    hip.device.matvec_group_norm(kinds, ws, up(hip, x), up(hip, d), up(hip, w), sum_out, 1e-6, got, rows, k)
+    for r, p, g, n in zip(ref, plain, got, rows):
+        want = r.download(np.uint16, n)
+        assert np.array_equal(p.download(np.uint16, n), want)
+        assert np.array_equal(g.download(np.uint16, n), want)
+    assert np.array_equal(sum_out.download(np.uint16, k), resid)
