@@ -244,37 +244,6 @@ __global__ void swiglu_kernel(const uint16_t* __restrict__ g, const uint16_t* __
     }
 }
 
-// fp16 weights [N][K] (the DequantizeToFp16 path) for K not a multiple of 8 or
-// longer than the other kernels stage: one wave per row, 128-bit loads when K
-// is a multiple of 8, fp32 accumulation.
-template <bool kF32>
-__global__ __launch_bounds__(kBlk) void matvec_f16_kernel(const uint16_t* __restrict__ w,
-                                                          const uint16_t* __restrict__ x, void* __restrict__ y,
-                                                          int K, int N) {
-    const int lane = threadIdx.x & (kWave - 1);
-    const int row = blockIdx.x * (kBlk / kWave) + threadIdx.x / kWave;
-    if (row >= N) return;
-    const uint16_t* r = w + (size_t)row * K;
-    float a = 0.f;
-    if ((K & 7) == 0) {
-        for (int k = lane * 8; k < K; k += kWave * 8) {
-            const u32x4 wv = *reinterpret_cast<const u32x4*>(r + k);
-            const u32x4 xv = *reinterpret_cast<const u32x4*>(x + k);
-            a = dot2(wv.x, xv.x, a);
-            a = dot2(wv.y, xv.y, a);
-            a = dot2(wv.z, xv.z, a);
-            a = dot2(wv.w, xv.w, a);
-        }
-    } else {
-        for (int k = lane; k < K; k += kWave) a = fmaf(h2f(r[k]), h2f(x[k]), a);
-    }
-    a = wave_sum(a);
-    if (lane == 0) {
-        if constexpr (kF32) static_cast<float*>(y)[row] = a;
-        else static_cast<uint16_t*>(y)[row] = f2h_rne(a);
-    }
-}
-
 // Greedy argmax with the host rule of qwen_model.cpp:455-463: the first
 // (lowest index) strictly greatest finite value wins; all non-finite -> 0.
 // Two launches: blocks reduce contiguous ranges to a partial, one block
@@ -480,11 +449,7 @@ hipError_t launch_matvec_f16(const uint16_t* w, const uint16_t* x, void* y, bool
     // whole 256-value blocks: the streaming GEMV kernels (the fused fp16
     // launches use the same ones, so their results are these bits)
     if (K % 256 == 0 && K <= CITLALI_MAX_IN_FEATURES) return launch_matvec_f16_blocks(w, x, y, f32_out, K, N, s);
-    if (f16_rows_length(K)) return launch_matvec_f16_rows(w, x, y, f32_out, K, N, s);
-    const dim3 g((unsigned)((N + (kBlk / kWave) - 1) / (kBlk / kWave)));
-    if (f32_out) launch_kernel(matvec_f16_kernel<true>, g, dim3(kBlk), 0, s, w, x, y, K, N);
-    else launch_kernel(matvec_f16_kernel<false>, g, dim3(kBlk), 0, s, w, x, y, K, N);
-    return hipGetLastError();
+    return launch_matvec_f16_rows(w, x, y, f32_out, K, N, s);
 }
 
 hipError_t launch_argmax(const float* logits, int n, int32_t* out_index, int32_t* state, int32_t* tokens,

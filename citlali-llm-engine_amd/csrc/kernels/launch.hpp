@@ -101,8 +101,7 @@ bool matvec_gate_up_length(int K);
 // through the streaming kernels of the K-quant GEMVs
 hipError_t launch_matvec_f16_blocks(const uint16_t* w, const uint16_t* x, void* y, bool f32_out, int K, int N,
                                     hipStream_t s);
-// fp16 weights [N][K] of any K that f16_rows_length takes (matvec_f16.hip)
-bool f16_rows_length(int K);
+// fp16 weights [N][K] of any other K (matvec_f16.hip)
 hipError_t launch_matvec_f16_rows(const uint16_t* w, const uint16_t* x, void* y, bool f32_out, int K, int N,
                                   hipStream_t s);
 hipError_t launch_matvec_q4k(const uint8_t* w, const uint16_t* x, void* y, bool f32_out, int K, int N,

@@ -1,9 +1,9 @@
 // matvec_f16.hip -- GEMV over fp16 weight rows (kernels.cu:27-35, 381-412 of
 // the reference) of the lengths that the streaming kernels of
-// matvec_kquant.hip have no instantiation for: any multiple of 8.  Products
-// and sums in fp32 (v_dot2_f32_f16), fp16 outputs rounded nearest-even.
+// matvec_kquant.hip have no instantiation for.  Products and sums in fp32
+// (v_dot2_f32_f16), fp16 outputs rounded nearest-even.
 //
-// gfx950 design
+// gfx950 design of the ring kernel (multiples of 8)
 //  * A wave takes one row at a time and copies it 1 KB per instruction (512
 //    values, lane l the 16 bytes at 16 l of the step), whole cache lines,
 //    nontemporal, into four LDS slots of its own, the ring running on over the
@@ -12,8 +12,7 @@
 //  * x is staged in LDS in its own order, padded with zeros to whole steps;
 //    in a partial last step the lanes past the row end re-read its last
 //    values and count them as zero.
-//  * A row's sum: per lane four fp32 chains (one per weight word) over the
-//    steps in order, added pairwise, then the wave sum.
+//  * A row's sum: per lane short fp32 chains (see one_chain), then the wave sum.
 // Bound by HBM.  Against the walk over 256-value blocks of four rows that
 // served these lengths before (us, rotated weights): 5120 x 17408 39.5 -> 28.8
 // (6.2 TB/s), 18944 x 3584 25.5 -> 22.1, 300 x 19968 16.3 -> 10.1.  The
@@ -35,11 +34,50 @@ constexpr int kWaves = kBlock / kWave;
 constexpr int kStepValues = kWave * 8;
 constexpr int kStepBytes = kStepValues * 2;
 constexpr int kDepth = 4;   // steps in flight per wave; eight measured no faster
+constexpr int kFlush = 4;   // steps between additions to a lane's total
 
 __host__ __device__ constexpr int steps_of(int K) { return (K + kStepValues - 1) / kStepValues; }
 constexpr int lds_bytes(int K) { return (steps_of(K) + kWaves * kDepth) * kStepBytes; }
 
+// One wave per row, x and the row straight into registers: K not a multiple of
+// 8 or longer than the ring kernel stages.
 template <bool kF32>
+__global__ __launch_bounds__(kBlock) void matvec_f16_kernel(const uint16_t* __restrict__ w,
+                                                          const uint16_t* __restrict__ x, void* __restrict__ y,
+                                                          int K, int N) {
+    const int lane = threadIdx.x & (kWave - 1);
+    const int row = blockIdx.x * (kBlock / kWave) + threadIdx.x / kWave;
+    if (row >= N) return;
+    const uint16_t* r = w + (size_t)row * K;
+    float a = 0.f;
+    if ((K & 7) == 0) {
+        for (int k = lane * 8; k < K; k += kWave * 8) {
+            const u32x4 wv = *reinterpret_cast<const u32x4*>(r + k);
+            const u32x4 xv = *reinterpret_cast<const u32x4*>(x + k);
+            a = dot2(wv.x, xv.x, a);
+            a = dot2(wv.y, xv.y, a);
+            a = dot2(wv.z, xv.z, a);
+            a = dot2(wv.w, xv.w, a);
+        }
+    } else {
+        for (int k = lane; k < K; k += kWave) a = fmaf(h2f(r[k]), h2f(x[k]), a);
+    }
+    a = wave_sum(a);
+    if (lane == 0) {
+        if constexpr (kF32) static_cast<float*>(y)[row] = a;
+        else static_cast<uint16_t*>(y)[row] = f2h_rne(a);
+    }
+}
+
+// A lane's sums run as one chain over its words in order (the order of
+// matvec_f16_kernel, so the two give the same bits), or, for long rows of whole
+// blocks, as four, one per weight word, that are added to a total every kFlush
+// steps, with what the addition rounds off kept beside it (Knuth's two-sum):
+// chains over the whole row were up to 1.3 times further from 64-bit sums than
+// the walk over 256-value blocks that served these lengths before.
+__host__ __device__ constexpr bool one_chain(int K) { return K % 256 != 0 || K <= 1536; }
+
+template <bool kF32, bool kOneChain>
 __global__ __launch_bounds__(kBlock, 2) void f16_rows_kernel(const uint16_t* __restrict__ w,
                                                              const uint16_t* __restrict__ x, void* __restrict__ y,
                                                              int K, int n) {
@@ -76,7 +114,7 @@ __global__ __launch_bounds__(kBlock, 2) void f16_rows_kernel(const uint16_t* __r
     wait_vm<kDepth>();   // x is in LDS
     lds_only_barrier();
 
-    float a0 = 0.f, a1 = 0.f, a2 = 0.f, a3 = 0.f;
+    float a0 = 0.f, a1 = 0.f, a2 = 0.f, a3 = 0.f, total = 0.f, lost = 0.f;
     int row = first, t = 0, slot = 0, issued = kDepth;
     for (int c = 0; c < S; ++c) {
         const int later = issued - c - 1;   // steps in flight behind this one
@@ -98,17 +136,29 @@ __global__ __launch_bounds__(kBlock, 2) void f16_rows_kernel(const uint16_t* __r
             const uint32_t keep = t * kStepBytes + lane_at <= last_at ? 0xffffffffu : 0u;
             b = b & u32x4{keep, keep, keep, keep};
         }
-        a0 = dot2(b.x, xv.x, a0);
-        a1 = dot2(b.y, xv.y, a1);
-        a2 = dot2(b.z, xv.z, a2);
-        a3 = dot2(b.w, xv.w, a3);
-        if (++t == T) {   // wave-uniform
-            const float s = wave_sum((a0 + a1) + (a2 + a3));
+        if constexpr (kOneChain) {
+            a0 = dot2(b.w, xv.w, dot2(b.z, xv.z, dot2(b.y, xv.y, dot2(b.x, xv.x, a0))));
+        } else {
+            a0 = dot2(b.x, xv.x, a0);
+            a1 = dot2(b.y, xv.y, a1);
+            a2 = dot2(b.z, xv.z, a2);
+            a3 = dot2(b.w, xv.w, a3);
+        }
+        ++t;
+        if (!kOneChain && (t % kFlush == 0 || t == T)) {   // wave-uniform
+            const float p = (a0 + a1) + (a2 + a3), sum = total + p, z = sum - total;
+            lost += (total - (sum - z)) + (p - z);
+            total = sum;
+            a0 = a1 = a2 = a3 = 0.f;
+        }
+        if (t == T) {   // wave-uniform
+            // (an infinite total stays what it is)
+            const float s = wave_sum(kOneChain ? a0 : fabsf(lost) < INFINITY ? total + lost : total);
             if (lane == 0) {
                 if constexpr (kF32) static_cast<float*>(y)[row] = s;
                 else static_cast<uint16_t*>(y)[row] = f2h_rne(s);
             }
-            a0 = a1 = a2 = a3 = 0.f;
+            a0 = total = lost = 0.f;
             t = 0;
             row += stride;
         }
@@ -116,22 +166,29 @@ __global__ __launch_bounds__(kBlock, 2) void f16_rows_kernel(const uint16_t* __r
     wait_vm<0>();   // no copy outlives the workgroup's LDS
 }
 
-template <bool kF32>
-hipError_t launch(const uint16_t* w, const uint16_t* x, void* y, int K, int n, hipStream_t s) {
+template <bool kF32, bool kOneChain>
+hipError_t launch_ring(const uint16_t* w, const uint16_t* x, void* y, int K, int n, hipStream_t s) {
     // three workgroups per CU where their LDS fits (5120 x 17408: 30.1 us with
     // two, 28.8 with three, 31.5 with four)
     const int lds = lds_bytes(K), per_cu = std::max(1, std::min(3, 160 * 1024 / lds));
     const int grid = std::min((n + kWaves - 1) / kWaves, per_cu * device_cus());
-    constexpr auto kernel = f16_rows_kernel<kF32>;
+    constexpr auto kernel = f16_rows_kernel<kF32, kOneChain>;
     const hipError_t e = allow_lds<kernel>(lds);
     if (e != hipSuccess) return e;
     launch_kernel(kernel, dim3(grid), dim3(kBlock), (size_t)lds, s, w, x, y, K, n);
     return hipGetLastError();
 }
 
-}  // namespace
+template <bool kF32>
+hipError_t launch(const uint16_t* w, const uint16_t* x, void* y, int K, int n, hipStream_t s) {
+    if (K % 8 != 0 || K > CITLALI_MAX_IN_FEATURES) {
+        launch_kernel(matvec_f16_kernel<kF32>, dim3((n + kWaves - 1) / kWaves), dim3(kBlock), 0, s, w, x, y, K, n);
+        return hipGetLastError();
+    }
+    return one_chain(K) ? launch_ring<kF32, true>(w, x, y, K, n, s) : launch_ring<kF32, false>(w, x, y, K, n, s);
+}
 
-bool f16_rows_length(int K) { return K > 0 && K % 8 == 0 && K <= CITLALI_MAX_IN_FEATURES; }
+}  // namespace
 
 hipError_t launch_matvec_f16_rows(const uint16_t* w, const uint16_t* x, void* y, bool f32_out, int K, int N,
                                   hipStream_t s) {

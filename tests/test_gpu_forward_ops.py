@@ -147,11 +147,11 @@ def test_argmax_matches_host_rule(hip, orc):
 
 @pytest.mark.parametrize("f32", [False, True])
 @pytest.mark.parametrize("k,n", [
-    (1024, 3072), (2560, 100), (28672, 64),       # whole 256-value blocks, any count: the flat walk
+    (1024, 3072), (2560, 100), (28672, 64),       # whole 256-value blocks
     (4096, 1024), (4096, 4096), (4096, 12288),    # Qwen3-8B shapes: one pass / streamed
     (8192, 1000), (12288, 4096), (16384, 300),    # longer rows (x from LDS beyond two steps)
     (2560, 300), (5120, 257),                     # rows ending in a partial wave step
-    (17408, 30), (25600, 20),                     # beyond four steps: the flat walk
+    (17408, 30), (25600, 20),                     # beyond four steps: the LDS ring
     (1000, 64),                                   # K not a multiple of 256: one wave per row
 ])
 def test_matvec_fp16(hip, orc, k, n, f32):
@@ -397,3 +397,20 @@ def test_matvec_fp16_other_lengths(hip, orc, k):
         assert np.all(np.abs(got[:n] - wf @ xf) <= bound)
         hip.device.matvec("fp16", dw, dx, dy, k, n)
         assert np.array_equal(dy.download(np.uint16, n), got[:n].astype(np.float16).view(np.uint16))
+
+
+@pytest.mark.parametrize("k,bound", [(9216, 1.03e-7), (18944, 1.12e-7), (28672, 1.18e-7)])
+def test_matvec_fp16_long_rows_sum_in_short_chains(hip, k, bound):
+    """Relative rms error of fp32 outputs over 2000 rows against 64 bits, no
+    larger than that of the walk over 256-value blocks (the bounds: what it
+    showed on these inputs, rounded up)."""
+    n = 2000
+    gen = np.random.default_rng(k)
+    w = gen.standard_normal(n * k, dtype=np.float32).astype(np.float16)
+    x = gen.standard_normal(k, dtype=np.float32).astype(np.float16)
+    ref = np.concatenate([p.astype(np.float64) @ x.astype(np.float64) for p in np.split(w.reshape(n, k), 10)])
+    dy = hip.DeviceArray(n * 4)
+    hip.device.matvec("fp16", up(hip, w.view(np.uint16)), up(hip, x.view(np.uint16)), dy, k, n, f32_out=True)
+    err = np.linalg.norm(dy.download(np.float32, n) - ref) / np.linalg.norm(ref)
+    print(f"[matvec_fp16 sums] {n} x {k}: relative rms error {err:.3g}", flush=True)
+    assert err <= bound
