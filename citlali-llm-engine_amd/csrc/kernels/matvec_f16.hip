@@ -40,7 +40,7 @@ __host__ __device__ constexpr int steps_of(int K) { return (K + kStepValues - 1)
 constexpr int lds_bytes(int K) { return (steps_of(K) + kWaves * kDepth) * kStepBytes; }
 
 // One wave per row, x and the row straight into registers: K not a multiple of
-// 8 or longer than the ring kernel stages.
+// 8 or longer than the ring kernel stages, and launches too small for it.
 template <bool kF32>
 __global__ __launch_bounds__(kBlock) void matvec_f16_kernel(const uint16_t* __restrict__ w,
                                                           const uint16_t* __restrict__ x, void* __restrict__ y,
@@ -179,9 +179,20 @@ hipError_t launch_ring(const uint16_t* w, const uint16_t* x, void* y, int K, int
     return hipGetLastError();
 }
 
+// Launches for which the ring kernel's set-up (x and zeros to LDS, the rings
+// filled) costs more than it gains, among the one-chain lengths, where both
+// kernels give the same bits.  us, wave per row / ring: 12000 x 8 3.0 / 4.1,
+// 3584 x 200 2.8 / 3.9, 12000 x 200 4.3 / 4.5 (40000: 8.1 / 7.9), 3584 x 1000 3.8
+// / 4.2 (12000: 6.8 / 6.6); longer rows, whose loads a wave waits for in turn,
+// 200 x 1800 2.6 / 3.2 (1024: 4.3 / 3.4), 128 x 2504 2.6 / 3.4 (200: 3.9 / 3.4),
+// 64 x 5000 3.1 / 4.1 (128: 6.1 / 4.1), 32 x 19000 6.5 / 8.6 (64: 19.6 / 8.5).
+bool small_launch(int K, int n) {
+    return one_chain(K) && ((long long)K * n < (K <= 1024 ? 8 << 20 : 480 << 10) || n <= (K <= 9216 ? 64 : 32));
+}
+
 template <bool kF32>
 hipError_t launch(const uint16_t* w, const uint16_t* x, void* y, int K, int n, hipStream_t s) {
-    if (K % 8 != 0 || K > CITLALI_MAX_IN_FEATURES) {
+    if (K % 8 != 0 || K > CITLALI_MAX_IN_FEATURES || small_launch(K, n)) {
         launch_kernel(matvec_f16_kernel<kF32>, dim3((n + kWaves - 1) / kWaves), dim3(kBlock), 0, s, w, x, y, K, n);
         return hipGetLastError();
     }

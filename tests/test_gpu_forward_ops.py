@@ -399,6 +399,22 @@ def test_matvec_fp16_other_lengths(hip, orc, k):
         assert np.array_equal(dy.download(np.uint16, n), got[:n].astype(np.float16).view(np.uint16))
 
 
+@pytest.mark.parametrize("k", [8, 200, 768, 1000, 1536, 1800, 5000])
+def test_matvec_fp16_bits_do_not_depend_on_the_row_count(hip, k):
+    """Few rows run one wave per row, many (8 M weights, 480 K in rows past
+    1024) the LDS ring: the same sums."""
+    rng = hip.synth.Rng(k)
+    n = (8 << 20) // k + 100 if k <= 1024 else 3000
+    w, x = hip.synth.normal_f16(rng, n * k), hip.synth.normal_f16(rng, k)
+    dw, dx, dy = up(hip, w), up(hip, x), hip.DeviceArray(n * 4)
+    print(f"[matvec_fp16 row counts] {n} x {k}", flush=True)
+    hip.device.matvec("fp16", dw, dx, dy, k, n, f32_out=True)
+    many = dy.download(np.float32, n)
+    for few in (1, 29):
+        hip.device.matvec("fp16", dw, dx, dy, k, few, f32_out=True)
+        np.testing.assert_array_equal(dy.download(np.float32, few), many[:few])
+
+
 @pytest.mark.parametrize("k,bound", [(9216, 1.03e-7), (18944, 1.12e-7), (28672, 1.18e-7)])
 def test_matvec_fp16_long_rows_sum_in_short_chains(hip, k, bound):
     """Relative rms error of fp32 outputs over 2000 rows against 64 bits, no
