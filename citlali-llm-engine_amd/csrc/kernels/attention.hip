@@ -12,10 +12,11 @@
 //    serves every query head of the GQA group, so K and V are read from HBM
 //    once per kv head (the reference re-reads them per query head).
 //  * Each wave streams tiles of positions with the next tile's loads issued
-//    before the current one is consumed; both products run on the matrix
-//    cores, for every head_dim and group (the padding columns cost nothing
-//    that bounds the kernel: it waits for memory and LDS, not for MFMA).
-//    Exponentials are taken in base 2 with log2(e) folded into the scale.
+//    before the current one is consumed.  With enough heads per kv head both
+//    products run on the matrix cores (the padding columns cost nothing that
+//    bounds that kernel: it waits for memory and LDS, not for MFMA), else on
+//    the VALU (on_valu).  Exponentials are taken in base 2 with log2(e) folded
+//    into the scale.
 //  * The four waves merge in LDS; a chunk writes (max, sum, acc[head_dim])
 //    per head and a second kernel merges the chunks of each query head by
 //    log-sum-exp.  A sequence that fits one chunk is written directly.
@@ -36,6 +37,15 @@ constexpr int kBlock = 256;
 constexpr int kWaves = kBlock / kWave;
 constexpr int kMaxSplits = 512;   // plan_attention never makes more chunks
 
+// Shapes on attn_valu_kernel.  us, split + merge, VALU / matrix cores: 8/8 heads
+// of 64 4.3 / 4.7 at 256 positions, 8.4 / 8.8 at 8192; 100 sequences of
+// 40..400 13.6 / 15.8; 4/4 heads of 128 5.8 / 6.7 at 256, 9.0 / 9.5 at 4096, 32
+// sequences of 250..2500 20.4 / 24.3 (32/32 heads past 20000 positions 64.6 /
+// 58.7); 16/8 heads of 64 7.3 / 7.1 at 512, 100 sequences of 150..1500 35.9 /
+// 37.3.  With four heads of 64 and more the matrix cores win: 12/4 heads 8.3 /
+// 6.9 at 512, 32/4 heads 9.3 / 4.9 at 256.
+constexpr bool on_valu(int head_dim, int gp) { return gp == 1 || (head_dim == 64 && gp == 2); }
+
 // Positions a sequence covers and its chunk count.  A position at or beyond
 // the caller's bound `max_len` is cut there, so neither the cache reads nor
 // the chunk index leave their buffers.
@@ -47,6 +57,238 @@ __device__ __forceinline__ SeqSpan seq_span(const int32_t* positions, int positi
     int L = (positions ? positions[seq] : position) + 1;
     L = min(L, max_len);
     return {L, L > 0 ? (L + chunk - 1) / chunk : 0};
+}
+
+// ---------------------------------------------------------------------------
+// Chunk kernel without GQA, and of two heads per kv head at head_dim 64 (see
+// on_valu): scores by v_dot2_f32_f16 (lane = (position, head), q of the lane's
+// head in VGPRs), values by fp32 multiply-adds (lane = (position group, 8-dim
+// slice)), K and V tiles staged through wave-private LDS.  One or two heads
+// leave most MFMA columns empty, so the matrix cores save little here.
+// ---------------------------------------------------------------------------
+template <int HD, int GP>
+struct ValuCfg {
+    static_assert((HD == 64 && (GP == 1 || GP == 2)) || (HD == 128 && GP == 1), "on_valu");
+    static constexpr int kChunks = HD / 8;                 // 16-byte slices per row
+    static constexpr int kTP = 32;                         // positions per tile
+    static constexpr int kStride = HD + 8;                 // padded LDS row (halves)
+    static constexpr int kRowsPerLoad = kWave / kChunks;
+    static constexpr int kLoads = kTP / kRowsPerLoad;      // per tile, for K and for V
+    // value phase: lane = (position group, 8-dim slice), every head of the group
+    static constexpr int kVGroups = kWave / kChunks;
+    static constexpr int kVPerLane = kTP / kVGroups;       // positions per lane per tile
+    static constexpr int kTileHalves = kTP * kStride;
+    // wave-private region: K tile, V tile, p[kTP][GP], alpha[GP]; 16-byte multiple
+    static constexpr size_t kWaveLds =
+        (((size_t)kTileHalves * 2 * 2 + (size_t)GP * kTP * 4 + (size_t)GP * 4) + 15) & ~(size_t)15;
+    // workgroup merge: (max, sum)[kWaves][GP], then acc[kWaves * kVGroups][GP][HD]
+    static constexpr size_t kMlFloats = ((size_t)kWaves * GP * 2 + 3) & ~(size_t)3;
+    static constexpr size_t kMergeLds = (kMlFloats + (size_t)kWaves * kVGroups * GP * HD) * sizeof(float);
+    static constexpr size_t kBytes = kWaveLds * kWaves > kMergeLds ? kWaveLds * kWaves : kMergeLds;
+    static_assert(kLoads >= 1 && kVPerLane >= 1 && kTP % kVGroups == 0, "tile");
+};
+
+// Grid: (chunk, kv_head, seq).  `positions` (device, per sequence) or the
+// scalar `position` gives the last cached position of each sequence.
+template <int HD, int GP>
+__global__ __launch_bounds__(kBlock) void attn_valu_kernel(
+    const uint16_t* __restrict__ q, const uint16_t* __restrict__ k_cache, const uint16_t* __restrict__ v_cache,
+    long long seq_stride, const int32_t* __restrict__ positions, int position, int max_len, int heads,
+    int kv_heads, int group, int chunk, float scale_log2, float* __restrict__ part, int n_splits,
+    uint16_t* __restrict__ out) {
+    using C = ValuCfg<HD, GP>;
+    extern __shared__ __align__(16) uint8_t smem[];
+
+    const int split = blockIdx.x, kvh = blockIdx.y, seq = blockIdx.z;
+    const SeqSpan span = seq_span(positions, position, seq, chunk, max_len);
+    const int L = span.len, n_valid = span.n_valid;
+    const int b0 = split * chunk;
+    if (b0 >= L) return;
+    const int b1 = min(L, b0 + chunk);
+
+    const int lane = threadIdx.x & (kWave - 1);
+    const int wave = threadIdx.x / kWave;
+    // the chunk's positions split over the four waves in whole tiles (a
+    // short sequence's only chunk still occupies every wave)
+    const int sub = (((b1 - b0 + kWaves - 1) / kWaves + C::kTP - 1) / C::kTP) * C::kTP;
+    const int w0 = min(b1, b0 + wave * sub);
+    const int w1 = min(b1, w0 + sub);
+
+    uint8_t* wl = smem + (size_t)wave * C::kWaveLds;
+    uint16_t* kt = reinterpret_cast<uint16_t*>(wl);
+    uint16_t* vt = kt + C::kTileHalves;
+    float* pt = reinterpret_cast<float*>(vt + C::kTileHalves);   // [kTP][GP]
+    float* at = pt + GP * C::kTP;                                 // [GP]
+
+    const uint16_t* kbase = k_cache + (size_t)seq * seq_stride + (size_t)kvh * HD;
+    const uint16_t* vbase = v_cache + (size_t)seq * seq_stride + (size_t)kvh * HD;
+    const size_t row_step = (size_t)kv_heads * HD;
+
+    // scores-phase identity
+    const int sh = lane % GP, sp = lane / GP;
+    const bool s_head_ok = sh < group;
+    const bool s_lane_ok = sp < C::kTP;
+    // q of the lane's head in VGPRs.  Unconditional loads (a padding head
+    // reads the group's last head and is zeroed) keep every global load
+    // outside branches, so the compiler's load counting stays exact and the
+    // waits below never cover the tiles still in flight.
+    uint32_t qv[HD / 2];
+    {
+        const int hq = kvh * group + (s_head_ok ? sh : group - 1);
+        const uint16_t* qh = q + ((size_t)seq * heads + hq) * HD;
+        const uint32_t keep = s_head_ok ? 0xffffffffu : 0u;
+#pragma unroll
+        for (int c = 0; c < C::kChunks; ++c) {
+            const u32x4 v = *reinterpret_cast<const u32x4*>(qh + c * 8);
+            qv[4 * c + 0] = v.x & keep; qv[4 * c + 1] = v.y & keep;
+            qv[4 * c + 2] = v.z & keep; qv[4 * c + 3] = v.w & keep;
+        }
+    }
+    // value-phase identity: lane = (position group vg, 8-dim slice vc)
+    const int vc = lane % C::kChunks, vg = lane / C::kChunks;
+    float acc[GP][8];
+#pragma unroll
+    for (int h = 0; h < GP; ++h)
+#pragma unroll
+        for (int k = 0; k < 8; ++k) acc[h][k] = 0.f;
+
+    float m_run = -INFINITY, l_run = 0.f;   // per scores lane (head sh)
+
+    // load identity; one tile of K and V rows in flight per wave
+    const int lrow = lane / C::kChunks, lc = lane % C::kChunks;
+    u32x4 kr[C::kLoads], vr[C::kLoads];
+    auto load_tile = [&](int t0) {
+#pragma unroll
+        for (int i = 0; i < C::kLoads; ++i) {
+            // branch-free: rows past the range re-read the last one (never used)
+            const int pos = min(t0 + i * C::kRowsPerLoad + lrow, w1 - 1);
+            kr[i] = *reinterpret_cast<const u32x4*>(kbase + (size_t)pos * row_step + lc * 8);
+            vr[i] = *reinterpret_cast<const u32x4*>(vbase + (size_t)pos * row_step + lc * 8);
+        }
+    };
+
+    // One staged tile; with nv <= 0 it changes nothing (scores -inf, weights 0).
+    auto process_tile = [&](int t0) {
+        const int nv = min(C::kTP, w1 - t0);
+
+        // ---- scores + online softmax (lane = position sp, head sh) ----
+        float s2 = -INFINITY;
+        if (s_lane_ok && s_head_ok && sp < nv) {
+            const uint16_t* kr_row = kt + sp * C::kStride;
+            float a0 = 0.f, a1 = 0.f;
+#pragma unroll
+            for (int c = 0; c < C::kChunks; ++c) {
+                const u32x4 kk = *reinterpret_cast<const u32x4*>(kr_row + c * 8);
+                a0 = dot2(qv[4 * c + 0], kk.x, a0);
+                a1 = dot2(qv[4 * c + 1], kk.y, a1);
+                a0 = dot2(qv[4 * c + 2], kk.z, a0);
+                a1 = dot2(qv[4 * c + 3], kk.w, a1);
+            }
+            s2 = (a0 + a1) * scale_log2;
+        }
+        const float mt = column_max<GP>(s2);
+        const float m_new = fmaxf(m_run, mt);
+        const bool live = m_new != -INFINITY;
+        const float alpha = live ? __builtin_amdgcn_exp2f(m_run - m_new) : 1.f;
+        const float pw = live ? __builtin_amdgcn_exp2f(s2 - m_new) : 0.f;
+        const float ps = column_sum<GP>(pw);
+        l_run = l_run * alpha + ps;
+        m_run = m_new;
+        if (s_lane_ok) pt[lane] = pw;   // lane = sp * GP + sh
+        if (sp == 0) at[sh] = alpha;
+        wave_lds_sync();
+
+        // ---- values: every head for kVPerLane positions of this lane ----
+        float al[GP];
+        load_floats<GP>(at, al);
+#pragma unroll
+        for (int h = 0; h < GP; ++h)
+#pragma unroll
+            for (int k = 0; k < 8; ++k) acc[h][k] *= al[h];
+        // rows past nv hold finite copies of a valid row and weight 0
+#pragma unroll
+        for (int j = 0; j < C::kVPerLane; ++j) {
+            const int p = vg + j * C::kVGroups;
+            const u32x4 vv = *reinterpret_cast<const u32x4*>(vt + p * C::kStride + vc * 8);
+            float pp[GP];
+            load_floats<GP>(pt + p * GP, pp);
+            const float v8[8] = {h2f(vv.x & 0xffffu), h2f(vv.x >> 16), h2f(vv.y & 0xffffu), h2f(vv.y >> 16),
+                                 h2f(vv.z & 0xffffu), h2f(vv.z >> 16), h2f(vv.w & 0xffffu), h2f(vv.w >> 16)};
+#pragma unroll
+            for (int h = 0; h < GP; ++h)
+#pragma unroll
+                for (int k = 0; k < 8; ++k) acc[h][k] = fmaf(pp[h], v8[k], acc[h][k]);
+        }
+        wave_lds_sync();
+    };
+
+    // A tile is consumed while the next one loads: its registers are refilled
+    // as soon as it is in LDS.  Loads are unconditional (past the range they
+    // re-read row w1 - 1, in bounds even for an empty range since w1 = b1 >= 1
+    // there), so no load sits in a branch; sched_barrier pins the issue order.
+    __builtin_amdgcn_sched_barrier(0);
+    load_tile(w0);
+    __builtin_amdgcn_sched_barrier(0);
+    for (int t0 = w0; t0 < w1; t0 += C::kTP) {
+        // every row is stored: rows past the range hold a copy of row w1 - 1
+        // and get weight 0
+#pragma unroll
+        for (int i = 0; i < C::kLoads; ++i) {
+            const int r = i * C::kRowsPerLoad + lrow;
+            *reinterpret_cast<u32x4*>(kt + r * C::kStride + lc * 8) = kr[i];
+            *reinterpret_cast<u32x4*>(vt + r * C::kStride + lc * 8) = vr[i];
+        }
+        wave_lds_sync();
+        __builtin_amdgcn_sched_barrier(0);
+        load_tile(t0 + C::kTP);
+        __builtin_amdgcn_sched_barrier(0);
+        process_tile(t0);
+    }
+
+    // ---- merge the position groups and the four waves in LDS ----
+    __syncthreads();   // every wave is done with its tiles
+    float* ml = reinterpret_cast<float*>(smem);   // [kWaves][GP] (max, sum)
+    float* ms = ml + C::kMlFloats;                // [kWaves * kVGroups][GP][HD]
+    if (sp == 0) {
+        ml[(wave * GP + sh) * 2] = m_run;
+        ml[(wave * GP + sh) * 2 + 1] = l_run;
+    }
+#pragma unroll
+    for (int h = 0; h < GP; ++h) {
+        f32x4* e = reinterpret_cast<f32x4*>(ms + ((size_t)(wave * C::kVGroups + vg) * GP + h) * HD + vc * 8);
+        e[0] = f32x4{acc[h][0], acc[h][1], acc[h][2], acc[h][3]};
+        e[1] = f32x4{acc[h][4], acc[h][5], acc[h][6], acc[h][7]};
+    }
+    __syncthreads();
+
+    for (int idx = threadIdx.x; idx < group * HD; idx += kBlock) {
+        const int h = idx / HD, d = idx - h * HD;
+        float M = -INFINITY;
+#pragma unroll
+        for (int w = 0; w < kWaves; ++w) M = fmaxf(M, ml[(w * GP + h) * 2]);
+        float Ls = 0.f, A = 0.f;
+#pragma unroll
+        for (int w = 0; w < kWaves; ++w) {
+            const float mw = ml[(w * GP + h) * 2];
+            const float f = mw == -INFINITY ? 0.f : exp2f(mw - M);
+            Ls += ml[(w * GP + h) * 2 + 1] * f;
+            float a = 0.f;
+#pragma unroll
+            for (int g = 0; g < C::kVGroups; ++g) a += ms[((size_t)(w * C::kVGroups + g) * GP + h) * HD + d];
+            A += a * f;
+        }
+        const int hq = kvh * group + h;
+        if (n_valid == 1) {
+            out[((size_t)seq * heads + hq) * HD + d] = f2h_rne(A / Ls);
+        } else {
+            float* pe = part + (((size_t)seq * heads + hq) * n_splits + split) * (HD + 4);
+            pe[d] = A;
+            if (d == 0) {
+                pe[HD] = M;
+                pe[HD + 1] = Ls;
+            }
+        }
+    }
 }
 
 // ---------------------------------------------------------------------------
@@ -138,8 +380,8 @@ __global__ __launch_bounds__(NW * kWave, kRows ? 4 : 1) void attn_mfma_kernel(
     uint16_t* __restrict__ out, QkPrep prep) {
     using T = AttnTile<HD>;
     constexpr int kTile = T::kPos, kStride = T::kStride;
-    static_assert(GP >= 1 && GP <= 8, "group");
-    static_assert(!kPrep || (HD == 128 && GP >= 2), "the q/k prologue is built for head_dim 128 with GQA");
+    static_assert(!on_valu(HD, GP) && GP <= 8, "group");
+    static_assert(!kPrep || HD == 128, "the q/k prologue is built for head_dim 128 with GQA");
     extern __shared__ __align__(16) uint8_t smem[];
 
     const int split = blockIdx.x, kvh = blockIdx.y, seq = blockIdx.z;
@@ -631,15 +873,33 @@ hipError_t launch_chunks(const AttnArgs& a, const AttnPlan& p, const QkPrep& pre
 }
 
 template <int HD, int GP>
+hipError_t launch_valu(const AttnArgs& a, const AttnPlan& p, hipStream_t stream) {
+    const float scale_log2 = (float)(1.4426950408889634 / sqrt((double)HD));
+    launch_kernel_in_call(p.n_splits <= 1, (attn_valu_kernel<HD, GP>), dim3(p.n_splits, a.kv_heads, a.nseq),
+                          dim3(kBlock), ValuCfg<HD, GP>::kBytes, stream, a.q, a.k_cache, a.v_cache, a.seq_stride,
+                          a.positions, a.position, a.max_len, a.heads, a.kv_heads, a.heads / a.kv_heads, p.chunk,
+                          scale_log2, a.workspace, p.n_splits, a.out);
+    const hipError_t e = hipGetLastError();
+    if (e != hipSuccess || p.n_splits <= 1) return e;
+    launch_merge<HD>(a, p, stream);
+    return hipGetLastError();
+}
+
+template <int HD, int GP>
 hipError_t launch_group(const AttnArgs& a, const AttnPlan& p, hipStream_t s) {
-    if (a.prep != nullptr) {
-        if constexpr (HD == 128 && GP >= 2)
-            return p.rows ? launch_chunks<HD, GP, true, true>(a, p, *a.prep, s)
-                          : launch_chunks<HD, GP, false, true>(a, p, *a.prep, s);
-        return hipErrorInvalidValue;   // the q/k prologue is not built for this shape
+    if constexpr (on_valu(HD, GP)) {
+        if (a.prep != nullptr) return hipErrorInvalidValue;   // the q/k prologue is not built for this shape
+        return launch_valu<HD, GP>(a, p, s);
+    } else {
+        if (a.prep != nullptr) {
+            if constexpr (HD == 128)
+                return p.rows ? launch_chunks<HD, GP, true, true>(a, p, *a.prep, s)
+                              : launch_chunks<HD, GP, false, true>(a, p, *a.prep, s);
+            return hipErrorInvalidValue;   // the q/k prologue is not built for this shape
+        }
+        return p.rows ? launch_chunks<HD, GP, true, false>(a, p, QkPrep{}, s)
+                      : launch_chunks<HD, GP, false, false>(a, p, QkPrep{}, s);
     }
-    return p.rows ? launch_chunks<HD, GP, true, false>(a, p, QkPrep{}, s)
-                  : launch_chunks<HD, GP, false, false>(a, p, QkPrep{}, s);
 }
 
 template <int HD>

@@ -308,3 +308,52 @@ def test_batched_other_shapes_tile_edges(hip, orc, heads, kv, hd, nseq, bound):
                             kv, hd)
         # one fp16 rounding of the output plus fp32 noise
         assert np.all(np.abs(got[s] - ref) <= np.abs(ref) * 2 ** -10 + 1e-4), (n, np.abs(got[s] - ref).max())
+
+
+# Shapes whose value sums run in fp32 (attn_valu_kernel) or with weights split
+# over the matrix cores, each with few and with many heads per kv head
+VALUE_SUMS = [(4, 4, 64), (8, 4, 64), (4, 4, 128)]
+
+
+def _sink(seed, L, heads, kv, hd):
+    """q, K, V in which position 0 has all but about 2^-24 of every head's
+    weight and V[0] = 0: the output is what the other weights keep."""
+    gen = np.random.default_rng(seed)
+    u = gen.standard_normal(hd)
+    u /= np.linalg.norm(u)
+    q = (0.25 * gen.standard_normal((heads, hd)) + 4 * u).astype(np.float16)
+    k = gen.standard_normal((L, kv, hd)).astype(np.float16)
+    v = (gen.standard_normal((L, kv, hd)) * 200 + 400).astype(np.float16)
+    k[0], v[0] = (u * np.sqrt(hd) * 17 / 4).astype(np.float16), 0
+    return (a.reshape(-1).view(np.uint16) for a in (q, k, v))
+
+
+@pytest.mark.parametrize("heads,kv,hd", VALUE_SUMS)
+@pytest.mark.parametrize("L", [100, 2000])
+def test_small_weights_keep_their_value(hip, orc, heads, kv, hd, L):
+    """Weights far below the largest one count in full: no output is more than
+    the last fp16 rounding (2^-11, or half the subnormal spacing) and the fp32
+    scores' own error (a few 2^-24 of scores up to 32, in the exponent) off."""
+    q, k, v = _sink(L + heads, L, heads, kv, hd)
+    got = _run(hip, q, k, v, L - 1, L, heads, kv, hd)
+    ref = orc.attention(q, k, v, L - 1, heads, kv, hd)
+    assert np.abs(ref).min() > 2.0 ** -16
+    err = np.abs(got - ref)
+    print(f"[attention sink] {heads}/{kv} heads of {hd}, L = {L}: {np.max(err / np.abs(ref)):.2g}", flush=True)
+    assert np.all(err <= 2.0 ** -11 * np.abs(ref) + 2.0 ** -25 + 2.0 ** -17 * np.abs(ref))
+
+
+@pytest.mark.parametrize("heads,kv,hd", VALUE_SUMS)
+@pytest.mark.parametrize("L", [40, 300, 5000])
+def test_infinite_value_stays_infinite(hip, orc, heads, kv, hd, L):
+    """An Inf in V (not in a sequence's last chunk, which the merge may read
+    twice) is an Inf of its sign in its dim for every head of its kv head, and
+    nothing else changes."""
+    k, v = _cache(hip, 900 + L, L, kv, hd)
+    q = hip.synth.normal_f16(hip.synth.Rng(901), heads * hd)
+    ref = _run(hip, q, k, v, L - 1, L, heads, kv, hd).reshape(kv, heads // kv, hd)
+    v3 = v.reshape(L, kv, hd)
+    v3[5, 1, 7], v3[20, 2, 0], v3[33, 2, hd - 1] = 0x7c00, 0xfc00, 0x7c00
+    got = _run(hip, q, k, v3.reshape(-1), L - 1, L, heads, kv, hd).reshape(kv, heads // kv, hd)
+    ref[1, :, 7], ref[2, :, 0], ref[2, :, hd - 1] = np.inf, -np.inf, np.inf
+    np.testing.assert_array_equal(got, ref)
