@@ -319,8 +319,10 @@ __global__ __launch_bounds__(kBlock) void attn_valu_kernel(
 //    layout is the B operand P^T as it stands, so every accumulator of a
 //    lane belongs to the lane's head column and the online-softmax rescale
 //    needs no lane moves (none on a wave's first tile).  P goes in as
-//    fp16 hi + lo halves (two MFMAs), so its fp32 value counts to about
-//    2^-22.  V rows are staged in a wave-private LDS tile and gathered per
+//    fp16 hi + lo halves (two MFMAs): a weight counts to 2^-22 of itself, and
+//    no weight to less than 2^-25 (head_dim 128) or 2^-39 (64, see kScale) of
+//    the tile's largest.  (fp32 MFMAs instead: 1 us more per attention of 32/4
+//    heads of 64.)  V rows are staged in a wave-private LDS tile and gathered per
 //    lane as 4 positions x 4 dims, the A operand (dims 64c + 4col + e feed
 //    output block 4c + e, rows 4grp + i of which are dims 64c + 16grp + 4i + e).
 // ---------------------------------------------------------------------------
@@ -354,6 +356,10 @@ struct MfmaLds {
 
 __device__ __forceinline__ f32x4 mfma16(half4 a, half4 b, f32x4 c) {
     return __builtin_amdgcn_mfma_f32_16x16x16f16(a, b, c, 0, 0, 0);
+}
+
+__device__ __forceinline__ f32x4 mfma4(float a, float b, f32x4 c) {
+    return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
 }
 
 __device__ __forceinline__ half4 as_half4(uint32_t lo, uint32_t hi) {
@@ -476,7 +482,19 @@ __global__ __launch_bounds__(NW * kWave, kRows ? 4 : 1) void attn_mfma_kernel(
     };
 
     const uint16_t* kv_new = reinterpret_cast<const uint16_t*>(smem + Lds::kKv) + (size_t)wave * 2 * HD;
-    auto process = [&](int t0, auto first_tile) {
+    // kScale: the weights as the value product takes them.  At head_dim 64 they
+    // are raised by 2^14 (undone after the loop), so that their low halves stay
+    // normal fp16 numbers down to 2^-17 of the largest weight and the halves end
+    // at 2^-39 of it instead of 2^-25.
+    constexpr float kScale = HD == 64 ? 16384.f : 1.f;
+    // fp32_values: the value product in fp32, for values that are not finite
+    auto process = [&](int t0, auto first_tile, auto fp32_values) {
+        if constexpr (decltype(fp32_values)::value) {
+            // rows past the range hold a copy of row w1 - 1 and have weight 0
+#pragma unroll
+            for (int u = 0; u < 4; ++u)
+                if (t0 + slot_row(u) >= w1) vr[u] = u32x4{0u, 0u, 0u, 0u};
+        }
         if constexpr (kPrep) {
             // the step's row comes from the prologue's k' and v in LDS
 #pragma unroll
@@ -572,11 +590,17 @@ __global__ __launch_bounds__(NW * kWave, kRows ? 4 : 1) void attn_mfma_kernel(
             for (int b = 0; b < T::kOut; ++b) o[b] *= alpha;
         }
         half4 ph[T::kSubs], pl[T::kSubs];
+        if constexpr (HD == 64) {
 #pragma unroll
-        for (int j = 0; j < 4 * T::kSubs; ++j) {
-            const _Float16 h = (_Float16)pv[j];
-            ph[j / 4][j % 4] = h;
-            pl[j / 4][j % 4] = (_Float16)(pv[j] - (float)h);
+            for (int j = 0; j < 4 * T::kSubs; ++j) pv[j] *= kScale;
+        }
+        if constexpr (!decltype(fp32_values)::value) {
+#pragma unroll
+            for (int j = 0; j < 4 * T::kSubs; ++j) {
+                const _Float16 h = (_Float16)pv[j];
+                ph[j / 4][j % 4] = h;
+                pl[j / 4][j % 4] = (_Float16)(pv[j] - (float)h);
+            }
         }
         if constexpr (!kRows) wave_lds_sync();   // the V rows stored above
 #pragma unroll
@@ -590,6 +614,16 @@ __global__ __launch_bounds__(NW * kWave, kRows ? 4 : 1) void attn_mfma_kernel(
                         *reinterpret_cast<const u32x2*>(vt + (4 * grp + (16 * b + j)) * kStride + 64 * c + 4 * col);
                     w[j][0] = x.x;
                     w[j][1] = x.y;
+                }
+                if constexpr (decltype(fp32_values)::value) {
+                    // positions 4grp + j of the four lane groups per MFMA
+#pragma unroll
+                    for (int j = 0; j < 4; ++j)
+#pragma unroll
+                        for (int e = 0; e < 4; ++e)
+                            o[4 * c + e] = mfma4(h2f((w[j][e >> 1] >> (16 * (e & 1))) & 0xffffu), pv[4 * b + j],
+                                                 o[4 * c + e]);
+                    continue;
                 }
 #pragma unroll
                 for (int e = 0; e < 4; ++e) {
@@ -672,10 +706,30 @@ __global__ __launch_bounds__(NW * kWave, kRows ? 4 : 1) void attn_mfma_kernel(
         }
     }
     if constexpr (kPrep) {
-        for (int t0 = w0; t0 < w1; t0 += kTile) process(t0, std::false_type{});
+        for (int t0 = w0; t0 < w1; t0 += kTile) process(t0, std::false_type{}, std::false_type{});
     } else {
-        if (w0 < w1) process(w0, std::true_type{});
-        for (int t0 = w0 + kTile; t0 < w1; t0 += kTile) process(t0, std::false_type{});
+        if (w0 < w1) process(w0, std::true_type{}, std::false_type{});
+        for (int t0 = w0 + kTile; t0 < w1; t0 += kTile) process(t0, std::false_type{}, std::false_type{});
+    }
+    if constexpr (HD == 64) {
+        // An infinite value times a weight's low half (0, or of either sign) is
+        // NaN where the weight itself would give Inf: the wave does its range
+        // again in fp32.
+        bool nan = false;
+#pragma unroll
+        for (int b = 0; b < T::kOut; ++b)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) nan |= o[b][i] != o[b][i];
+        if (__builtin_amdgcn_ballot_w64(nan) != 0) {
+#pragma unroll
+            for (int b = 0; b < T::kOut; ++b) o[b] = f32x4{0.f, 0.f, 0.f, 0.f};
+            m_run = -INFINITY;
+            l_run = 0.f;
+            load_tile(w0);
+            for (int t0 = w0; t0 < w1; t0 += kTile) process(t0, std::false_type{}, std::true_type{});
+        }
+#pragma unroll
+        for (int b = 0; b < T::kOut; ++b) o[b] *= 1.f / kScale;
     }
 
     // ---- merge the waves in LDS ----
@@ -929,11 +983,13 @@ int attention_plan_length(int length, int max_context) {
 // (sequence, kv head) units, within a range of chunk lengths that keeps the
 // per-workgroup set-up and the partial write amortised -- at head_dim 128
 // with GQA 64 positions up to 1024 with at most 16 units, 512 with more;
-// 256..512 at head_dim 64 and without GQA, whose bytes per position of one
-// launch unit are fewer (measured on MI355X: one sequence at 512..32768
-// positions, 16 sequences of 4096..32768); the chunk a multiple of a few
-// tiles, and at most kMaxSplits chunks (bounds the merge's per-thread loop
-// and the partials workspace).
+// 256..512 for the other shapes (measured on MI355X: one sequence at
+// 512..32768 positions, 16 sequences of 4096..32768) -- and at most kMaxSplits
+// chunks (bounds the merge's per-thread loop and the partials workspace).  The
+// chunk is a multiple of the four waves' tiles, but at head_dim 64 with more
+// than two heads per kv head of 64 or 32 positions only: there a chunk such as
+// 288 leaves a wave part-filled or without a tile.  (A multiple of 128 would
+// make the same three tiles per wave of it, in fewer workgroups.)
 AttnPlan plan_attention(int max_len, int nseq, int kv_heads, int heads, int head_dim, int target_blocks) {
     AttnPlan p{};
     const int group = heads / kv_heads;
@@ -949,14 +1005,16 @@ AttnPlan plan_attention(int max_len, int nseq, int kv_heads, int heads, int head
     chunk = ((chunk + quantum - 1) / quantum) * quantum;
     p.chunk = (int)chunk;
     p.n_splits = (int)((max_len + chunk - 1) / chunk);
-    // whole-row loads once the launch holds more than two workgroups per CU
-    // (HBM saturates; measured at 16 sequences of 4096..32768 positions, 32/8
-    // heads of 128: 207 against 241 us) or a wave streams eight tiles and more
-    // (split + merge, us, rows against direct: one sequence of 16384 16.4 /
+    // (matrix-core kernel) whole-row loads once the launch holds more than two
+    // workgroups per CU (HBM saturates; measured at 16 sequences of 4096..32768
+    // positions, 32/8 heads of 128: 207 against 241 us) or a chunk has 512
+    // positions, eight tiles a wave at head_dim 128 and four at 64 (split +
+    // merge, us, rows against direct: heads of 128, one sequence of 16384 16.4 /
     // 17.6, of 30011 25.5 / 26.8, 2 of 8192 16.3 / 17.4, 4 of 2000..8192 23.0 /
-    // 25.5, 16 of 100..1500 18.6 / 22.0); direct loads below, where a wave's few
-    // tiles wait for latency and the LDS round trip of K shows (8192 positions
-    // 10.6 against 11.3, 2048 7.2 against 7.8)
+    // 25.5, 16 of 100..1500 18.6 / 22.0; 32/8 heads of 64, one of 18000 13.6 / 15.1,
+    // 8 of 300..3000 13.6 / 15.4); direct loads below, where a wave's few tiles
+    // wait for latency and the LDS round trip of K shows (8192 positions 10.6
+    // against 11.3, 2048 7.2 against 7.8)
     p.rows = chunk >= 512 || units * p.n_splits > 2LL * target_blocks;
     return p;
 }

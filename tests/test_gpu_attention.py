@@ -310,9 +310,9 @@ def test_batched_other_shapes_tile_edges(hip, orc, heads, kv, hd, nseq, bound):
         assert np.all(np.abs(got[s] - ref) <= np.abs(ref) * 2 ** -10 + 1e-4), (n, np.abs(got[s] - ref).max())
 
 
-# Shapes whose value sums run in fp32 (attn_valu_kernel) or with weights split
-# over the matrix cores, each with few and with many heads per kv head
-VALUE_SUMS = [(4, 4, 64), (8, 4, 64), (4, 4, 128)]
+# Shapes whose value sums run in fp32 (one head per kv head, two of 64) and
+# shapes whose weights are split over the matrix cores with fp32's reach
+VALUE_SUMS = [(4, 4, 64), (8, 4, 64), (4, 4, 128), (12, 4, 64), (32, 4, 64)]
 
 
 def _sink(seed, L, heads, kv, hd):
@@ -347,8 +347,11 @@ def test_small_weights_keep_their_value(hip, orc, heads, kv, hd, L):
 @pytest.mark.parametrize("L", [40, 300, 5000])
 def test_infinite_value_stays_infinite(hip, orc, heads, kv, hd, L):
     """An Inf in V (not in a sequence's last chunk, which the merge may read
-    twice) is an Inf of its sign in its dim for every head of its kv head, and
-    nothing else changes."""
+    twice) is an Inf of its sign in its dim for every head of its kv head.
+    Every other value stays within one fp16 step (at most 2^-10 of it, 2^-24
+    below the normal numbers): where the weights are split over the matrix
+    cores, the waves that meet an Inf sum in fp32 instead, which may move a
+    value across one rounding."""
     k, v = _cache(hip, 900 + L, L, kv, hd)
     q = hip.synth.normal_f16(hip.synth.Rng(901), heads * hd)
     ref = _run(hip, q, k, v, L - 1, L, heads, kv, hd).reshape(kv, heads // kv, hd)
@@ -356,4 +359,6 @@ def test_infinite_value_stays_infinite(hip, orc, heads, kv, hd, L):
     v3[5, 1, 7], v3[20, 2, 0], v3[33, 2, hd - 1] = 0x7c00, 0xfc00, 0x7c00
     got = _run(hip, q, k, v3.reshape(-1), L - 1, L, heads, kv, hd).reshape(kv, heads // kv, hd)
     ref[1, :, 7], ref[2, :, 0], ref[2, :, hd - 1] = np.inf, -np.inf, np.inf
-    np.testing.assert_array_equal(got, ref)
+    inf = np.isinf(ref)
+    np.testing.assert_array_equal(got[inf], ref[inf])
+    assert np.all(np.abs(got[~inf] - ref[~inf]) <= 2.0 ** -10 * np.abs(ref[~inf]) + 2.0 ** -24)
