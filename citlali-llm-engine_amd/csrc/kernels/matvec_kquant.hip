@@ -29,6 +29,7 @@
 
 #include "device_common.hpp"
 #include "launch.hpp"
+#include "q6k_pieces.hpp"
 
 namespace citlali::hip {
 namespace {
@@ -847,6 +848,7 @@ struct TileAt {
     const uint8_t* w[2];
     void* y;
     int row, rows;   // first row and rows (up to 16) of the tile in its matrix
+    int n;           // rows of the matrix
 };
 
 // The tiles wg, wg + wgs, ... of `tiles`.  tile_of(t): the matrix (its first
@@ -908,15 +910,25 @@ __device__ __forceinline__ void tile_rows(const uint16_t* __restrict__ x, int nb
             ++s.u;
         }
     };
-    // The block rows of a step into a ring slot.  Every piece holds bytes of
-    // its block, so an aligned piece never reaches past the page of one.
-    const uint8_t* unit_base = nullptr;
+    // The block rows of a step into a ring slot.  A Q6_K matrix need not begin
+    // or end with a whole piece: the blocks at its two ends go through
+    // registers, value by value inside the matrix (the bytes outside are not
+    // used, so any value will do for them).
+    const uint8_t *unit_base = nullptr, *first_byte = nullptr, *last_half = nullptr;
     int unit = -1;
+    Q6KEnds ends{-1, -1};
     auto copy = [&](const Walk& s, int slot) {
         if (s.u != unit) {   // wave-uniform
             unit = s.u;
             const TileAt t = tile_of(wg + (unit / kMats) * wgs);
-            unit_base = (kMats == 2 && (unit & 1) ? t.w[1] : t.w[0]) + (size_t)t.row * row_bytes;
+            const uint8_t* w = kMats == 2 && (unit & 1) ? t.w[1] : t.w[0];
+            unit_base = w + (size_t)t.row * row_bytes;
+            if constexpr (QT::kBytes % 16 != 0) {
+                static_assert(QT::kBytes == kQ6KBlockBytes && kPieces == kQ6KPieces, "Q6_K");
+                ends = q6k_ends(reinterpret_cast<uintptr_t>(w), t.n, nb, t.row == 0, t.row + t.rows == t.n);
+                first_byte = w;
+                last_half = w + (size_t)t.n * row_bytes - 2;
+            }
 #pragma unroll
             for (int c = 0; c < kCopies; ++c) {
                 rel[c] = min(lr[c], t.rows - 1) * row_bytes;
@@ -929,11 +941,25 @@ __device__ __forceinline__ void tile_rows(const uint16_t* __restrict__ x, int nb
 #pragma unroll
             for (int c = 0; c < kCopies; ++c) copy16_to_lds(base + (uint32_t)rel[c], dst + c * kWave * 16);
         } else {
-            const int skew = (int)((uintptr_t)base & 15);
+            const int skew = (int)(reinterpret_cast<uintptr_t>(base) & 15);
             base -= skew;
+            if (s.b != ends.lo && s.b != ends.hi) {   // wave-uniform
 #pragma unroll
-            for (int c = 0; c < kCopies; ++c)
-                copy16_to_lds(base + (uint32_t)(((rel[c] + skew) & ~15) + pc16[c]), dst + c * kWave * 16);
+                for (int c = 0; c < kCopies; ++c)
+                    copy16_to_lds(base + (uint32_t)(q6k_piece(skew, rel[c], 0) + pc16[c]), dst + c * kWave * 16);
+            } else {
+#pragma unroll
+                for (int c = 0; c < kCopies; ++c) {
+                    const uint8_t* p = base + (uint32_t)(q6k_piece(skew, rel[c], 0) + pc16[c]);
+                    uint16_t* to = reinterpret_cast<uint16_t*>(dst + (c * kWave + lane) * 16);
+#pragma unroll 1
+                    for (int i = 0; i < 16; i += 2) {
+                        const uint8_t* h = p + i;
+                        h = h < first_byte ? first_byte : h > last_half ? last_half : h;
+                        to[i >> 1] = *reinterpret_cast<const uint16_t*>(h);
+                    }
+                }
+            }
         }
     };
 
@@ -1117,7 +1143,8 @@ struct SetTiles {
         const bool s1 = t >= e0, s2 = t >= e1;
         const uint8_t* w = pick3(s1, s2, w0, w1, w2);
         const int row = (t - pick3(s1, s2, 0, e0, e1)) * kRows;
-        return TileAt{{w, w}, pick3(s1, s2, y0, y1, y2), row, min(kRows, pick3(s1, s2, n0, n1, n2) - row)};
+        const int n = pick3(s1, s2, n0, n1, n2);
+        return TileAt{{w, w}, pick3(s1, s2, y0, y1, y2), row, min(kRows, n - row), n};
     }
 };
 
@@ -1148,7 +1175,7 @@ __global__ __launch_bounds__(kTileBlock, 4) void matvec_tile_gate_up_kernel(cons
     extern __shared__ __align__(16) uint8_t smem[];
     tile_rows<SH, kNormIters>(
         x, nb, smem, blockIdx.x, gridDim.x, tiles, nrm,
-        [=](int t) { return TileAt{{wg, wu}, nullptr, t * SH::kRows, min(SH::kRows, N - t * SH::kRows)}; },
+        [=](int t) { return TileAt{{wg, wu}, nullptr, t * SH::kRows, min(SH::kRows, N - t * SH::kRows), N}; },
         [=](const TileAt&, int row, const float (&s)[2]) {
             const float g = h2f(f2h_rne(s[0])), u = h2f(f2h_rne(s[1]));
             act[row] = f2h_rne(g / (1.0f + expf(-g)) * u);

@@ -186,10 +186,10 @@ def test_rows_permute_with_weights(hip):
     np.testing.assert_array_equal(dy.download(np.float32, n), y[perm])
 
 
-# Rows of the block counts that run on the tile kernels (tiles of 14 Q4_K or
-# 16 Q6_K rows, blocks dealt to eight waves): row counts around a tile and its
-# neighbours, block counts below, at and beyond the eight waves and up to the
-# largest, many tiles per workgroup.
+# Block counts that run on the tile kernels from some number of rows or blocks
+# on (tiles of 14 Q4_K or 16 Q6_K rows, blocks dealt to eight waves): row counts
+# around a tile and its neighbours, block counts below, at and beyond the eight
+# waves and up to the largest, many tiles per workgroup.
 TILE_ROWS = [1, 13, 14, 15, 16, 17, 33]
 TILE_K = [256, 768, 1792, 2304, 5120, 18944, 28416]
 
@@ -197,7 +197,7 @@ TILE_K = [256, 768, 1792, 2304, 5120, 18944, 28416]
 @pytest.mark.parametrize("kind", ["q4k", "q6k"])
 @pytest.mark.parametrize("k", TILE_K)
 def test_tile_rows_match_oracle(hip, orc, kind, k):
-    for n in TILE_ROWS + ([20011] if k == 768 else []):
+    for n in TILE_ROWS + ([32771] if k == 768 else []):
         print(f"[tile matvec] kind={kind} n={n} k={k}", flush=True)
         w, x = _inputs(hip, kind, n, k, seed=3 * n + k)
         # Q6_K weights are 4-byte aligned, so try an offset inside a 16-byte piece
