@@ -108,18 +108,15 @@ __device__ __forceinline__ uint32_t f2h2_ties_away(float a, float b) {
     return __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_pkrtz(add_half_ulp(a), add_half_ulp(b)));
 }
 
-// Eight consecutive values of a block as fp16, value(code) of the codes in
-// the bytes of c0, c1.
+// Eight consecutive values of a block, value(code) of the codes in the bytes of
+// c0, c1.
 template <typename Value>
-__device__ __forceinline__ u32x4 run_of_codes(uint32_t c0, uint32_t c1, Value value) {
-    float v[8];
+__device__ __forceinline__ void values_of_codes(uint32_t c0, uint32_t c1, Value value, float (&v)[8]) {
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
         v[i] = value((float)((c0 >> (8 * i)) & 0xffu));
         v[4 + i] = value((float)((c1 >> (8 * i)) & 0xffu));
     }
-    return u32x4{f2h2_ties_away(v[0], v[1]), f2h2_ties_away(v[2], v[3]), f2h2_ties_away(v[4], v[5]),
-                 f2h2_ties_away(v[6], v[7])};
 }
 
 // The share of a block that one thread dequantises, from wide loads that no
@@ -151,9 +148,9 @@ struct DequantQ4K {
         return fabsf(d) * 945.f + fabsf(dmin) * 63.f < 65000.f;
     }
     // s, m and s * code are exact in fp32: one rounding, as on the host
-    __device__ __forceinline__ u32x4 run(int k) const {
-        return run_of_codes((w.x >> (4 * k)) & 0x0f0f0f0fu, (w.y >> (4 * k)) & 0x0f0f0f0fu,
-                            [&](float q) { return fmaf(s[k], q, -m[k]); });
+    __device__ __forceinline__ void run(int k, float (&v)[8]) const {
+        values_of_codes((w.x >> (4 * k)) & 0x0f0f0f0fu, (w.y >> (4 * k)) & 0x0f0f0f0fu,
+                        [&](float q) { return fmaf(s[k], q, -m[k]); }, v);
     }
 };
 struct DequantQ6K {
@@ -176,12 +173,12 @@ struct DequantQ6K {
         s[3] = d * (float)(int8_t)(sc.y >> (sh + 16u));
         return fabsf(d) * 4096.f < 65000.f;
     }
-    __device__ __forceinline__ u32x4 run(int k) const {
+    __device__ __forceinline__ void run(int k, float (&v)[8]) const {
         const u32x2 lo = l[k & 1];
         const int nib = 4 * (k >> 1);
-        return run_of_codes(((lo.x >> nib) & 0x0f0f0f0fu) | (((u.x >> (2 * k)) & 0x03030303u) << 4),
-                            ((lo.y >> nib) & 0x0f0f0f0fu) | (((u.y >> (2 * k)) & 0x03030303u) << 4),
-                            [&](float q) { return s[k] * (q - 32.f); });
+        values_of_codes(((lo.x >> nib) & 0x0f0f0f0fu) | (((u.x >> (2 * k)) & 0x03030303u) << 4),
+                        ((lo.y >> nib) & 0x0f0f0f0fu) | (((u.y >> (2 * k)) & 0x03030303u) << 4),
+                        [&](float q) { return s[k] * (q - 32.f); }, v);
     }
 };
 
@@ -191,9 +188,11 @@ struct DequantQ6K {
 // thread, byte loads and a branching conversion, bound by instruction issue,
 // they took 129 and 97 us; with eight values per thread and plain stores 34
 // and 44; with the shares above and plain stores 29.6 and 35.5 -- the output
-// is not read again soon, so it is stored nontemporal.  A thread whose values could
-// overflow, whose scale is Inf or NaN or that holds the ragged end goes value
-// by value through the exact host rule.
+// is not read again soon, so it is stored nontemporal.  A partial last block
+// takes the same steps but stores its last run value by value (100,000 values:
+// 3.4 us; going back to the bytes value by value 7.6 and 10.3).  Values that
+// could overflow are converted one by one by the exact host rule, a run with a
+// NaN from the bytes.
 template <class QT>
 __global__ __launch_bounds__(256) void dequant_kernel(const uint8_t* __restrict__ w, uint64_t count,
                                                       uint16_t* __restrict__ out) {
@@ -204,15 +203,43 @@ __global__ __launch_bounds__(256) void dequant_kernel(const uint8_t* __restrict_
         const int r = (int)(i % QT::kThreads);
         const uint64_t e0 = b * kQK + QT::first(r);
         QT t;
-        if (t.load(blk, r) && b * kQK + kQK <= count) {
+        const bool in_range = t.load(blk, r), whole = b * kQK + kQK <= count;
+        float v[8];
+        if (in_range) {
 #pragma unroll
-            for (int k = 0; k < QT::kRuns; ++k) __builtin_nontemporal_store(t.run(k), reinterpret_cast<u32x4_a2*>(out + e0 + k * QT::kApart));
-        } else {
-            for (int k = 0; k < QT::kRuns; ++k)
-                for (int e = 0; e < 8; ++e) {
-                    const uint64_t o = e0 + k * QT::kApart + e;
-                    if (o < count) out[o] = f2h_ties_away(QT::value(blk, QT::first(r) + k * QT::kApart + e));
+            for (int k = 0; k < QT::kRuns; ++k) {
+                t.run(k, v);
+                const u32x4 h{f2h2_ties_away(v[0], v[1]), f2h2_ties_away(v[2], v[3]), f2h2_ties_away(v[4], v[5]),
+                              f2h2_ties_away(v[6], v[7])};
+                const uint64_t at = e0 + k * QT::kApart;
+                if (whole || at + 8 <= count) {
+                    __builtin_nontemporal_store(h, reinterpret_cast<u32x4_a2*>(out + at));
+                } else {
+#pragma unroll
+                    for (int e = 0; e < 8; ++e)
+                        if (at + e < count) out[at + e] = (uint16_t)(h[e >> 1] >> (16 * (e & 1)));
                 }
+            }
+        } else {
+#pragma unroll
+            for (int k = 0; k < QT::kRuns; ++k) {
+                const uint64_t at = e0 + k * QT::kApart;
+                if (at >= count) break;
+                const int n = count - at < 8 ? (int)(count - at) : 8;
+                t.run(k, v);
+                bool nan = false;
+#pragma unroll
+                for (int e = 0; e < 8; ++e) nan |= __builtin_isnan(v[e]);
+                if (!nan) {
+#pragma unroll
+                    for (int e = 0; e < 8; ++e)
+                        if (e < n) out[at + e] = f2h_ties_away(v[e]);
+                } else {
+#pragma unroll 1
+                    for (int e = 0; e < n; ++e)
+                        out[at + e] = f2h_ties_away(QT::value(blk, QT::first(r) + k * QT::kApart + e));
+                }
+            }
         }
     }
 }

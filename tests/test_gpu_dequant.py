@@ -114,3 +114,19 @@ def test_device_dequant_scale_range_and_alignment(hip, orc, kind, w_off, o_off):
     got = out[o_off:o_off + 2 * count].copy().view(np.uint16)
     np.testing.assert_array_equal(got, orc.dequant_f16(kind, blocks.reshape(-1), count))
     assert not out[:o_off].any() and not out[o_off + 2 * count:].any(), "wrote outside the output"
+
+
+@pytest.mark.parametrize("kind", ["q4k", "q6k"])
+def test_device_dequant_partial_last_block(hip, orc, kind):
+    """Counts that end inside a block, a run of eight values or on either's
+    edge: the host routine's values, and nothing behind them."""
+    rng = hip.synth.Rng(5)
+    w = hip.synth.q4k_blocks(rng, 40) if kind == "q4k" else hip.synth.q6k_blocks(rng, 40)
+    ref = orc.dequant_f16(kind, w, 40 * 256)
+    dw, do = hip.DeviceArray.from_numpy(w), hip.DeviceArray(41 * 512)
+    for count in [1, 7, 8, 9, 31, 32, 33, 127, 129, 255, 256, 257, 300, 1000, 256 * 39 + 1, 256 * 40 - 1]:
+        do.zero()
+        hip.device.dequant_f16(kind, dw, count, do)
+        got = do.download(np.uint16)
+        np.testing.assert_array_equal(got[:count], ref[:count], err_msg=str(count))
+        assert not got[count:].any(), count
