@@ -748,8 +748,8 @@ CITLALI_EXPORT int citlali_hip_graph_destroy(void* graph) {
 
 namespace {
 // Row lengths the grouped / prologue / gate-up GEMV kernels cover
-bool norm_length_ok(int in_f) { return matvec_fused_length(in_f, true); }
-bool group_length_ok(int in_f) { return matvec_fused_length(in_f, true); }   // hidden-sized inputs
+bool norm_length_ok(int in_f) { return matvec_fused_length(in_f); }
+bool group_length_ok(int in_f) { return matvec_fused_length(in_f); }   // hidden-sized inputs
 bool gate_up_length_ok(int in_f) { return matvec_gate_up_length(in_f); }
 // GEMV weight types of the grouped / fused entry points: GGUF Q4_K (12),
 // Q6_K (14) and F16 (1, fp16 rows), as the kernels' kinds 4, 6, 1

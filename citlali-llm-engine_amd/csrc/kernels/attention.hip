@@ -4,7 +4,8 @@
 // Semantics follow kernels.cu:545-649 of the reference: for query head h
 // (kv head h / (heads/kv_heads)) and cached positions t = 0..position,
 // s_t = (q_h . K[t]) / sqrt(head_dim); p = softmax(s); out_h = sum_t p_t V[t],
-// fp32 arithmetic, fp16 output rounded nearest-even.  Cache layout is the
+// fp32 sums, fp16 output rounded nearest-even (the matrix-core kernel takes p
+// as two fp16 halves, see there).  Cache layout is the
 // reference's [position][kv_head][head_dim] (kernels.cu:524-533).
 //
 // gfx950 design

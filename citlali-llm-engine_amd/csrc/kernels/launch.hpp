@@ -88,17 +88,15 @@ inline hipError_t allow_lds(int lds) {
 }
 
 // ---- fused dequant GEMV (matvec_kquant.hip) ----
-// kind: 4 = Q4_K, 6 = Q6_K, 1 = fp16 weights
-size_t matvec_lds_bytes(int kind, int K);
 // in_features of the grouped GEMV and the input prologue: 1024, 2048, 2560,
-// 3072, 4096, 5120, 6144, 8192, 9728, 12288, 16384 (with norm = false also
-// 17408 and 25600, plain K-quant GEMVs of the streaming kernels)
-bool matvec_fused_length(int K, bool norm);
+// 3072, 4096, 5120, 6144, 8192, 9728, 12288, 16384
+bool matvec_fused_length(int K);
 // in_features of the gate/up + SwiGLU launch: 1024, 2048, 2560, 3072, 4096,
 // 5120, 8192
 bool matvec_gate_up_length(int K);
-// fp16 weights [N][K], K a multiple of 256 up to CITLALI_MAX_IN_FEATURES,
-// through the streaming kernels of the K-quant GEMVs
+// fp16 weights [N][K], K a multiple of 256 up to CITLALI_MAX_IN_FEATURES: the
+// streaming kernels of the K-quant GEMVs where they have the length, else
+// launch_matvec_f16_rows
 hipError_t launch_matvec_f16_blocks(const uint16_t* w, const uint16_t* x, void* y, bool f32_out, int K, int N,
                                     hipStream_t s);
 // fp16 weights [N][K] of any other K (matvec_f16.hip)
@@ -140,7 +138,7 @@ struct AttnPlan {
     int gp;        // padded GQA group (1, 2, 4, 8)
     int chunk;     // positions per workgroup
     int n_splits;  // chunks of the longest sequence
-    bool rows;     // whole-row nontemporal tile loads through LDS
+    bool rows;     // matrix-core kernel: whole-row nontemporal tile loads through LDS
 };
 bool attention_supported(int head_dim, int group);
 // The length a decode step's attention is planned for: the smallest power
@@ -199,8 +197,7 @@ hipError_t launch_matvec_group(int count, const int* kinds, const uint8_t* const
                                uint16_t* const* y, const int* n, int K, const NormIn* norm, hipStream_t s);
 hipError_t launch_matvec_gate_up_swiglu(int kind, const uint8_t* wg, const uint8_t* wu, const uint16_t* x,
                                         uint16_t* act, int K, int N, const NormIn* norm, hipStream_t s);
-// kind 4 / 6 / 1 GEMV with the input prologue; K 1024, 2048, 3072 or a
-// multiple of 4096 up to 16384
+// kind 4 / 6 / 1 GEMV with the input prologue; K a matvec_fused_length
 hipError_t launch_matvec_norm(int kind, const uint8_t* w, const uint16_t* x, const NormIn& norm, void* y,
                               bool f32_out, int K, int N, hipStream_t s);
 hipError_t launch_fill_zero(void* p, size_t bytes, hipStream_t s);

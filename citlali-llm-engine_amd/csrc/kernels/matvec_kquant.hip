@@ -1498,21 +1498,16 @@ hipError_t launch_gate_up(int kind, const uint8_t* wg, const uint8_t* wu, const 
 
 }  // namespace
 
-bool matvec_fused_length(int K, bool norm) {
+bool matvec_fused_length(int K) {
     if (K <= 0 || K % kQK != 0) return false;
     switch (K / kQK) {
         case 4: case 8: case 10: case 12: case 16: case 20: case 24: case 32: case 38: case 48: case 64: return true;
-        case 68: case 100: return !norm;
         default: return false;
     }
 }
 
 bool matvec_gate_up_length(int K) {
     return K == 1024 || K == 2048 || K == 2560 || K == 3072 || K == 4096 || K == 5120 || K == 8192;
-}
-
-size_t matvec_lds_bytes(int kind, int K) {
-    return kind == 6 ? lds_bytes<Q6K>(K) : kind == 1 ? lds_bytes<F16>(K) : lds_bytes<Q4K>(K);
 }
 
 hipError_t launch_matvec_f16_blocks(const uint16_t* w, const uint16_t* x, void* y, bool f32_out, int K, int N,
@@ -1545,8 +1540,8 @@ hipError_t launch_matvec_norm(int kind, const uint8_t* w, const uint16_t* x, con
 
 // count matrices (1..3) reading x: kinds[i] 4 = Q4_K, 6 = Q6_K, 1 = fp16
 // (all or none), n[i] rows, fp16 outputs y[i].  hipErrorInvalidValue,
-// nothing launched, for a length other than 1024, 2048, 3072, 4096, 8192,
-// 12288 or 16384 or fp16 mixed with quantized matrices.
+// nothing launched, for a length that is no matvec_fused_length or fp16 mixed
+// with quantized matrices.
 hipError_t launch_matvec_group(int count, const int* kinds, const uint8_t* const* w, const uint16_t* x,
                                uint16_t* const* y, const int* n, int K, const NormIn* norm, hipStream_t s) {
     RowSet set[2];
@@ -1572,8 +1567,7 @@ hipError_t launch_matvec_group(int count, const int* kinds, const uint8_t* const
                 : launch_group<false>(nb, set, cnt, f16 != 0, x, K, kNoNorm, s);
 }
 
-// kind 4: Q4_K, 6: Q6_K, 1: fp16; in_features 1024, 2048, 3072, 4096 or
-// 8192 (4, 8, 12, 16 or 32 blocks of 256)
+// kind 4: Q4_K, 6: Q6_K, 1: fp16; in_features a matvec_gate_up_length
 hipError_t launch_matvec_gate_up_swiglu(int kind, const uint8_t* wg, const uint8_t* wu, const uint16_t* x,
                                         uint16_t* act, int K, int N, const NormIn* norm, hipStream_t s) {
     return norm ? launch_gate_up<true>(kind, wg, wu, x, act, K, N, *norm, s)

@@ -106,7 +106,10 @@ int citlali_hip_embed_q6k(const uint8_t* table, int32_t token_id, uint16_t* out,
  * otherwise the library keeps its own per-device workspace (allocated on the
  * first call that needs it, kept until citlali_hip_release_workspace()).
  * It no longer receives the raw scores.  head_dim 64 or 128, heads/kv_heads
- * between 1 and 8.  The split of the positions over workgroups is planned
+ * between 1 and 8.  Cached values are expected finite: an Inf in V is an Inf in
+ * the output of its dim (unless its weight is 0 or it lies in the last chunk of
+ * several), but NaN at head_dim 128 with two heads per kv head and more, whose
+ * weights are split in two for the matrix cores.  The split of the positions over workgroups is planned
  * for citlali_hip_attention_plan_length(position + 1, max_context), so all
  * steps of one such length run the same launches. */
 int citlali_hip_attention(const uint16_t* q, const uint16_t* k_cache, const uint16_t* v_cache, float* scores,

@@ -93,11 +93,11 @@ def test_fused_long_context(hip, device_position):
 
 @pytest.mark.parametrize("device_position", [False, True])
 def test_fused_row_loads(hip, device_position):
-    """Past 64K positions one sequence of 8 KV heads plans more than 512
-    (KV head, chunk) units, and the split kernel switches to its row-load form
-    (rows staged through LDS instead of direct loads), where the prologue
-    substitutes the step's k/v row into the staged K/V rows.  ctx 70000: the
-    plan is 69 chunks of 1024 (72 units of 8 KV heads would be 576)."""
+    """Chunks of 512 positions and more (one sequence of 8 KV heads from
+    16384 positions on) and launches of more than 512 (KV head, chunk) units
+    (past 64K positions) take the chunk kernel's row-load form (rows staged
+    through LDS instead of direct loads), where the prologue substitutes the
+    step's k/v row into the staged K/V rows.  ctx 70000: 69 chunks of 1024."""
     ctx = 70000
     for pos in (66000, 69999):
         plan = hip.device.attention_plan_length(pos + 1, ctx)
